@@ -53,12 +53,34 @@ struct DevSys {
     int lmax;                 // largest primitive angular momentum (3: f functions present)
 };
 
+// Distinct pairs of a one-basis system (device arrays).  A contracted pair is
+// {I <= J}, number J(J+1)/2 + I; its primitive pairs (i of I, j of J; i <= j
+// when I = J, the off-diagonal ones counted twice in their coefficient) are
+// consecutive in the pair list.  Slots: the pair list sorted by angular
+// momentum and padded to groups of 64, one per lane of a wave.
+struct PairPlan {
+    i64 ncp, npl, nslot, nq;  // contracted pairs, primitive pairs, slots, distinct nuclear pairs
+    int le, lp;               // largest angular momentum, electronic and nuclear
+    const int *cp_start;      // ncp + 1: pair-list range of a contracted pair
+    const int *pl_idx, *pl_deg; // entry of ep; bra + ket powers per direction, a byte each
+    const int *slot;          // pair-list entry per slot, -1 for padding
+    const int *gdeg, *gL;     // per 64 slots: largest degree per direction, largest total degree
+    const int *pp_idx, *pp_deg; // nuclear pair q = j(j+1)/2 + i: entry of pp, powers
+    const double *pl_coef, *pp_coef;
+    // geminal terms: every ordered (k,l) with b_k b_l; then the one-geminal
+    // terms gamma_k with b_k and the k <= l terms gamma_k + gamma_l with
+    // b_k b_l / 2 (k < l: twice that); {1, 0}
+    const double *gk, *gl, *wkl, *gx, *wx, *one;
+};
+
 struct System {
     DevSys d;
     std::vector<void *> allocs;
     std::vector<i64> eord, pord;
     std::vector<i64> kpestr; // host copy (1-based)
     int maxl;
+    PairPlan plan{};
+    std::vector<i64> cp_start; // host copy
 };
 
 NRX_HIDDEN System *get_sys(i64 h);
@@ -109,6 +131,26 @@ struct DevBuf {
     double *d() { return (double *)p; }
 };
 
+// stream-ordered scratch, freed on its stream when it goes out of scope
+struct StreamBuf {
+    void *p = nullptr;
+    hipStream_t st = 0;
+    ~StreamBuf()
+    {
+        if (p) (void)hipFreeAsync(p, st);
+    }
+    int alloc(size_t bytes, hipStream_t s)
+    {
+        st = s;
+        hipError_t e = hipMallocAsync(&p, bytes, s);
+        if (e != hipSuccess) {
+            p = nullptr;
+            return fail(NEORX_E_NOMEM, "hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
+        }
+        return NEORX_OK;
+    }
+};
+
 // storage type of an in-core tensor read by the contractions
 enum { NRX_F64 = 0, NRX_F32 = 1, NRX_BF16 = 2 };
 
@@ -134,3 +176,12 @@ NRX_HIDDEN int nrx_eg3_slabs2(i64 ne, i64 nblk, const double *d_x, const double 
 // dirS, exS (gs may be NULL: the S rows stay zero)
 NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double *g, const double *gs, double *part,
                              hipStream_t st);
+
+// ------------------------------------------------------------------
+// tensors from distinct pairs (nrx_stars.hip), l <= 2.  Enqueued on st, with
+// stream-ordered scratch.
+// ------------------------------------------------------------------
+// GAM3_IC1 (mult: RXCHFmult_GAM3_XCHF) of the distinct nuclear pairs
+// [q0, q1).  npbf > 0: into the full tensor G, both orders of each pair;
+// npbf = 0: one block of nebf^6 per pair, from G on.
+NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, hipStream_t st);

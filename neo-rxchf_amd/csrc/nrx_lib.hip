@@ -156,6 +156,104 @@ static void pair_table(i64 n, const double *ex, const i64 *am, const double *cen
         for (i64 j = 0; j < n; ++j) make_pair(host_prim(n, ex, am, cen, i), host_prim(n, ex, am, cen, j), tab[i * n + j]);
 }
 
+// PairPlan of a system from its pair tables (one device block, one copy)
+static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc, const double *agnbfcc,
+                     const double *bcoef, const double *gamma, const std::vector<PairRec> &ept,
+                     const std::vector<PairRec> &ppt)
+{
+    const i64 ne = s->d.nebf, pe = s->d.npebf, np = s->d.npbf;
+    auto deg = [](const PairRec &q) {
+        int m = 0;
+        for (int d = 0; d < 3; ++d) m |= (q.la[d] + q.lb[d]) << (8 * d);
+        return m;
+    };
+    auto byte = [](int m, int d) { return (m >> (8 * d)) & 255; };
+    auto total = [&](int m) { return byte(m, 0) + byte(m, 1) + byte(m, 2); };
+    std::vector<int> cps{0}, idx, dg, slot, gd, gl, pidx, pdg;
+    std::vector<double> cf, pcf, term;
+    for (i64 J = 0; J < ne; ++J)
+        for (i64 I = 0; I <= J; ++I) {
+            for (i64 i = s->kpestr[I] - 1; i < kpeend[I]; ++i)
+                for (i64 j = I == J ? i : s->kpestr[J] - 1; j < kpeend[J]; ++j) {
+                    idx.push_back((int)(i * pe + j));
+                    dg.push_back(deg(ept[i * pe + j]));
+                    cf.push_back(agebfcc[i] * agebfcc[j] * (I == J && i < j ? 2.0 : 1.0));
+                }
+            cps.push_back((int)idx.size());
+        }
+    for (i64 j = 0; j < np; ++j)
+        for (i64 i = 0; i <= j; ++i) {
+            pidx.push_back((int)(i * np + j));
+            pdg.push_back(deg(ppt[i * np + j]));
+            pcf.push_back(agnbfcc[i] * agnbfcc[j]);
+        }
+    PairPlan &P = s->plan;
+    P.ncp = (i64)cps.size() - 1;
+    P.npl = (i64)idx.size();
+    P.nq = (i64)pidx.size();
+    // slots: by largest power per direction, then by the powers, so that the
+    // lanes of a group share their loop bounds
+    slot.resize(P.npl);
+    std::iota(slot.begin(), slot.end(), 0);
+    auto top = [&](int m) { return std::max(byte(m, 0), std::max(byte(m, 1), byte(m, 2))); };
+    std::stable_sort(slot.begin(), slot.end(), [&](int a, int b) {
+        if (top(dg[a]) != top(dg[b])) return top(dg[a]) < top(dg[b]);
+        return dg[a] < dg[b];
+    });
+    slot.resize((P.npl + 63) / 64 * 64, -1);
+    P.nslot = (i64)slot.size();
+    for (i64 g = 0; g < P.nslot; g += 64) {
+        int m[3] = {0, 0, 0}, L = 0;
+        for (i64 k = g; k < g + 64; ++k)
+            if (slot[k] >= 0) {
+                for (int d = 0; d < 3; ++d) m[d] = std::max(m[d], byte(dg[slot[k]], d));
+                L = std::max(L, total(dg[slot[k]]));
+            }
+        gd.push_back(m[0] | m[1] << 8 | m[2] << 16);
+        gl.push_back(L);
+    }
+    P.le = P.lp = 0;
+    for (i64 i = 0; i < pe; ++i) P.le = std::max(P.le, total(dg.empty() ? 0 : deg(ept[i * pe + i])) / 2);
+    for (i64 i = 0; i < np; ++i) P.lp = std::max(P.lp, total(deg(ppt[i * np + i])) / 2);
+    // geminal terms: gk, gl, wkl [ng^2]; gx, wx [ng + ng(ng+1)/2]; {1, 0}
+    std::vector<double> gk, gll, wkl, gx(gamma, gamma + ng), wx(bcoef, bcoef + ng);
+    for (i64 k = 0; k < ng; ++k)
+        for (i64 l = 0; l < ng; ++l) {
+            gk.push_back(gamma[k]);
+            gll.push_back(gamma[l]);
+            wkl.push_back(bcoef[k] * bcoef[l]);
+            if (l >= k) {
+                gx.push_back(gamma[k] + gamma[l]);
+                wx.push_back(bcoef[k] * bcoef[l] * (l > k ? 1.0 : 0.5));
+            }
+        }
+    // one block: the doubles, then the ints
+    std::vector<const std::vector<double> *> dv{&cf, &pcf, &gk, &gll, &wkl, &gx, &wx};
+    std::vector<const std::vector<int> *> iv{&cps, &idx, &dg, &slot, &gd, &gl, &pidx, &pdg};
+    std::vector<double> blk{1.0, 0.0};
+    std::vector<size_t> off;
+    for (auto *v : dv) {
+        off.push_back(blk.size());
+        blk.insert(blk.end(), v->begin(), v->end());
+    }
+    for (auto *v : iv) {
+        off.push_back(blk.size());
+        const size_t at = blk.size();
+        blk.resize(at + (v->size() + 1) / 2, 0.0);
+        std::memcpy(blk.data() + at, v->data(), v->size() * sizeof(int));
+    }
+    const double *b = nullptr;
+    int rc = upload(s, blk.data(), blk.size(), &b);
+    if (rc) return rc;
+    const double **dp[] = {&P.pl_coef, &P.pp_coef, &P.gk, &P.gl, &P.wkl, &P.gx, &P.wx};
+    const int **ip[] = {&P.cp_start, &P.pl_idx, &P.pl_deg, &P.slot, &P.gdeg, &P.gL, &P.pp_idx, &P.pp_deg};
+    P.one = b;
+    for (int k = 0; k < 7; ++k) *dp[k] = b + off[k];
+    for (int k = 0; k < 8; ++k) *ip[k] = (const int *)(b + off[7 + k]);
+    s->cp_start.assign(cps.begin(), cps.end());
+    return NEORX_OK;
+}
+
 extern "C" int neorx_system_create(int64_t nebf, int64_t npebf, int64_t npbf, int64_t nat, int64_t ngtg, double pmass,
                                    const double *cat, const double *zan, const double *bcoef, const double *gamma,
                                    const int64_t *kpestr, const int64_t *kpeend, const int64_t *ampeb2c,
@@ -244,6 +342,7 @@ extern "C" int neorx_system_create(int64_t nebf, int64_t npebf, int64_t npbf, in
     r |= upload(s, s->pord.data(), npbf, &d.pord);
     r |= upload(s, ept.data(), ept.size(), &d.ep);
     r |= upload(s, ppt.data(), ppt.size(), &d.pp);
+    if (!r && maxl <= 2) r = pair_plan(s, ngtg, kpeend, agebfcc, agnbfcc, bcoef, gamma, ept, ppt);
     if (r) {
         for (void *p : s->allocs) (void)hipFree(p);
         delete s;
@@ -453,26 +552,6 @@ __global__ void k_zero_u32n(unsigned *p, int n)
 // entries are 32-bit positions, and the bin counters)
 static const i64 PRIM_CHUNK = (i64)1 << 24;
 
-// stream-ordered scratch: the sorted tuple list, bin codes and counters
-struct StreamBuf {
-    void *p = nullptr;
-    hipStream_t st = 0;
-    ~StreamBuf()
-    {
-        if (p) (void)hipFreeAsync(p, st);
-    }
-    int alloc(size_t bytes, hipStream_t s)
-    {
-        st = s;
-        hipError_t e = hipMallocAsync(&p, bytes, s);
-        if (e != hipSuccess) {
-            p = nullptr;
-            return fail(NEORX_E_NOMEM, "hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
-        }
-        return NEORX_OK;
-    }
-};
-
 template <int CLS, int SRC>
 static int launch_prims(const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os, hipStream_t st,
                         double *ox = nullptr, double *oy = nullptr)
@@ -484,6 +563,7 @@ static int launch_prims(const DevSys &d, i64 start, i64 ntup, const i64 *idx, do
             return fail(NEORX_E_ARG, "class %d enumerates two electron bases; this handle has one", CLS);
     if (ntup <= 0) return NEORX_OK;
     i64 cap = std::min(ntup, PRIM_CHUNK);
+    // stream-ordered scratch: bin counters, the sorted tuple list and the bin codes
     StreamBuf ws; // header: counts[32], cursors[32]; list: cap x u32; codes: cap x u8
     int rc = ws.alloc(256 + cap * sizeof(unsigned) + cap, st);
     if (rc) return rc;
@@ -963,6 +1043,11 @@ template <int CLS> static int gam3_build_dev(System *s, double *d_gm3, void *str
 {
     i64 ne = s->d.nebf, np = s->d.npbf, blk = ne * ne * ne * ne * ne * ne;
     hipStream_t st = (hipStream_t)stream;
+    if (s->maxl <= 2) {
+        int r = nrx_gam3_pairs(s, CLS == 7, 0, s->plan.nq, np, d_gm3, st);
+        if (!r) HIPCHK(hipStreamSynchronize(st));
+        return r;
+    }
     i64 cap = slab_cap(s, 3);
     // one (ip,jp) block of unsymmetrised values at a time: the scratch is
     // nebf^6 doubles, not the whole tensor again
@@ -2147,6 +2232,15 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     return NEORX_OK;
 }
 
+// rows of every (ip,jp) from those of the distinct nuclear pairs (n values each)
+__global__ void k_unfold_pairs(i64 np, i64 n, const double *__restrict__ q, double *__restrict__ out)
+{
+    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < np * np * n; t += (i64)gridDim.x * blockDim.x) {
+        const i64 ip = t / n / np, jp = t / n % np, a = min(ip, jp), b = max(ip, jp);
+        out[t] = q[(b * (b + 1) / 2 + a) * n + t % n];
+    }
+}
+
 extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const double *d_dp, double *d_fe,
                                    double *d_fp, double *d_e, void *stream)
 {
@@ -2158,14 +2252,30 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     i64 ne = s->d.nebf, np = s->d.npbf, ne6 = ne * ne * ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
     i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne6));
-    DevBuf X, G, Y, part, fpd;
-    int rc = X.alloc(nb * ne6 * 8);
-    if (!rc) rc = G.alloc(nb * ne6 * 8);
-    if (!rc) rc = Y.alloc(slab_cap(s, 3) * 8);
+    const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
+    DevBuf X, G, Y, part, partq, fpd;
+    int rc = G.alloc(nb * ne6 * 8);
+    if (!rc && !pairs) rc = X.alloc(nb * ne6 * 8);
+    if (!rc && !pairs) rc = Y.alloc(slab_cap(s, 3) * 8);
     if (!rc) rc = part.alloc(npp * ne * (ne + 1) * 8);
+    if (!rc && pairs) rc = partq.alloc(s->plan.nq * ne * (ne + 1) * 8);
     if (!rc) rc = fpd.alloc(npp * 8);
     if (rc) return rc;
-    for (i64 p0 = 0; p0 < npp; p0 += nb) {
+    if (pairs) {
+        for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
+            const i64 q1 = std::min(s->plan.nq, q0 + nb);
+            rc = nrx_gam3_pairs(s, false, q0, q1, 0, G.d(), st);
+            if (rc) return rc;
+            hipLaunchKernelGGL((k_eg3_slab<double, 16, 1>), dim3((unsigned)((q1 - q0) * ne)), dim3(eg3_threads(ne)),
+                               eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G.d(),
+                               partq.d() + q0 * ne * (ne + 1));
+            HIPCHK(hipGetLastError());
+        }
+        hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * (ne + 1), 256)), dim3(256), 0, st, np,
+                           ne * (ne + 1), partq.d(), part.d());
+        HIPCHK(hipGetLastError());
+    }
+    for (i64 p0 = 0; !pairs && p0 < npp; p0 += nb) {
         i64 p1 = std::min(npp, p0 + nb), n = (p1 - p0) * ne6;
         rc = build3_block(s, p0, p1, X.d(), Y.d(), st);
         if (rc) return rc;
