@@ -185,3 +185,6 @@ NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double 
 // [q0, q1).  npbf > 0: into the full tensor G, both orders of each pair;
 // npbf = 0: one block of nebf^6 per pair, from G on.
 NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, hipStream_t st);
+// GAM2_IC1 (G = GM2ICR, Gs = GM2sICR) or, with rxne, RXCHFne_GAM2_IC1 (GM2ICR,
+// GM2exICR), nuclear pairs and blocks as above
+NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 npbf, double *G, double *Gs, hipStream_t st);

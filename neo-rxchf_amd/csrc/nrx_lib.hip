@@ -1023,6 +1023,11 @@ extern "C" int neorx_gam2_ic1_dev(int64_t handle, double *d_gm2, double *d_gm2s,
     if (!d_gm2 || !d_gm2s) return fail(NEORX_E_ARG, "null output");
     i64 ne = s->d.nebf, np = s->d.npbf, ng2 = ne * ne * ne * ne * np * np;
     hipStream_t st = (hipStream_t)stream;
+    if (s->maxl <= 2) {
+        int r = nrx_gam2_pairs(s, false, 0, s->plan.nq, np, d_gm2, d_gm2s, st);
+        if (!r) HIPCHK(hipStreamSynchronize(st));
+        return r;
+    }
     i64 cap = slab_cap(s, 2);
     DevBuf X, Xs, Y, Ys;
     int rc = X.alloc(ng2 * 8);
@@ -2190,6 +2195,15 @@ extern "C" int neorx_precision_switch_dev(int64_t nebf, const double *d_de, doub
 // (ip,jp) pairs at a time, symmetrised and contracted into the Fock partials
 // of that block; no ng2/ng3/ng4 tensor is stored
 // ------------------------------------------------------------------
+// rows of every (ip,jp) from those of the distinct nuclear pairs (n values each)
+__global__ void k_unfold_pairs(i64 np, i64 n, const double *__restrict__ q, double *__restrict__ out)
+{
+    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < np * np * n; t += (i64)gridDim.x * blockDim.x) {
+        const i64 ip = t / n / np, jp = t / n % np, a = min(ip, jp), b = max(ip, jp);
+        out[t] = q[(b * (b + 1) / 2 + a) * n + t % n];
+    }
+}
+
 extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const double *d_dp, double *d_fe,
                                    double *d_fp, double *d_se2, double *d_sp2, double *d_e, double *d_s, void *stream)
 {
@@ -2200,21 +2214,40 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     i64 ne = s->d.nebf, np = s->d.npbf, ne4 = ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
     i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne4));
-    DevBuf X, Xs, G, Gs, Y, Ys, part, fpd, fpsd;
+    const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
+    DevBuf X, Xs, G, Gs, Y, Ys, part, partq, fpd, fpsd;
     i64 cap = slab_cap(s, 2);
-    int rc = X.alloc(nb * ne4 * 8);
-    if (!rc) rc = Xs.alloc(nb * ne4 * 8);
-    if (!rc) rc = G.alloc(nb * ne4 * 8);
+    int rc = G.alloc(nb * ne4 * 8);
     if (!rc) rc = Gs.alloc(nb * ne4 * 8);
-    if (!rc) rc = Y.alloc(cap * 8);
-    if (!rc) rc = Ys.alloc(cap * 8);
+    if (!pairs) {
+        if (!rc) rc = X.alloc(nb * ne4 * 8);
+        if (!rc) rc = Xs.alloc(nb * ne4 * 8);
+        if (!rc) rc = Y.alloc(cap * 8);
+        if (!rc) rc = Ys.alloc(cap * 8);
+    } else if (!rc) {
+        rc = partq.alloc(s->plan.nq * ne * 4 * ne * 8);
+    }
     if (!rc) rc = part.alloc(npp * ne * 4 * ne * 8);
     if (!rc) rc = fpd.alloc(npp * 8);
     if (!rc) rc = fpsd.alloc(npp * 8);
     if (rc) return rc;
     HIPCHK(hipMemsetAsync(fpd.p, 0, npp * 8, st));
     HIPCHK(hipMemsetAsync(fpsd.p, 0, npp * 8, st));
-    for (i64 p0 = 0; p0 < npp; p0 += nb) {
+    if (pairs) {
+        // (underflow() of a primitive value, below 1e-100, is no part of this
+        // form: the values never exist one by one)
+        for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
+            const i64 q1 = std::min(s->plan.nq, q0 + nb);
+            rc = nrx_gam2_pairs(s, false, q0, q1, 0, G.d(), Gs.d(), st);
+            if (!rc)
+                rc = eg2_slab_launch<double>(ne, (q1 - q0) * ne, d_de, G.d(), Gs.d(), partq.d() + q0 * ne * 4 * ne, st);
+            if (rc) return rc;
+        }
+        hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * 4 * ne, 256)), dim3(256), 0, st, np, ne * 4 * ne,
+                           partq.d(), part.d());
+        HIPCHK(hipGetLastError());
+    }
+    for (i64 p0 = 0; !pairs && p0 < npp; p0 += nb) {
         i64 p1 = std::min(npp, p0 + nb), n = (p1 - p0) * ne4;
         rc = build2_block(s, p0, p1, X.d(), Xs.d(), Y.d(), Ys.d(), 1, st);
         if (rc) return rc;
@@ -2230,15 +2263,6 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     return NEORX_OK;
-}
-
-// rows of every (ip,jp) from those of the distinct nuclear pairs (n values each)
-__global__ void k_unfold_pairs(i64 np, i64 n, const double *__restrict__ q, double *__restrict__ out)
-{
-    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < np * np * n; t += (i64)gridDim.x * blockDim.x) {
-        const i64 ip = t / n / np, jp = t / n % np, a = min(ip, jp), b = max(ip, jp);
-        out[t] = q[(b * (b + 1) / 2 + a) * n + t % n];
-    }
 }
 
 extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const double *d_dp, double *d_fe,
@@ -2836,6 +2860,11 @@ extern "C" int neorx_rxchfne_gam2_ic1_dev(int64_t handle, double *d_gm2, double 
     if (!d_gm2 || !d_gm2ex) return fail(NEORX_E_ARG, "null output");
     i64 ne = s->d.nebf, np = s->d.npbf, ng2 = ne * ne * ne * ne * np * np;
     hipStream_t st = (hipStream_t)stream;
+    if (s->maxl <= 2) {
+        int r = nrx_gam2_pairs(s, true, 0, s->plan.nq, np, d_gm2, d_gm2ex, st);
+        if (!r) HIPCHK(hipStreamSynchronize(st));
+        return r;
+    }
     i64 cap = slab_cap(s, 2);
     DevBuf X, Xs, Y, Ys;
     int rc = X.alloc(ng2 * 8);

@@ -1,7 +1,7 @@
-// nrx_stars.hip -- the e-e-e-p tensor GAM_3 from the distinct primitive pairs
-// of its particles (l <= 2).
+// nrx_stars.hip -- the contracted tensors GAM_2, GAM_3 and the RXCHF-ne GAM_2
+// from the distinct primitive pairs of their particles (l <= 2).
 //
-// Every term of the e-e-e-p value is the product of a star -- two electrons
+// GAM_3.  Every term of the e-e-e-p value is the product of a star -- two electrons
 // and the proton joined by their geminals -- or a part of one, with a lone
 // electron that only the Coulomb and one-electron operators reach.  Averaged
 // over the six electron permutations (gam3_IC1_OMP.f:149-263) the tensor is
@@ -24,13 +24,36 @@
 //   k_lone_sum the lone electron's contraction
 //   k_gam3_expand   the sum over c and the full tensor in the reference packing
 //
+// GAM_2 has the same parts.  Averaged over the electrons (gam2_IC1_OMP.f:
+// 141-177),
+//   GM2(a,b) = L(a; b) + L(b; a) + B(a,b),
+//   L(c; a)  = sum_t w_t [ O_t(a,p) h(c) - <1/r_pc> + <1/r_ac> ]
+// over the terms t of X above: a star of one electron with a lone one, again
+// through k_star and k_lone.  B holds what both geminals bond:
+//   B(a,b) = sum_kl b_k b_l [ T + V_p - V_a - V_b - <1/r_ap> - <1/r_bp> + <1/r_ab> ]
+// with g(a,p) = gamma_k and g(b,p) = gamma_l, V the nuclear attractions of the
+// star's members.  The kinetic part T of the average
+// needs no derivative of a geminal under the kinetic operator of the other
+// side: for an electron the two forms of the reference, g g T and g T g, are
+// each other's transpose, and for the proton
+//   (g_a T g_b + g_b T g_a)/2 = (T g_a g_b + g_a g_b T)/2 + (1/2m) grad g_a . grad g_b,
+// so T is the mean of the operator on the bra and on the ket -- one polynomial
+// per pair and direction (k_pair_kin) -- plus (2 gamma_k gamma_l / m)
+// <(r_p - r_a).(r_p - r_b)>.  k_bond evaluates the seven terms, a lane per
+// star, geminal pair and term, at the capacity of the star's powers.
+// RXCHF-ne: GM2 is L with the lone electron second and without h, GM2ex the
+// <1/r_ab> of B.
+//
 // k_lone is bound by FP64 issue: about 150 FMAs per density and lone pair (27
 // densities per star with three geminals), its operands in scalar registers
 // (the star's coefficients are wave-uniform) and LDS.  Lanes over the lone
 // pairs rather than over stars for that reason: a lane per star would read
 // 200 bytes per 150 FMAs.  GAM3_IC1 over 8 contracted functions (16 s/p
 // primitives), 4 nuclear ones: 491 ms a tuple at a time, 6.5 ms here; 7
-// functions in GAM3_DSCF + GAM2_DSCF: 4.38 ms, 0.96 ms.
+// functions in GAM3_DSCF + GAM2_DSCF: 4.38 ms, 0.96 ms.  GAM2_IC1 over 24
+// functions (36 s/p primitives), 8 nuclear: 504 ms, 46.9 ms, of it 41 ms in
+// k_bond and 2.8 ms in k_lone; RXCHFne_GAM2_IC1 over 24 s/p/d functions, 4
+// nuclear: 12.6 ms, 0.96 ms.
 #include "nrx_tuples.h"
 
 namespace {
@@ -271,6 +294,7 @@ struct LoneJob {
     i64 q0, st0, nst; // as the StarJob that filled rec
     int nterm, NE;
     i64 oq;           // output rows between nuclear pairs
+    double hs;        // factor of the overlap x one-electron term (1, or 0 without it)
 };
 
 template <int KIND, int NC, int LMAX>
@@ -334,7 +358,7 @@ __global__ void __launch_bounds__(64) k_lone(DevSys S, PairPlan P, LoneJob J, co
     }
     if (const int pl = P.slot[k]; pl >= 0) {
         const double cp = KIND > 1 ? P.pp_coef[J.q0 + q] : 1.0;
-        out[(q * J.oq + u - J.u0) * P.npl + pl] = cp * (kc * tot + hc * ovt);
+        out[(q * J.oq + u - J.u0) * P.npl + pl] = cp * (kc * tot + J.hs * (hc * ovt));
     }
 }
 
@@ -423,11 +447,280 @@ __global__ void __launch_bounds__(256) k_gam3_expand(PairPlan P, i64 ne, i64 q0,
 }
 
 // ------------------------------------------------------------------
+// GAM_2: the terms that both geminals bond
+// ------------------------------------------------------------------
+constexpr int KT = 7;         // coefficients of a kinetic polynomial (degree <= 2 l + 2)
+
+// -1/4 (u_A K_B + K_A u_B) per direction, u = X^L (X = y + s), K = the second
+// derivative of X^L exp(-beta X^2) over exp(-beta X^2):
+// 4 beta^2 X^{L+2} - 2 beta (2L+1) X^L + L(L-1) X^{L-2}
+NRX_DI void kin_half(int L, double sL, double be, int l, double s, PolyT<KT> &r)
+{
+    p_const(r, 4.0 * be * be);
+    p_mul_lin(r, sL);
+    p_mul_lin(r, sL);
+    r.c[0] -= 2.0 * be * (2 * L + 1);
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, sL, i < L);
+    r.c[0] += L == 2 ? 2.0 : 0.0;
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, s, i < l);
+}
+
+// kinetic polynomials of the pair list, then of the nuclear pairs (times 1/m)
+__global__ void __launch_bounds__(64) k_pair_kin(DevSys S, PairPlan P, double *__restrict__ kt)
+{
+    const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= 3 * (P.npl + P.nq)) return;
+    const i64 k = t / 3;
+    const int d = (int)(t % 3);
+    const bool nuc = k >= P.npl;
+    const PairRec &q = nuc ? S.pp[P.pp_idx[k - P.npl]] : S.ep[P.pl_idx[k]];
+    PolyT<KT> a, b;
+    kin_half(q.lb[d], q.sB[d], q.beta, q.la[d], q.sA[d], a);
+    kin_half(q.la[d], q.sA[d], q.p - q.beta, q.lb[d], q.sB[d], b);
+    const double f = nuc ? -0.25 / S.pmass : -0.25;
+    NRX_UNROLL for (int i = 0; i < KT; ++i) kt[t * KT + i] = f * (a.c[i] + b.c[i]);
+}
+
+// Capacity tiers of a star (largest degree per direction, total degree): the
+// Coulomb terms need NL >= degree + 1 and NB >= total + 1.
+constexpr int BT_N_TIERS = 5;
+constexpr int BTIER_NL[BT_N_TIERS] = {3, 5, 7, 9, 13}, BTIER_NB[BT_N_TIERS] = {5, 7, 9, 13, 13};
+NRX_DI int bond_tier(int m)
+{
+    const int dg = max(deg_of(m, 0), max(deg_of(m, 1), deg_of(m, 2))), L = deg_of(m, 0) + deg_of(m, 1) + deg_of(m, 2);
+    int k = 0;
+    while (k < BT_N_TIERS - 1 && (dg >= BTIER_NL[k] || L >= BTIER_NB[k])) ++k;
+    return k;
+}
+
+__global__ void k_zero_counts(unsigned *p)
+{
+    if (threadIdx.x < 16) p[threadIdx.x] = 0u;
+}
+
+// the stars of a launch sorted by tier (count, then scatter): lists of star
+// numbers, tier by tier from counts[]; cursors at counts + 8
+__global__ void __launch_bounds__(256) k_bond_bin(PairPlan P, StarJob J, int scatter, unsigned *__restrict__ counts,
+                                                  unsigned *__restrict__ list)
+{
+    __shared__ unsigned lc[BT_N_TIERS], lb[BT_N_TIERS];
+    if (threadIdx.x < BT_N_TIERS) lc[threadIdx.x] = 0u;
+    __syncthreads();
+    const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    int tier = -1;
+    unsigned pos = 0;
+    if (t < J.nst * J.nq) {
+        i64 a, b;
+        tri_decode(J.st0 + t % J.nst, b, a);
+        tier = bond_tier(P.pl_deg[a] + P.pl_deg[b] + P.pp_deg[J.q0 + t / J.nst]);
+        pos = atomicAdd(&lc[tier], 1u);
+    }
+    __syncthreads();
+    if (threadIdx.x < BT_N_TIERS) {
+        const unsigned n = lc[threadIdx.x];
+        if (!scatter) {
+            if (n) atomicAdd(&counts[threadIdx.x], n);
+        } else {
+            lb[threadIdx.x] = bin_offset(counts, threadIdx.x) + (n ? atomicAdd(&counts[8 + threadIdx.x], n) : 0u);
+        }
+    }
+    if (!scatter) return;
+    __syncthreads();
+    if (tier >= 0) list[lb[tier] + pos] = (unsigned)t;
+}
+
+// particle i's polynomial f in the hub coordinate (hub_map's map, its
+// Gaussian quantities given)
+template <int NF, int NR>
+NRX_DI void to_hub(const PolyT<NF> &f, double iW, double beta, double m0, PolyT<NR> &r)
+{
+    PolyT<NF> t;
+    p_smooth(f, 0.5 * iW, t);
+    p_compose(t, m0, beta, t);
+    p_copy(t, r);
+}
+
+// kinetic energy T of the star (see the head of the file) and its overlap;
+// kt: the kinetic polynomials of a, b and p
+template <int NL> NRX_DI double bond_kin(const Sys &s, const double *const *kt, double pmass, double &ovl)
+{
+    constexpr int ND = NL + 2; // kinetic terms raise the degree by 2
+    constexpr int FS = NS < NL ? NS : NL, FT = KT < ND ? KT : ND, FR = FS + 1;
+    const double ga = s.gam[0], gb = s.gam[1], cross = 2.0 * ga * gb / pmass;
+    double Pr = 1.0, R = 0.0;
+    NRX_DIRS for (int d = 0; d < 3; ++d) {
+        double w = s.q[2]->p, cq = 0.0, fac = 1.0, iW[2], be[2], m0[2], dl[2];
+        NRX_UNROLL for (int i = 0; i < 2; ++i) {
+            const PairRec &Q = *s.q[i];
+            const double g = s.gam[i], rW = rsqrt(Q.p + g);
+            iW[i] = rW * rW;
+            be[i] = g * iW[i];
+            dl[i] = Q.P[d] - s.q[2]->P[d];
+            m0[i] = -be[i] * dl[i];
+            const double kap = Q.p * be[i], Wq = w + kap, iWq = rcp(Wq), df = cq - dl[i];
+            fac *= sqrt(PI) * rW * exp(-(w * kap * iWq) * df * df);
+            cq = (w * cq + kap * dl[i]) * iWq;
+            w = Wq;
+        }
+        const double rw = rsqrt(w), iw = rw * rw, norm = fac * (sqrt(PI) * rw);
+        PolyT<FS> f;
+        PolyT<FS> ma, mb;
+        PolyT<FT> ta, tb;
+        PolyT<FR> ra, rb; // (r_p - r_i)_d times the polynomial of i
+        PolyT<FT> x;
+        x.n = FT;
+        auto maps = [&](int i, PolyT<FS> &m, PolyT<FT> &tm, PolyT<FR> &rr) {
+            fpoly(*s.q[i], d, f);
+            to_hub(f, iW[i], be[i], m0[i], m);
+            NRX_UNROLL for (int k = 0; k < FT; ++k) x.c[k] = kt[i][d * KT + k];
+            to_hub(x, iW[i], be[i], m0[i], tm);
+            // y_p - y_i - (P_i - P_p)
+            PolyT<FR> yf, ym;
+            NRX_UNROLL for (int k = 0; k < FR; ++k) yf.c[k] = k ? f.c[k - 1] : 0.0;
+            yf.n = FR;
+            to_hub(yf, iW[i], be[i], m0[i], ym);
+            NRX_UNROLL for (int k = 0; k < FR; ++k)
+                rr.c[k] = (k ? m.c[k - 1] : 0.0) - (k < FS ? dl[i] * m.c[k] : 0.0) - ym.c[k];
+            rr.n = FR;
+        };
+        maps(0, ma, ta, ra);
+        maps(1, mb, tb, rb);
+        PolyT<ND> q, ab, u;
+        p_mul(ma, mb, ab);
+        NRX_UNROLL for (int k = 0; k < FT; ++k) x.c[k] = kt[2][d * KT + k];
+        p_mul(ab, x, q);
+        p_mul(ta, mb, u);
+        PolyT<ND> v;
+        p_mul(ma, tb, v);
+        NRX_UNROLL for (int k = 0; k < ND; ++k) u.c[k] += v.c[k];
+        p_mul(ra, rb, v);
+        NRX_UNROLL for (int k = 0; k < ND; ++k) u.c[k] += cross * v.c[k];
+        fpoly(*s.q[2], d, f);
+        p_mul(u, f, u);
+        NRX_UNROLL for (int k = 0; k < ND; ++k) q.c[k] += u.c[k];
+        const double Td = norm * close_expect(q, iw, cq);
+        PolyT<NL> so;
+        p_mul(ab, f, so);
+        const double Sd = norm * close_expect(so, iw, cq);
+        R = R * Sd + Pr * Td;
+        Pr *= Sd;
+    }
+    const double K = s.q[0]->K * s.q[1]->K * s.q[2]->K;
+    ovl = K * Pr;
+    return K * R;
+}
+
+// The rows of a launch's values: a row per term and geminal pair, the launch's
+// stars along it.  All: every term of B and the overlap; rxne: <1/r_ab> alone.
+enum { BT_KIN = 0, BT_AP, BT_BP, BT_AB, BT_NP, BT_NA, BT_NB, BT_OVL, BT_ROWS };
+
+// Term blockIdx.y (or <1/r_ab>, rxne) of the tier's stars: a lane per star, the
+// geminal pair uniform over most waves, striding over the tier's list.
+// The kernel is bound by FP64 issue at one or two waves per SIMD: the
+// polynomial tables of a term fill the registers.
+template <int TIER>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(TIER < 2 ? 2 : 1)))
+k_bond(DevSys S, PairPlan P, StarJob J, int rxne, const double *__restrict__ kt, const unsigned *__restrict__ counts,
+       const unsigned *__restrict__ list, double *__restrict__ val)
+{
+    constexpr int NL = BTIER_NL[TIER], NBC = BTIER_NB[TIER];
+    const unsigned off = bin_offset(counts, TIER);
+    const i64 cnt = counts[TIER], nkl = J.nterm, row = J.nst * J.nq;
+    const int term = rxne ? BT_AB : (int)blockIdx.y;
+    for (i64 t = (i64)blockIdx.x * 64 + threadIdx.x; t < cnt * nkl; t += (i64)gridDim.x * 64) {
+        const i64 star = list[off + t % cnt], k = t / cnt, q = J.q0 + star / J.nst;
+        i64 a, b;
+        tri_decode(J.st0 + star % J.nst, b, a);
+        SysParams SP = d_params(S);
+        Sys s = mksys(SP, 3, S.ep + P.pl_idx[a], S.ep + P.pl_idx[b], S.pp + P.pp_idx[q], 0, J.gk[k], J.gl[k], 0);
+        double v;
+        if (term == BT_KIN) {
+            const double *kp[3] = {kt + a * 3 * KT, kt + b * 3 * KT, kt + (P.npl + q) * 3 * KT};
+            double o;
+            v = bond_kin<NL>(s, kp, S.pmass, o);
+            val[(BT_OVL * nkl + k) * row + star] = J.w[k] * o;
+        } else if (term <= BT_BP) {
+            v = -coul<NL, NBC>(s, term == BT_AP ? 0 : 1, 2);
+        } else if (term == BT_AB) {
+            v = coul<NL, NBC>(s, 0, 1);
+        } else if (term == BT_NP) {
+            v = nuc_sum<NL, NBC>(s, 2, S.nat, S.cat, S.zan, false);
+        } else {
+            v = -nuc_sum<NL, NBC>(s, term == BT_NA ? 0 : 1, S.nat, S.cat, S.zan, false);
+        }
+        val[((rxne ? 0 : term) * nkl + k) * row + star] = J.w[k] * v;
+    }
+}
+
+// row 0 of the values becomes the sum of rows 0 .. nB-1 (B of a primitive
+// star), row 1 that of the nO rows from rO on (its overlap)
+__global__ void __launch_bounds__(256) k_bond_rows(i64 n, i64 nB, i64 rO, i64 nO, double *__restrict__ val)
+{
+    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (i64)gridDim.x * blockDim.x) {
+        double e = 0.0, y = 0.0;
+        for (i64 k = 0; k < nB; ++k) e += val[k * n + t];
+        for (i64 k = 0; k < nO; ++k) y += val[(rO + k) * n + t];
+        val[t] = e;
+        if (nO) val[n + t] = y;
+    }
+}
+
+// contracted stars: B[q][u] and Y[q][u] (null to skip), sums over their
+// primitive stars of the value rows 0 and 1
+__global__ void __launch_bounds__(256) k_bond_sum(PairPlan P, StarJob J, LoneJob L, const double *__restrict__ val,
+                                                  double *__restrict__ B, double *__restrict__ Y)
+{
+    const i64 n = L.nu * J.nq, row = J.nst * J.nq;
+    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < n; t += (i64)gridDim.x * blockDim.x) {
+        const i64 q = t / L.nu, u = L.u0 + t % L.nu;
+        i64 Bc, Ac;
+        tri_decode(u, Bc, Ac);
+        double e = 0.0, y = 0.0;
+        for (int b = P.cp_start[Bc]; b < P.cp_start[Bc + 1]; ++b)
+            for (int a = P.cp_start[Ac]; a < (Ac == Bc ? b + 1 : P.cp_start[Ac + 1]); ++a) {
+                const i64 star = q * J.nst + (i64)b * (b + 1) / 2 + a - J.st0;
+                const double cf = P.pl_coef[a] * P.pl_coef[b] * (Ac == Bc && a < b ? 2.0 : 1.0);
+                e += cf * val[star];
+                if (Y) y += cf * val[row + star];
+            }
+        const double cp = P.pp_coef[J.q0 + q];
+        B[q * L.oq + t % L.nu] = cp * e;
+        if (Y) Y[q * L.oq + t % L.nu] = cp * y;
+    }
+}
+
+// Full tensors of the nuclear pairs q0 ..: G = L(a;b) + L(b;a) + B, Gs = Y
+// (ne = 0), or with ne set G = 2 L[a][b] (star electron first), Gs = B.  np > 0: every (ip,jp)
+// of the full tensor; np = 0: one block per pair.
+__global__ void __launch_bounds__(256) k_gam2_expand(i64 ne, i64 nc, i64 q0, i64 nq, i64 np, int rxne,
+                                                     const double *__restrict__ Lq, const double *__restrict__ B,
+                                                     const double *__restrict__ Y, double *__restrict__ G,
+                                                     double *__restrict__ Gs)
+{
+    const i64 ne2 = ne * ne, ne4 = ne2 * ne2, ntri = nc * (nc + 1) / 2, nblk = np > 0 ? np * np : nq;
+    for (i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x; t < nblk * ne4; t += (i64)gridDim.x * blockDim.x) {
+        const i64 blk = t / ne4, p1 = t / ne2 % ne2, p2 = t % ne2;
+        const i64 q = np > 0 ? tri_index(blk / np, blk % np) - q0 : blk;
+        const i64 A = tri_index(p1 / ne, p1 % ne), C = tri_index(p2 / ne, p2 % ne), u = q * ntri + tri_index(A, C);
+        const double l1 = Lq[(q * nc + A) * nc + C];
+        if (rxne) {
+            G[t] = 2.0 * l1;
+            Gs[t] = B[u];
+        } else {
+            G[t] = l1 + Lq[(q * nc + C) * nc + A] + B[u];
+            Gs[t] = Y[u];
+        }
+    }
+}
+
+// ------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------
 // bytes of star records and lone partial sums of one launch; they stay in the
 // last-level cache
 constexpr i64 REC_BYTES = (i64)192 << 20;
+// most blocks of one k_bond launch and term; the blocks stride over the list
+constexpr i64 BOND_BLOCKS = 8192;
 // bytes of contracted star values T held at once (at least one nuclear pair)
 constexpr i64 T_BYTES = (i64)4 << 30;
 
@@ -519,7 +812,7 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
     double *T = (double *)wT.p, *rec = (double *)wR.p;
     { // V: pair densities and lone pairs
         StarJob J{0, P.npl, 0, 1, 1, NE1, P.one + 1, P.one + 1, P.one};
-        LoneJob L{0, nc, 0, 0, P.npl, 1, NE1, nc};
+        LoneJob L{0, nc, 0, 0, P.npl, 1, NE1, nc, 0.0};
         rc = star_launch<1>(d, P, J, rec, st);
         if (!rc) rc = lone_launch<1>(d, P, L, 1, rec, lone, Vp, st);
         if (rc) return rc;
@@ -541,7 +834,7 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
                 // T[q][u][C], straight from the lanes or through the sums over lone primitives
                 double *part = rec + nq * nst * nt * 3 * RS, *o = T + (k * ntri + u0) * nc;
                 const bool sum = P.npl > nc;
-                LoneJob L{u0, nu, q + k, st0, nst, nt, NE, sum ? nu : ntri};
+                LoneJob L{u0, nu, q + k, st0, nst, nt, NE, sum ? nu : ntri, 1.0};
                 rc = lone_launch<3>(d, P, L, nq, rec, lone, sum ? part : o, st);
                 if (rc) return rc;
                 if (sum) {
@@ -556,5 +849,92 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
                            X + (q - q0) * nc, O);
         HIPCHK(hipGetLastError());
     }
+    return NEORX_OK;
+}
+
+// GAM_2 and its overlaps (rxne: the RXCHF-ne tensors) of the distinct nuclear
+// pairs [q0, q1)
+int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G, double *Gs, hipStream_t st)
+{
+    const DevSys &d = s->d;
+    const PairPlan &P = s->plan;
+    const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2, nqa = q1 - q0;
+    const int ng = (int)d.ngtg, nt = ng * ng, nx = ng * (ng + 1) / 2 + (rxne ? 0 : ng);
+    const int NE2 = rec_ne(2 * P.le + 2 * P.lp), nterms = rxne ? 1 : BT_OVL;
+    const i64 nrows = (i64)nt * (rxne ? 1 : BT_ROWS);
+    StreamBuf w0, wR;
+    int rc = w0.alloc((LONE_F * P.nslot + 3 * KT * (P.npl + P.nq) + nqa * (nc * nc + 2 * ntri)) * 8 + 64, st);
+    if (rc) return rc;
+    double *lone = (double *)w0.p, *kt = lone + LONE_F * P.nslot, *L = kt + 3 * KT * (P.npl + P.nq),
+           *B = L + nqa * nc * nc, *Y = B + nqa * ntri;
+    unsigned *counts = (unsigned *)(Y + nqa * ntri);
+    hipLaunchKernelGGL(k_lone_prep, dim3((unsigned)(P.nslot / 64)), dim3(64), 0, st, d, P, lone);
+    hipLaunchKernelGGL(k_pair_kin, dim3(nblocks(3 * (P.npl + P.nq), 64)), dim3(64), 0, st, d, P, kt);
+    HIPCHK(hipGetLastError());
+    // bytes per primitive star of the bond terms (values, list entry; two rows
+    // at least for the sums) and per nuclear pair of the lone part
+    const i64 star_b = std::max<i64>(nrows, 2) * 8 + 4;
+    const i64 lone_b = (P.npl * nx * 2 * (REC_HEAD + 3 * NE2) + (P.npl > nc ? nc * P.npl : 0)) * 8;
+    auto span = [&](i64 B0, i64 B1, i64 &nst, i64 &nu) {
+        const i64 a = s->cp_start[B0], b = s->cp_start[B1];
+        nst = b * (b + 1) / 2 - a * (a + 1) / 2;
+        nu = B1 * (B1 + 1) / 2 - B0 * (B0 + 1) / 2;
+        return nst * star_b;
+    };
+    i64 nst = 0, nu = 0, big = 0;
+    for (i64 k = 0; k < nc; ++k) big = std::max(big, span(k, k + 1, nst, nu));
+    const i64 all = span(0, nc, nst, nu);
+    const i64 nqr = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / big));
+    const i64 nql = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / lone_b));
+    if ((rc = wR.alloc(std::max({nql * lone_b, nqr * big, std::min(nqr * all, REC_BYTES)}), st))) return rc;
+    double *rec = (double *)wR.p;
+    for (i64 q = q0; q < q1; q += nql) { // L
+        const i64 nq = std::min(nql, q1 - q);
+        StarJob J{0, P.npl, q, nq, nx, NE2, P.gx + (rxne ? ng : 0), P.gx, P.wx + (rxne ? ng : 0)};
+        LoneJob Lj{0, nc, q, 0, P.npl, nx, NE2, nc, rxne ? 0.0 : 1.0};
+        double *part = rec + nq * P.npl * nx * 2 * (REC_HEAD + 3 * NE2), *o = L + (q - q0) * nc * nc;
+        rc = star_launch<2>(d, P, J, rec, st);
+        if (!rc) rc = lone_launch<2>(d, P, Lj, nq, rec, lone, P.npl > nc ? part : o, st);
+        if (rc) return rc;
+        if (P.npl > nc)
+            hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nc * nq * nc, 256)), dim3(256), 0, st, P, nc, nq, nc, part, o);
+        HIPCHK(hipGetLastError());
+    }
+    const int dmax = 4 * P.le + 2 * P.lp; // per direction and in total
+    for (i64 q = q0; q < q1; q += nqr) { // B, Y
+        const i64 nq = std::min(nqr, q1 - q);
+        for (i64 B0 = 0, B1; B0 < nc; B0 = B1) {
+            B1 = B0 + 1;
+            while (B1 < nc && nq * span(B0, B1 + 1, nst, nu) <= REC_BYTES) ++B1;
+            span(B0, B1, nst, nu);
+            const i64 s0 = s->cp_start[B0], n = nst * nq;
+            StarJob J{s0 * (s0 + 1) / 2, nst, q, nq, nt, 0, P.gk, P.gl, P.wkl};
+            LoneJob U{B0 * (B0 + 1) / 2, nu, q, 0, 0, 0, 0, ntri, 0.0};
+            unsigned *list = (unsigned *)(rec + std::max<i64>(nrows, 2) * n);
+            hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, counts);
+            hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 0, counts, list);
+            hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 1, counts, list);
+            const dim3 g((unsigned)std::min<i64>(BOND_BLOCKS, (n * nt + 63) / 64), (unsigned)nterms);
+#define NRX_BOND(K)                                                                                                   \
+    if (K == 0 || dmax >= BTIER_NL[K ? K - 1 : 0] || dmax >= BTIER_NB[K ? K - 1 : 0])                                 \
+    hipLaunchKernelGGL((k_bond<K>), g, dim3(64), 0, st, d, P, J, (int)rxne, kt, counts, list, rec)
+            NRX_BOND(4);
+            NRX_BOND(3);
+            NRX_BOND(2);
+            NRX_BOND(1);
+            NRX_BOND(0);
+#undef NRX_BOND
+            hipLaunchKernelGGL(k_bond_rows, dim3(grid_blocks(n, 256)), dim3(256), 0, st, n, (i64)nterms * nt,
+                               (i64)BT_OVL * nt, rxne ? (i64)0 : (i64)nt, rec);
+            const i64 o = (q - q0) * ntri + U.u0;
+            hipLaunchKernelGGL(k_bond_sum, dim3(grid_blocks(nu * nq, 256)), dim3(256), 0, st, P, J, U, rec,
+                               B + o, rxne ? nullptr : Y + o);
+            HIPCHK(hipGetLastError());
+        }
+    }
+    const i64 nout = (np_full > 0 ? np_full * np_full : nqa) * ne * ne * ne * ne;
+    hipLaunchKernelGGL(k_gam2_expand, dim3(grid_blocks(nout, 256)), dim3(256), 0, st, ne, nc, q0, nqa, np_full, (int)rxne,
+                       L, B, Y, G, Gs);
+    HIPCHK(hipGetLastError());
     return NEORX_OK;
 }

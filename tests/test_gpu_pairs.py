@@ -89,3 +89,24 @@ def test_gam3_from_pairs(torch_dev, name):
         assert np.isfinite(g).all()
         check_close(np.append(got, np.abs(g).max()), np.append(ref, np.abs(g).max()), what=f"class {cls}")
     S.close()
+
+
+@pytest.mark.parametrize("name", SYSTEMS)
+def test_gam2_from_pairs(torch_dev, name):
+    """GAM2_IC1 (class 2, averaged over the electrons) and RXCHFne_GAM2_IC1
+    (class 4: the first output as it is, the second averaged)."""
+    s = synth.small(**SYSTEMS[name])
+    S = neorx.System(s)
+    en = sample(s, 2, 60, 12)
+    at = flat_index(s, en)
+    print(f"case gam2 pairs {name} nebf={s['nebf']} npebf={s['npebf']} npbf={s['npbf']}", flush=True)
+    both = list(permutations(range(2)))
+    sym2, sym4 = (contracted(torch_dev, S, s, c, 2, en, both) for c in (2, 4))
+    one4 = contracted(torch_dev, S, s, 4, 2, en, both[:1])
+    g, gs = S.GAM2_IC1()
+    n, nx = S.RXCHFne_GAM2_IC1()
+    for got, ref, what in ((g, sym2[:, 0], "GM2ICR"), (gs, sym2[:, 1], "GM2sICR"), (n, one4[:, 0], "RXCHF-ne GM2ICR"),
+                           (nx, sym4[:, 1], "GM2exICR")):
+        assert np.isfinite(got).all()
+        check_close(np.append(got[at], np.abs(got).max()), np.append(ref, np.abs(got).max()), what=what)
+    S.close()
