@@ -151,6 +151,28 @@ struct StreamBuf {
     }
 };
 
+// Scratch of one call that ends by synchronising its stream.  The blocks go
+// back to a process-wide free list (per device, at most WORK_KEEP bytes, the
+// oldest released first; larger blocks are freed) once the stream has drained,
+// so no two calls in flight share one, whatever their threads and streams.
+// neorx_release_resident and neorx_finalize empty the list.  A device
+// allocation costs 0.1 ms or more, as much as a small builder's kernels.
+struct Work {
+    hipStream_t st;
+    struct Block {
+        int dev;
+        void *p;
+        size_t n;
+    };
+    std::vector<Block> held;
+    explicit Work(hipStream_t s) : st(s) {}
+    Work(const Work &) = delete;
+    Work &operator=(const Work &) = delete;
+    NRX_HIDDEN ~Work();
+    NRX_HIDDEN int get(void **p, size_t bytes);
+    int get(double *&p, i64 n) { return get((void **)&p, (size_t)n * 8); }
+};
+
 // storage type of an in-core tensor read by the contractions
 enum { NRX_F64 = 0, NRX_F32 = 1, NRX_BF16 = 2 };
 
@@ -178,13 +200,13 @@ NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double 
                              hipStream_t st);
 
 // ------------------------------------------------------------------
-// tensors from distinct pairs (nrx_stars.hip), l <= 2.  Enqueued on st, with
-// stream-ordered scratch.
+// tensors from distinct pairs (nrx_stars.hip), l <= 2.  Enqueued on W's
+// stream, with scratch from W.
 // ------------------------------------------------------------------
 // GAM3_IC1 (mult: RXCHFmult_GAM3_XCHF) of the distinct nuclear pairs
 // [q0, q1).  npbf > 0: into the full tensor G, both orders of each pair;
 // npbf = 0: one block of nebf^6 per pair, from G on.
-NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, hipStream_t st);
+NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, Work &W);
 // GAM2_IC1 (G = GM2ICR, Gs = GM2sICR) or, with rxne, RXCHFne_GAM2_IC1 (GM2ICR,
 // GM2exICR), nuclear pairs and blocks as above
-NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 npbf, double *G, double *Gs, hipStream_t st);
+NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 npbf, double *G, double *Gs, Work &W);

@@ -82,6 +82,74 @@ System *get_sys(i64 h)
     return it == g_sys.end() ? nullptr : it->second;
 }
 
+// free list of Work blocks, oldest first
+namespace {
+std::mutex g_work_mu;
+std::vector<Work::Block> g_work;
+constexpr size_t WORK_KEEP = (size_t)512 << 20;
+
+void work_release()
+{
+    std::lock_guard<std::mutex> lk(g_work_mu);
+    for (auto &b : g_work) (void)hipFree(b.p);
+    g_work.clear();
+}
+} // namespace
+
+int Work::get(void **p, size_t bytes)
+{
+    Block b{0, nullptr, std::max<size_t>(bytes, 8)};
+    HIPCHK(hipGetDevice(&b.dev));
+    {
+        // the smallest block that holds the request without wasting most of itself
+        std::lock_guard<std::mutex> lk(g_work_mu);
+        size_t best = g_work.size();
+        for (size_t i = 0; i < g_work.size(); ++i)
+            if (g_work[i].dev == b.dev && g_work[i].n >= b.n && g_work[i].n <= 2 * b.n + ((size_t)1 << 20) &&
+                (best == g_work.size() || g_work[i].n < g_work[best].n))
+                best = i;
+        if (best < g_work.size()) {
+            b = g_work[best];
+            g_work.erase(g_work.begin() + (long)best);
+        }
+    }
+    if (!b.p) {
+        b.n = (b.n + 65535) / 65536 * 65536;
+        hipError_t e = hipMalloc(&b.p, b.n);
+        if (e != hipSuccess) { // give the kept blocks up first
+            (void)hipGetLastError();
+            work_release();
+            e = hipMalloc(&b.p, b.n);
+        }
+        if (e != hipSuccess) return fail(NEORX_E_NOMEM, "hipMalloc(%zu) failed: %s", b.n, hipGetErrorString(e));
+    }
+    held.push_back(b);
+    *p = b.p;
+    return NEORX_OK;
+}
+
+Work::~Work()
+{
+    if (held.empty()) return;
+    (void)hipStreamSynchronize(st);
+    std::lock_guard<std::mutex> lk(g_work_mu);
+    size_t kept = 0;
+    for (auto &b : g_work) kept += b.n;
+    for (auto &b : held) {
+        if (b.n > WORK_KEEP / 2) {
+            (void)hipFree(b.p);
+            continue;
+        }
+        while (kept + b.n > WORK_KEEP) {
+            kept -= g_work.front().n;
+            (void)hipFree(g_work.front().p);
+            g_work.erase(g_work.begin());
+        }
+        g_work.push_back(b);
+        kept += b.n;
+    }
+}
+
 extern "C" int neorx_init(int64_t device)
 {
     std::lock_guard<std::mutex> lk(g_mu);
@@ -906,6 +974,7 @@ void res_keep(DevBuf &b, const double *h, i64 n)
 
 extern "C" int neorx_release_resident(void)
 {
+    work_release();
     std::lock_guard<std::mutex> lk(g_res_mu);
     while (!g_res.empty()) res_drop_locked(g_res.size() - 1);
     return NEORX_OK;
@@ -1024,7 +1093,8 @@ extern "C" int neorx_gam2_ic1_dev(int64_t handle, double *d_gm2, double *d_gm2s,
     i64 ne = s->d.nebf, np = s->d.npbf, ng2 = ne * ne * ne * ne * np * np;
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
-        int r = nrx_gam2_pairs(s, false, 0, s->plan.nq, np, d_gm2, d_gm2s, st);
+        Work W(st);
+        int r = nrx_gam2_pairs(s, false, 0, s->plan.nq, np, d_gm2, d_gm2s, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }
@@ -1049,7 +1119,8 @@ template <int CLS> static int gam3_build_dev(System *s, double *d_gm3, void *str
     i64 ne = s->d.nebf, np = s->d.npbf, blk = ne * ne * ne * ne * ne * ne;
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
-        int r = nrx_gam3_pairs(s, CLS == 7, 0, s->plan.nq, np, d_gm3, st);
+        Work W(st);
+        int r = nrx_gam3_pairs(s, CLS == 7, 0, s->plan.nq, np, d_gm3, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }
@@ -1359,6 +1430,12 @@ __global__ void k_eg2_reduce(i64 ne, i64 np, const double *__restrict__ DE, cons
     }
 }
 
+__global__ void k_zero(i64 n, double *__restrict__ x)
+{
+    i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < n) x[t] = 0.0;
+}
+
 // y += x
 __global__ void k_axpy(i64 n, const double *__restrict__ x, double *__restrict__ y)
 {
@@ -1391,28 +1468,28 @@ static int eg2_dev(int64_t nebf, int64_t npbf, const double *d_de, const double 
     if (ne <= 0 || np <= 0) return fail(NEORX_E_ARG, "bad sizes");
     hipStream_t st = (hipStream_t)stream;
     i64 nblk = np * np * ne;
-    DevBuf part, fpd, fpsd;
-    rc = part.alloc(nblk * 4 * ne * 8);
-    if (!rc) rc = fpd.alloc(np * np * 8);
-    if (!rc) rc = fpsd.alloc(np * np * 8);
+    Work W(st);
+    double *part, *fpd;
+    rc = W.get(part, nblk * 4 * ne + 2 * np * np);
     if (rc) return rc;
-    HIPCHK(hipMemsetAsync(fpd.p, 0, np * np * 8, st));
-    HIPCHK(hipMemsetAsync(fpsd.p, 0, np * np * 8, st));
-    rc = eg2_slab_launch<T>(ne, nblk, d_de, d_gm2, d_gm2s, part.d(), st);
+    fpd = part + nblk * 4 * ne;
+    double *fpsd = fpd + np * np;
+    hipLaunchKernelGGL(k_zero, dim3(nblocks(2 * np * np, 256)), dim3(256), 0, st, 2 * np * np, fpd);
+    rc = eg2_slab_launch<T>(ne, nblk, d_de, d_gm2, d_gm2s, part, st);
     if (rc) return rc;
     int withS = d_gm2s != nullptr;
     // FE/SE and the per-(ip,jp) proton terms into fpd/fpsd; then add fpd to FP
     hipLaunchKernelGGL(k_eg2_reduce, dim3(nblocks(ne * ne + np * np, 256)), dim3(256), 0, st, ne, np, d_de, d_dp,
-                       part.d(), withS, 0, d_fe, d_se, fpd.d(), fpsd.d(), d_e, d_s);
+                       part, withS, 0, d_fe, d_se, fpd, fpsd, d_e, d_s);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd.d(), withS ? fpsd.d() : nullptr, d_e,
+    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd, withS ? fpsd : nullptr, d_e,
                        withS ? d_s : nullptr);
     HIPCHK(hipGetLastError());
     // FP accumulates (add2fock), SP is overwritten
-    hipLaunchKernelGGL(k_axpy, dim3(nblocks(np * np, 256)), dim3(256), 0, st, np * np, fpd.d(), d_fp);
+    hipLaunchKernelGGL(k_axpy, dim3(nblocks(np * np, 256)), dim3(256), 0, st, np * np, fpd, d_fp);
     HIPCHK(hipGetLastError());
-    if (withS && d_sp) HIPCHK(hipMemcpyAsync(d_sp, fpsd.p, np * np * 8, hipMemcpyDeviceToDevice, st));
-    HIPCHK(hipStreamSynchronize(st)); // scratch buffers are released on return
+    if (withS && d_sp) HIPCHK(hipMemcpyAsync(d_sp, fpsd, np * np * 8, hipMemcpyDeviceToDevice, st));
+    HIPCHK(hipStreamSynchronize(st)); // the scratch goes back on return
     return NEORX_OK;
 }
 
@@ -1914,18 +1991,19 @@ static int eg3_dev(int64_t nebf, int64_t npbf, const double *d_de, const double 
     if (ne > EG3_MAX_NE) return fail(NEORX_E_UNSUPPORTED, "EG3IC1: nebf=%lld > %lld", (long long)ne, (long long)EG3_MAX_NE);
     hipStream_t st = (hipStream_t)stream;
     i64 nblk = np * np * ne;
-    DevBuf part, fpd;
-    rc = part.alloc(nblk * (ne + 1) * 8);
-    if (!rc) rc = fpd.alloc(np * np * 8);
+    Work W(st);
+    double *part;
+    rc = W.get(part, nblk * (ne + 1) + np * np);
     if (rc) return rc;
-    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, sizeof(T) == 8 ? NRX_F64 : NRX_F32, part.d(), st);
+    double *fpd = part + nblk * (ne + 1);
+    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, sizeof(T) == 8 ? NRX_F64 : NRX_F32, part, st);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + np * np, 256)), dim3(256), 0, st, ne, np, d_dp, part.d(),
-                       d_fe, fpd.d());
+    hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + np * np, 256)), dim3(256), 0, st, ne, np, d_dp, part,
+                       d_fe, fpd);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd.d(), nullptr, d_e, nullptr);
+    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd, nullptr, d_e, nullptr);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(k_axpy, dim3(nblocks(np * np, 256)), dim3(256), 0, st, np * np, fpd.d(), d_fp);
+    hipLaunchKernelGGL(k_axpy, dim3(nblocks(np * np, 256)), dim3(256), 0, st, np * np, fpd, d_fp);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     return NEORX_OK;
@@ -2215,51 +2293,51 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     hipStream_t st = (hipStream_t)stream;
     i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne4));
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
-    DevBuf X, Xs, G, Gs, Y, Ys, part, partq, fpd, fpsd;
+    Work W(st);
+    double *X = nullptr, *Xs = nullptr, *Y = nullptr, *Ys = nullptr, *partq = nullptr, *G, *Gs, *part, *fpd;
     i64 cap = slab_cap(s, 2);
-    int rc = G.alloc(nb * ne4 * 8);
-    if (!rc) rc = Gs.alloc(nb * ne4 * 8);
+    int rc = W.get(G, nb * ne4);
+    if (!rc) rc = W.get(Gs, nb * ne4);
     if (!pairs) {
-        if (!rc) rc = X.alloc(nb * ne4 * 8);
-        if (!rc) rc = Xs.alloc(nb * ne4 * 8);
-        if (!rc) rc = Y.alloc(cap * 8);
-        if (!rc) rc = Ys.alloc(cap * 8);
+        if (!rc) rc = W.get(X, nb * ne4);
+        if (!rc) rc = W.get(Xs, nb * ne4);
+        if (!rc) rc = W.get(Y, cap);
+        if (!rc) rc = W.get(Ys, cap);
     } else if (!rc) {
-        rc = partq.alloc(s->plan.nq * ne * 4 * ne * 8);
+        rc = W.get(partq, s->plan.nq * ne * 4 * ne);
     }
-    if (!rc) rc = part.alloc(npp * ne * 4 * ne * 8);
-    if (!rc) rc = fpd.alloc(npp * 8);
-    if (!rc) rc = fpsd.alloc(npp * 8);
+    if (!rc) rc = W.get(part, npp * ne * 4 * ne + 2 * npp);
     if (rc) return rc;
-    HIPCHK(hipMemsetAsync(fpd.p, 0, npp * 8, st));
-    HIPCHK(hipMemsetAsync(fpsd.p, 0, npp * 8, st));
+    fpd = part + npp * ne * 4 * ne;
+    double *fpsd = fpd + npp;
+    hipLaunchKernelGGL(k_zero, dim3(nblocks(2 * npp, 256)), dim3(256), 0, st, 2 * npp, fpd);
     if (pairs) {
         // (underflow() of a primitive value, below 1e-100, is no part of this
         // form: the values never exist one by one)
         for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
             const i64 q1 = std::min(s->plan.nq, q0 + nb);
-            rc = nrx_gam2_pairs(s, false, q0, q1, 0, G.d(), Gs.d(), st);
+            rc = nrx_gam2_pairs(s, false, q0, q1, 0, G, Gs, W);
             if (!rc)
-                rc = eg2_slab_launch<double>(ne, (q1 - q0) * ne, d_de, G.d(), Gs.d(), partq.d() + q0 * ne * 4 * ne, st);
+                rc = eg2_slab_launch<double>(ne, (q1 - q0) * ne, d_de, G, Gs, partq + q0 * ne * 4 * ne, st);
             if (rc) return rc;
         }
         hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * 4 * ne, 256)), dim3(256), 0, st, np, ne * 4 * ne,
-                           partq.d(), part.d());
+                           partq, part);
         HIPCHK(hipGetLastError());
     }
     for (i64 p0 = 0; !pairs && p0 < npp; p0 += nb) {
         i64 p1 = std::min(npp, p0 + nb), n = (p1 - p0) * ne4;
-        rc = build2_block(s, p0, p1, X.d(), Xs.d(), Y.d(), Ys.d(), 1, st);
+        rc = build2_block(s, p0, p1, X, Xs, Y, Ys, 1, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_gam2_symm, dim3(grid_blocks(n, 256)), dim3(256), 0, st, ne, n, X.d(), Xs.d(), G.d(), Gs.d());
-        rc = eg2_slab_launch<double>(ne, (p1 - p0) * ne, d_de, G.d(), Gs.d(), part.d() + p0 * ne * 4 * ne, st);
+        hipLaunchKernelGGL(k_gam2_symm, dim3(grid_blocks(n, 256)), dim3(256), 0, st, ne, n, X, Xs, G, Gs);
+        rc = eg2_slab_launch<double>(ne, (p1 - p0) * ne, d_de, G, Gs, part + p0 * ne * 4 * ne, st);
         if (rc) return rc;
     }
-    hipLaunchKernelGGL(k_eg2_reduce, dim3(nblocks(ne * ne + npp, 256)), dim3(256), 0, st, ne, np, d_de, d_dp, part.d(),
-                       1, 1, d_fe, d_se2, fpd.d(), fpsd.d(), d_e, d_s);
-    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd.d(), fpsd.d(), d_e, d_s);
-    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpd.d(), d_fp);
-    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpsd.d(), d_sp2);
+    hipLaunchKernelGGL(k_eg2_reduce, dim3(nblocks(ne * ne + npp, 256)), dim3(256), 0, st, ne, np, d_de, d_dp, part,
+                       1, 1, d_fe, d_se2, fpd, fpsd, d_e, d_s);
+    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd, fpsd, d_e, d_s);
+    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpd, d_fp);
+    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpsd, d_sp2);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     return NEORX_OK;
@@ -2277,41 +2355,42 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     hipStream_t st = (hipStream_t)stream;
     i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne6));
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
-    DevBuf X, G, Y, part, partq, fpd;
-    int rc = G.alloc(nb * ne6 * 8);
-    if (!rc && !pairs) rc = X.alloc(nb * ne6 * 8);
-    if (!rc && !pairs) rc = Y.alloc(slab_cap(s, 3) * 8);
-    if (!rc) rc = part.alloc(npp * ne * (ne + 1) * 8);
-    if (!rc && pairs) rc = partq.alloc(s->plan.nq * ne * (ne + 1) * 8);
-    if (!rc) rc = fpd.alloc(npp * 8);
+    Work W(st);
+    double *X = nullptr, *Y = nullptr, *partq = nullptr, *G, *part;
+    int rc = W.get(G, nb * ne6);
+    if (!rc && !pairs) rc = W.get(X, nb * ne6);
+    if (!rc && !pairs) rc = W.get(Y, slab_cap(s, 3));
+    if (!rc && pairs) rc = W.get(partq, s->plan.nq * ne * (ne + 1));
+    if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp);
     if (rc) return rc;
+    double *fpd = part + npp * ne * (ne + 1);
     if (pairs) {
         for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
             const i64 q1 = std::min(s->plan.nq, q0 + nb);
-            rc = nrx_gam3_pairs(s, false, q0, q1, 0, G.d(), st);
+            rc = nrx_gam3_pairs(s, false, q0, q1, 0, G, W);
             if (rc) return rc;
             hipLaunchKernelGGL((k_eg3_slab<double, 16, 1>), dim3((unsigned)((q1 - q0) * ne)), dim3(eg3_threads(ne)),
-                               eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G.d(),
-                               partq.d() + q0 * ne * (ne + 1));
+                               eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G,
+                               partq + q0 * ne * (ne + 1));
             HIPCHK(hipGetLastError());
         }
         hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * (ne + 1), 256)), dim3(256), 0, st, np,
-                           ne * (ne + 1), partq.d(), part.d());
+                           ne * (ne + 1), partq, part);
         HIPCHK(hipGetLastError());
     }
     for (i64 p0 = 0; !pairs && p0 < npp; p0 += nb) {
         i64 p1 = std::min(npp, p0 + nb), n = (p1 - p0) * ne6;
-        rc = build3_block(s, p0, p1, X.d(), Y.d(), st);
+        rc = build3_block(s, p0, p1, X, Y, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(k_gam3_symm, dim3(grid_blocks(n, 256)), dim3(256), 0, st, ne, n, X.d(), G.d());
+        hipLaunchKernelGGL(k_gam3_symm, dim3(grid_blocks(n, 256)), dim3(256), 0, st, ne, n, X, G);
         hipLaunchKernelGGL((k_eg3_slab<double, 16, 1>), dim3((unsigned)((p1 - p0) * ne)), dim3(eg3_threads(ne)),
-                           eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G.d(), part.d() + p0 * ne * (ne + 1));
+                           eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G, part + p0 * ne * (ne + 1));
         HIPCHK(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + npp, 256)), dim3(256), 0, st, ne, np, d_dp, part.d(), d_fe,
-                       fpd.d());
-    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd.d(), nullptr, d_e, nullptr);
-    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpd.d(), d_fp);
+    hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + npp, 256)), dim3(256), 0, st, ne, np, d_dp, part, d_fe,
+                       fpd);
+    hipLaunchKernelGGL(k_energy, dim3(1), dim3(64), 0, st, np, d_dp, fpd, nullptr, d_e, nullptr);
+    hipLaunchKernelGGL(k_axpy, dim3(nblocks(npp, 256)), dim3(256), 0, st, npp, fpd, d_fp);
     HIPCHK(hipGetLastError());
     HIPCHK(hipStreamSynchronize(st));
     return NEORX_OK;
@@ -2861,7 +2940,8 @@ extern "C" int neorx_rxchfne_gam2_ic1_dev(int64_t handle, double *d_gm2, double 
     i64 ne = s->d.nebf, np = s->d.npbf, ng2 = ne * ne * ne * ne * np * np;
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
-        int r = nrx_gam2_pairs(s, true, 0, s->plan.nq, np, d_gm2, d_gm2ex, st);
+        Work W(st);
+        int r = nrx_gam2_pairs(s, true, 0, s->plan.nq, np, d_gm2, d_gm2ex, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }

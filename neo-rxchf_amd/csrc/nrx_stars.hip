@@ -770,16 +770,17 @@ int rec_ne(int deg) { return (deg <= 4 ? deg : deg <= 6 ? 6 : deg <= 8 ? 8 : 12)
 
 // V, X and T of the distinct nuclear pairs, then G (see Gam3Out).  mult: the
 // RXCHFmult form, without the one-geminal terms.
-int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G, hipStream_t st)
+int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G, Work &W)
 {
+    hipStream_t st = W.st;
     const DevSys &d = s->d;
     const PairPlan &P = s->plan;
     const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2;
     const int ng = (int)d.ngtg, nt = ng * ng;
-    StreamBuf w0, wT, wR;
-    int rc = w0.alloc((LONE_F * P.nslot + nc * nc + nc * (q1 - q0) + nc * P.npl) * 8, st);
+    double *lone, *T, *rec;
+    int rc = W.get(lone, LONE_F * P.nslot + nc * nc + nc * (q1 - q0) + nc * P.npl);
     if (rc) return rc;
-    double *lone = (double *)w0.p, *V = lone + LONE_F * P.nslot, *X = V + nc * nc, *Vp = X + nc * (q1 - q0);
+    double *V = lone + LONE_F * P.nslot, *X = V + nc * nc, *Vp = X + nc * (q1 - q0);
     hipLaunchKernelGGL(k_lone_prep, dim3((unsigned)(P.nslot / 64)), dim3(64), 0, st, d, P, lone);
     HIPCHK(hipGetLastError());
     StarJob X1{0, P.npl, q0, q1 - q0, 0, 0, P.gx, nullptr, P.wx};
@@ -806,10 +807,9 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
     const i64 nqt = std::max<i64>(1, std::min<i64>({q1 - q0, T_BYTES / (ntri * nc * 8), (i64)32768})); // nuclear pairs T holds
     const i64 nqr = std::max<i64>(1, std::min<i64>(nqt, REC_BYTES / big));               // and one launch takes
     const i64 vcap = P.npl * (REC_HEAD + 3 * NE1) * 8;
-    if ((rc = wT.alloc(nqt * ntri * nc * 8, st))) return rc;
-    if ((rc = wR.alloc(std::max(vcap, std::max(big * nqr, std::min(REC_BYTES, span(0, nc, nqr, nst, nu)))), st)))
-        return rc;
-    double *T = (double *)wT.p, *rec = (double *)wR.p;
+    if ((rc = W.get(T, nqt * ntri * nc))) return rc;
+    const i64 all = std::min(REC_BYTES, span(0, nc, nqr, nst, nu));
+    if ((rc = W.get(rec, (std::max({vcap, big * nqr, all}) + 7) / 8))) return rc;
     { // V: pair densities and lone pairs
         StarJob J{0, P.npl, 0, 1, 1, NE1, P.one + 1, P.one + 1, P.one};
         LoneJob L{0, nc, 0, 0, P.npl, 1, NE1, nc, 0.0};
@@ -854,18 +854,19 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
 
 // GAM_2 and its overlaps (rxne: the RXCHF-ne tensors) of the distinct nuclear
 // pairs [q0, q1)
-int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G, double *Gs, hipStream_t st)
+int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G, double *Gs, Work &W)
 {
+    hipStream_t st = W.st;
     const DevSys &d = s->d;
     const PairPlan &P = s->plan;
     const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2, nqa = q1 - q0;
     const int ng = (int)d.ngtg, nt = ng * ng, nx = ng * (ng + 1) / 2 + (rxne ? 0 : ng);
     const int NE2 = rec_ne(2 * P.le + 2 * P.lp), nterms = rxne ? 1 : BT_OVL;
     const i64 nrows = (i64)nt * (rxne ? 1 : BT_ROWS);
-    StreamBuf w0, wR;
-    int rc = w0.alloc((LONE_F * P.nslot + 3 * KT * (P.npl + P.nq) + nqa * (nc * nc + 2 * ntri)) * 8 + 64, st);
+    double *lone, *rec;
+    int rc = W.get(lone, LONE_F * P.nslot + 3 * KT * (P.npl + P.nq) + nqa * (nc * nc + 2 * ntri) + 8);
     if (rc) return rc;
-    double *lone = (double *)w0.p, *kt = lone + LONE_F * P.nslot, *L = kt + 3 * KT * (P.npl + P.nq),
+    double *kt = lone + LONE_F * P.nslot, *L = kt + 3 * KT * (P.npl + P.nq),
            *B = L + nqa * nc * nc, *Y = B + nqa * ntri;
     unsigned *counts = (unsigned *)(Y + nqa * ntri);
     hipLaunchKernelGGL(k_lone_prep, dim3((unsigned)(P.nslot / 64)), dim3(64), 0, st, d, P, lone);
@@ -886,8 +887,7 @@ int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G,
     const i64 all = span(0, nc, nst, nu);
     const i64 nqr = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / big));
     const i64 nql = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / lone_b));
-    if ((rc = wR.alloc(std::max({nql * lone_b, nqr * big, std::min(nqr * all, REC_BYTES)}), st))) return rc;
-    double *rec = (double *)wR.p;
+    if ((rc = W.get(rec, (std::max({nql * lone_b, nqr * big, std::min(nqr * all, REC_BYTES)}) + 7) / 8))) return rc;
     for (i64 q = q0; q < q1; q += nql) { // L
         const i64 nq = std::min(nql, q1 - q);
         StarJob J{0, P.npl, q, nq, nx, NE2, P.gx + (rxne ? ng : 0), P.gx, P.wx + (rxne ? ng : 0)};
