@@ -505,7 +505,7 @@ def main():
 # make nonzero (tests/count_flops.py); traffic = HBM bytes per launch of the
 # dominant kernel from rocprofv3 FETCH_SIZE + WRITE_SIZE (profiles/), scaled
 # by the copy-kernel calibration.
-FLOPS_PER_TUPLE = {1: 56733.7, 2: 113053.3, 3: 33681.3}
+FLOPS_PER_TUPLE = {1: 39040.9, 2: 105612.2, 3: 33681.3}
 TRAFFIC = {2: 366.37e6}  # e-e-p launch group (bin + scatter + tiers) at the default 1,048,576 sampled tuples
 
 if __name__ == "__main__":

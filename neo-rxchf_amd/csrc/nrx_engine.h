@@ -122,6 +122,8 @@ NRX_HD constexpr double dfact(int n) // (n)!! for odd n, 1 for n <= 0
     return r;
 }
 NRX_HD int imin(int a, int b) { return a < b ? a : b; }
+NRX_HD int imax(int a, int b) { return a > b ? a : b; }
+constexpr int cmin(int a, int b) { return a < b ? a : b; }
 
 // 1/x and 1/sqrt(x) for the engine's positive, well-scaled exponents (no
 // zeros, infinities or denormals): the hardware estimate refined by two
@@ -471,6 +473,14 @@ struct Sys {
     const double *bt; // Boys table
 };
 
+// particle i's pair and geminal, i not a constant (wave-uniform): selects
+// rather than an indexed array, which would live in memory
+NRX_HD const PairRec *qsel(const Sys &s, int i)
+{
+    return i == 0 ? s.q[0] : i == 1 ? s.q[1] : i == 2 ? s.q[2] : s.q[3];
+}
+NRX_HD double gsel(const Sys &s, int i) { return i == 0 ? s.gam[0] : i == 1 ? s.gam[1] : i == 2 ? s.gam[2] : 0.0; }
+
 NRX_HD double Kprod(const Sys &s)
 {
     double k = 1.0;
@@ -544,11 +554,11 @@ template <int NF, int NR> NRX_HD void hub_map(const Sys &s, int i, int d, const 
     p_copy(t, r);
 }
 
-template <int N> NRX_HD void p_add(const PolyT<N> &a, const PolyT<N> &b, PolyT<N> &r)
+template <int N> NRX_HD void p_add(const PolyT<N> &a, const PolyT<N> &b, PolyT<N> &r, double f = 1.0)
 {
-    NRX_UNROLL for (int k = 0; k < N; ++k) r.c[k] = a.c[k] + b.c[k];
+    NRX_UNROLL for (int k = 0; k < N; ++k) r.c[k] = a.c[k] + f * b.c[k];
     r.n = a.n > b.n ? a.n : b.n;
-    NRX_CNT(r.n);
+    NRX_CNT(2 * r.n);
 }
 
 // Kinetic energy of particle a (-1/(2m) <bra| d^2/dx_a^2 |ket>) for nv <= 2
@@ -764,17 +774,18 @@ template <int NL> NRX_HD double nuc_core(const Sys &s, int a, int d, PolyT<NL> &
     int core = h;
     VarT<NL> A;
     if (a != h) {
-        fpoly(*s.q[a], d, A.F);
-        A.w = s.q[a]->p;
+        const PairRec *qa = qsel(s, a);
+        fpoly(*qa, d, A.F);
+        A.w = qa->p;
         A.c = 0.0;
-        fac *= absorb_leaf(H.F, H.w, H.c, s.gam[a], s.q[h]->P[d] - s.q[a]->P[d], A, pic);
+        fac *= absorb_leaf(H.F, H.w, H.c, gsel(s, a), s.q[h]->P[d] - qa->P[d], A, pic);
         core = a;
     } else {
         A = H;
     }
     p_compose(A.F, A.c, 1.0, A.F);
     p_hermite(A.F, A.w, e);
-    X = s.q[core]->P[d] + A.c;
+    X = qsel(s, core)->P[d] + A.c;
     w = A.w;
     return fac;
 }
@@ -819,170 +830,198 @@ NRX_HD double nuc_sum(const Sys &s, int a, int nat, const double *cat, const dou
     return nuc_centres<NL, NBC>(e, X, w, fac * 2.0 * pic * rcp(w), nat, cat, zan, flush, s.bt);
 }
 
-// One kinetic operator of kin_pair: particle a, partner c (c < 0: none),
-// nv <= 2 variants with ket-geminal exponents gk[v], mass.
-struct KinOp {
-    int a, c, nv;
-    double gk[2], mass;
-};
+// ------------------------------------------------------------------
+// kinetic operators on a star, without derivatives of geminals
+// ------------------------------------------------------------------
+// u_o(y) times K(y), u = (y + so)^lo, K = the second derivative of X^L
+// exp(-beta X^2), X = y + sL, over exp(-beta X^2):
+// X^L (4 beta^2 X^2 - 2 beta (2L+1)) + L(L-1) X^(L-2)
+template <int N> NRX_HD void kin_poly(int L, double sL, double be, int lo, double so, PolyT<N> &r)
+{
+    p_const(r, 4.0 * be * be);
+    p_mul_lin(r, sL);
+    p_mul_lin(r, sL);
+    r.c[0] -= 2.0 * be * (2 * L + 1);
+    p_mul_lin(r, sL, L >= 1);
+    p_mul_lin(r, sL, L >= 2);
+    r.c[0] += L >= 2 ? (double)(L * (L - 1)) : 0.0;
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX - 2; ++i) p_mul_lin(r, sL, i < L - 2);
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, so, i < lo);
+}
+// u_o(y) times the first derivative, X^(L-1) (L - 2 beta X^2)
+template <int N> NRX_HD void der_poly(int L, double sL, double be, int lo, double so, PolyT<N> &r)
+{
+    p_const(r, -2.0 * be);
+    p_mul_lin(r, sL);
+    p_mul_lin(r, sL, L >= 1);
+    r.c[0] += (double)L;
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX - 1; ++i) p_mul_lin(r, sL, i < L - 1);
+    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, so, i < lo);
+}
+// wk (operator on the ket) + wb (operator on the bra) of -1/2 d^2/dx^2
+template <int N> NRX_HD void pair_kin_poly(const PairRec &q, int x, double wk, double wb, PolyT<N> &r)
+{
+    PolyT<N> b;
+    kin_poly(q.lb[x], q.sB[x], q.beta, q.la[x], q.sA[x], r);
+    kin_poly(q.la[x], q.sA[x], q.p - q.beta, q.lb[x], q.sB[x], b);
+    NRX_UNROLL for (int k = 0; k < N; ++k) r.c[k] = -0.5 * (wk * r.c[k] + wb * b.c[k]);
+    r.n = imin(q.la[x] + q.lb[x] + 3, N);
+}
+// i dj/dx - j di/dx (bra i, ket j) over the pair's Gaussian
+template <int N> NRX_HD void pair_wronskian(const PairRec &q, int x, PolyT<N> &r)
+{
+    PolyT<N> b;
+    der_poly(q.lb[x], q.sB[x], q.beta, q.la[x], q.sA[x], r);
+    der_poly(q.la[x], q.sA[x], q.p - q.beta, q.lb[x], q.sB[x], b);
+    NRX_UNROLL for (int k = 0; k < N; ++k) r.c[k] -= b.c[k];
+    r.n = imin(q.la[x] + q.lb[x] + 2, N);
+}
 
-// Two kinetic operators on one configuration (for instance the electron's
-// and the proton's of an e-p star): the Gaussian factors, the particles'
-// polynomials mapped to the hub coordinate and the overlap of each direction
-// are computed once and shared, as are the product-rule overlaps S_d.
-// out1[v], out2[v] as kin_multi's out; ovl_out (if set) the overlap.  With
-// NUC set, nuc_out = nuc_sum(s, hub, ...) at capacity NC: the hub's core
-// variable is the product polynomial of the overlap, on the same Gaussian.
-template <int NL, int NC = NL, int NBC = NB, bool NUC = false>
-NRX_HD void kin_pair(const Sys &s, const KinOp &o1, const KinOp &o2, double pic, double *out1, double *out2,
-                     double *ovl_out = nullptr, double *nuc_out = nullptr, int nat = 0, const double *cat = nullptr,
-                     const double *zan = nullptr, bool flush = false)
+// Gaussian data of a leaf in the hub coordinate of direction x: a polynomial
+// f of the leaf maps to smooth(f, iW/2)(m0 + beta y)
+struct LeafMap {
+    double iW, beta, m0, dl;
+};
+template <int NF, int NR> NRX_HD void to_hub(const PolyT<NF> &f, const LeafMap &m, PolyT<NR> &r)
+{
+    PolyT<NF> t;
+    p_smooth(f, 0.5 * m.iW, t);
+    p_compose(t, m.m0, m.beta, t);
+    p_copy(t, r);
+}
+// (x_hub - x_leaf) f: y m - dl m - M[y f], m = M[f]
+template <int NF, int NM, int NR>
+NRX_HD void rel_map(const PolyT<NF> &f, const PolyT<NM> &m, const LeafMap &g, PolyT<NR> &r)
+{
+    PolyT<NR> yf, ym;
+    NRX_UNROLL for (int k = 0; k < NR; ++k) yf.c[k] = (k && k - 1 < NF) ? f.c[k - 1] : 0.0;
+    yf.n = imin(f.n + 1, NR);
+    to_hub(yf, g, ym);
+    NRX_UNROLL for (int k = 0; k < NR; ++k)
+        r.c[k] = ((k && k - 1 < NM) ? m.c[k - 1] : 0.0) - (k < NM ? g.dl * m.c[k] : 0.0) - ym.c[k];
+    r.n = yf.n;
+    NRX_CNT(3 * r.n);
+}
+
+// Kinetic energy of a star of one or two electrons (particles 0 .. n-2) and
+// the hub, and its overlap, both normalised with pic:
+//   T = sum_i [ wk_i <ket operator of i> + wb_i <bra operator of i> ]
+//       + cross <(r_h - r_0) . (r_h - r_j)>       (j = 0 for n = 2, else 1)
+//       + <(c0 (r_h - r_0) + c1 (r_h - r_1)) . (i grad j - j grad i)_h>
+// with i, j the hub's bra and ket.  A kinetic operator between geminals
+// needs no derivative of one that shares the particle: for an electron
+// <i| g T g' |j> with both geminals on one side is the operator on the other
+// function; for the hub (mass m)
+//   g_a T g_b = (T g_a g_b + g_a g_b T)/2 + (1/2m) grad g_a . grad g_b
+//               + (1/2m) [gamma_b (r_h - r_b) - gamma_a (r_h - r_a)] . (i grad j - j grad i) g_a g_b / (i j),
+// and g_k T g_l + g_l T g_k on one link has no antisymmetric part.  Against the
+// second derivative of the ket with its geminal (kin_multi's form, six
+// polynomial products per direction, operator and variant) this takes five per
+// direction in all: 2^20 e-e-p tuples of the 60/16 system 10.78 -> 10.21 ms,
+// 230,401 e-p tuples 1.02 -> 0.77 ms.
+struct StarKin {
+    double wk[3], wb[3], cross, c0, c1;
+};
+// NL holds the star's degree + 2.
+template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double pic, double &ovl_out)
 {
     NRX_FENCE();
-    // the kinetic polynomials (degree <= tuple degree < NL) at capacity min(NK, NL)
-    constexpr int FK = NK < NL ? NK : NL;
+    double Pr = 1.0, R = 0.0;
     const int h = s.n - 1;
-    double Pr = 1.0, R[2][2] = {{0.0, 0.0}, {0.0, 0.0}};
-    PolyT<NC> ne[3]; // the hub's Hermite coefficients per direction (NUC)
-    double nX[3] = {0.0, 0.0, 0.0}, nfac = 1.0, nw = 1.0;
-    NRX_DIRS for (int d = 0; d < 3; ++d) {
+    constexpr int N = NL;
+    NRX_DIRS for (int x = 0; x < 3; ++x) {
+        constexpr int FS = cmin(NS, N), FT = cmin(NS + 2, N), FR = cmin(NS + 1, N);
         double w = s.q[h]->p, cq = 0.0, fac = 1.0;
-        NRX_UNROLL for (int i = 0; i < NPART - 1; ++i) {
+        LeafMap g[2];
+        NRX_UNROLL for (int i = 0; i < 2; ++i) {
             if (i >= h) continue;
             const PairRec &Q = *s.q[i];
-            double g = s.gam[i], rW = rsqrt(Q.p + g), iW = rW * rW, fl = sqrt(pic) * rW;
-            if (g != 0.0) {
-                double kap = Q.p * (g * iW), cl = Q.P[d] - s.q[h]->P[d], Wq = w + kap, iWq = rcp(Wq);
-                double diff = cq - cl;
-                fl *= exp(-(w * kap * iWq) * diff * diff);
-                cq = (w * cq + kap * cl) * iWq;
-                w = Wq;
-            }
-            fac *= fl;
+            const double gi = s.gam[i], rW = rsqrt(Q.p + gi);
+            g[i].iW = rW * rW;
+            g[i].beta = gi * g[i].iW;
+            g[i].dl = Q.P[x] - s.q[h]->P[x];
+            g[i].m0 = -g[i].beta * g[i].dl;
+            const double kap = Q.p * g[i].beta, Wq = w + kap, iWq = rcp(Wq), df = cq - g[i].dl;
+            fac *= sqrt(pic) * rW * exp(-(w * kap * iWq) * df * df);
+            cq = (w * cq + kap * g[i].dl) * iWq;
+            w = Wq;
         }
         const double rw = rsqrt(w), iw = rw * rw, norm = fac * (sqrt(pic) * rw);
-        // every particle's own polynomial in the hub coordinate
-        PolyT<NL> m[NPART];
-        NRX_UNROLL for (int i = 0; i < NPART; ++i) {
-            if (i > h) {
-                p_const(m[i], 1.0);
-                continue;
+        PolyT<FS> f, m0;
+        PolyT<FT> t, k;
+        PolyT<FR> r0;
+        PolyT<N> q, env, u;
+        fpoly(*s.q[0], x, f);
+        to_hub(f, g[0], m0);
+        rel_map(f, m0, g[0], r0);
+        pair_kin_poly(*s.q[0], x, o.wk[0], o.wb[0], k);
+        to_hub(k, g[0], t);
+        if (h == 1) {
+            // (r_h - r_0)^2: (y - dl) r0 - M[y (r0's polynomial)], with
+            // M[y^2 f] from the square of the leaf coordinate
+            PolyT<FT> y2, m2;
+            NRX_UNROLL for (int i = 0; i < FT; ++i) y2.c[i] = (i > 1 && i - 2 < FS) ? f.c[i - 2] : 0.0;
+            y2.n = imin(f.n + 2, FT);
+            to_hub(y2, g[0], m2);
+            PolyT<FR> yf, m1;
+            NRX_UNROLL for (int i = 0; i < FR; ++i) yf.c[i] = (i && i - 1 < FS) ? f.c[i - 1] : 0.0;
+            yf.n = imin(f.n + 1, FR);
+            to_hub(yf, g[0], m1);
+            // (y-dl)^2 m0 - 2 (y-dl) m1 + m2
+            NRX_UNROLL for (int i = 0; i < FT; ++i) {
+                const double a0 = i < FS ? m0.c[i] : 0.0, a1 = (i && i - 1 < FS) ? m0.c[i - 1] : 0.0,
+                             a2 = (i > 1 && i - 2 < FS) ? m0.c[i - 2] : 0.0;
+                const double b0 = i < FR ? m1.c[i] : 0.0, b1 = (i && i - 1 < FR) ? m1.c[i - 1] : 0.0;
+                m2.c[i] += (a2 - 2.0 * g[0].dl * a1 + g[0].dl * g[0].dl * a0) - 2.0 * (b1 - g[0].dl * b0);
+                t.c[i] += o.cross * m2.c[i];
             }
-            PolyT<NS> f;
-            fpoly(*s.q[i], d, f);
-            hub_map(s, i, d, f, m[i]);
-        }
-        PolyT<NL> q;
-        p_const(q, 1.0);
-        NRX_UNROLL for (int i = 0; i < NPART; ++i)
-            if (i <= h) p_mul(q, m[i], q);
-        const double Sd = norm * close_expect(q, iw, cq);
-        if constexpr (NUC) {
-            PolyT<NC> qc, ed;
-            p_copy(q, qc);
-            p_compose(qc, cq, 1.0, qc);
-            p_hermite(qc, w, ed);
-            // the direction loop stays rolled: store by uniform branches
-            if (d == 0)
-                ne[0] = ed;
-            else if (d == 1)
-                ne[1] = ed;
-            else
-                ne[2] = ed;
-            double x = s.q[h]->P[d] + cq;
-            nX[0] = (d == 0) ? x : nX[0];
-            nX[1] = (d == 1) ? x : nX[1];
-            nX[2] = (d == 2) ? x : nX[2];
-            nfac *= fac;
-            nw = w;
-        }
-        NRX_UNROLL for (int k = 0; k < 2; ++k) {
-            const KinOp &o = (k == 0) ? o1 : o2;
-            const int a = o.a, c = o.c;
-            const PairRec &A = *s.q[a];
-            PolyT<NL> env, base;
-            p_const(env, 1.0);
-            NRX_UNROLL for (int i = 0; i < NPART; ++i)
-                if (i <= h && i != a && i != c) p_mul(env, m[i], env);
-            if (c >= 0)
-                p_mul(env, m[c], base);
-            else
-                base = env;
-            int L = A.lb[d];
-            double sA = A.sA[d], sB = A.sB[d];
-            int la = A.la[d];
-            NRX_UNROLL for (int v = 0; v < 2; ++v) {
-                if (v >= o.nv) continue;
-                double g = (c >= 0) ? o.gk[v] : 0.0;
-                double al = A.beta + g;
-                double dl = (g != 0.0) ? g * (A.B[d] - s.q[c]->B[d]) : 0.0;
-                // the F0, F1, F2 of kin_multi
-                double cf0[5] = {(double)(L * (L - 1)), -4.0 * L * dl, -4.0 * L * al + 4.0 * dl * dl - 2.0 * al,
-                                 8.0 * al * dl, 4.0 * al * al};
-                double cf1[5] = {0.0, 4.0 * L * g, -8.0 * dl * g, -8.0 * al * g, 0.0};
-                int j0 = (L >= 2) ? 0 : 2 - L;
-                PolyT<FK> F0, F1;
-                p_const(F0, cf0[4]);
-                p_const(F1, cf1[4]);
-                NRX_UNROLL for (int j = 3; j >= 0; --j) {
-                    bool on = j >= j0;
-                    p_mul_lin(F0, sB, on);
-                    p_mul_lin(F1, sB, on);
-                    F0.c[0] += on ? cf0[j] : 0.0;
-                    F1.c[0] += on ? cf1[j] : 0.0;
-                }
-                NRX_UNROLL for (int i = 0; i < KIN_LM2; ++i) {
-                    p_mul_lin(F0, sB, i < L - 2);
-                    p_mul_lin(F1, sB, i < L - 2);
-                }
-                NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) {
-                    p_mul_lin(F0, sA, i < la);
-                    p_mul_lin(F1, sA, i < la);
-                }
-                PolyT<NL> m0;
-                hub_map(s, a, d, F0, m0);
-                p_mul(base, m0, q);
-                if (g != 0.0) {
-                    PolyT<FK> F2;
-                    p_const(F2, 4.0 * g * g);
-                    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(F2, sB, i < L);
-                    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(F2, sA, i < la);
-                    PolyT<FK> fc;
-                    fpoly(*s.q[c], d, fc);
-                    double xc = s.q[c]->sB[d];
-                    PolyT<NL> m1, m2, c1, c2, u;
-                    p_mul_lin(fc, xc);
-                    hub_map(s, c, d, fc, c1);
-                    p_mul_lin(fc, xc);
-                    hub_map(s, c, d, fc, c2);
-                    hub_map(s, a, d, F1, m1);
-                    hub_map(s, a, d, F2, m2);
-                    p_mul(m1, c1, u);
-                    p_mul(m2, c2, m2);
-                    p_add(u, m2, u);
-                    p_mul(env, u, u);
-                    p_add(q, u, q);
-                }
-                double t = norm * close_expect(q, iw, cq);
-                R[k][v] = R[k][v] * Sd + Pr * t;
+            t.n = FT;
+            NRX_CNT(14 * f.n);
+            p_copy(t, u);
+            p_copy(m0, env);
+        } else {
+            PolyT<FS> m1;
+            PolyT<FR> r1;
+            fpoly(*s.q[1], x, f);
+            to_hub(f, g[1], m1);
+            rel_map(f, m1, g[1], r1);
+            p_mul(t, m1, u);
+            pair_kin_poly(*s.q[1], x, o.wk[1], o.wb[1], k);
+            to_hub(k, g[1], t);
+            p_mul(m0, t, q);
+            p_add(u, q, u);
+            p_mul(r0, r1, q);
+            p_add(u, q, u, o.cross);
+            p_mul(m0, m1, env);
+            if (o.c0 != 0.0 || o.c1 != 0.0) {
+                PolyT<FR> wr;
+                PolyT<N> v;
+                pair_wronskian(*s.q[2], x, wr);
+                p_mul(r0, m1, q);
+                p_mul(m0, r1, v);
+                NRX_UNROLL for (int i = 0; i < N; ++i) v.c[i] = o.c0 * q.c[i] + o.c1 * v.c[i];
+                v.n = imin(imax(q.n, v.n), N);
+                p_mul(v, wr, q);
+            } else {
+                p_const(q, 0.0);
             }
         }
-        Pr *= Sd;
+        // hub polynomials: u f_h + env t_h (+ q)
+        fpoly(*s.q[h], x, f);
+        p_mul(u, f, u);
+        if (h == 2) p_add(u, q, u);
+        pair_kin_poly(*s.q[h], x, o.wk[h], o.wb[h], k);
+        p_mul(env, k, q);
+        p_add(u, q, u);
+        const double T = norm * close_expect(u, iw, cq);
+        p_mul(env, f, q);
+        const double S = norm * close_expect(q, iw, cq);
+        R = R * S + Pr * T;
+        Pr *= S;
     }
-    double kp = Kprod(s);
-    NRX_UNROLL for (int v = 0; v < 2; ++v) {
-        if (v < o1.nv) out1[v] = -0.5 * R[0][v] / o1.mass * kp;
-        if (v < o2.nv) out2[v] = -0.5 * R[1][v] / o2.mass * kp;
-    }
-    if (ovl_out) *ovl_out = kp * Pr;
-    if constexpr (NUC) {
-        // the Gaussian factors carry pic^(1/2) per leaf and direction; the
-        // nuclear attraction is normalised with PI
-        double r = PI / pic, sc = 1.0;
-        NRX_UNROLL for (int i = 0; i < NPART - 1; ++i)
-            if (i < h) sc *= r * sqrt(r);
-        *nuc_out = nuc_centres<NC, NBC>(ne, nX, nw, kp * nfac * sc * 2.0 * PI * rcp(nw), nat, cat, zan, flush, s.bt);
-    }
+    const double kp = Kprod(s);
+    ovl_out = kp * Pr;
+    return kp * R;
 }
 
 // hk[t+u] += ea[t] eb[u] (-1)^u
@@ -1185,54 +1224,36 @@ NRX_HD int tuple_degree(const PairRec *const *q, int n, bool kinetic)
 // Terms that depend on gamma_k + gamma_l only are summed over k <= l.
 // With MULT set: RXCHFmult_xcalc_GAM1_MD (rxchfmult/rxchfmult_gam1.f:399-840),
 // the same value without the one-geminal terms.
+// The two kinetic forms of a one-geminal term, and of (k,l) with (l,k), sum to
+// the mean of the operator on bra and ket (twice) plus, for two geminals,
+// grad g_k . grad g_l (1 + 1/m): one star_kin per configuration.
 template <int NL, int NBC, bool MULT = false>
 NRX_HD void gam1_tuple(const SysParams &S, const PairRec *e, const PairRec *p, double &ansE, double &ansS)
 {
     constexpr int NC = NL - 2; // capacity of the terms without a kinetic operator
-    double tegx = 0, tpgx = 0, texg = 0, tpxg = 0, tegg = 0, tpgg = 0;
-    double vcegx = 0, vcegg = 0, vcpgx = 0, vcpgg = 0, vmgx = 0, vmgg = 0;
-    double ogx = 0, ogg = 0;
+    const double im = 1.0 / S.pmass;
+    double te = 0.0, v = 0.0, ansSs = 0.0;
+    auto config = [&](double g, double cross, double w) {
+        Sys s = mksys(S, 2, e, p, 0, 0, g, 0, 0); // (e, p): hub = p
+        double ov;
+        te += w * star_kin<NL>(s, StarKin{{0.5, 0.5 * im, 0.0}, {0.5, 0.5 * im, 0.0}, cross, 0.0, 0.0}, PI_G2, ov);
+        // one copy of the code for both particles
+        NRX_DIRS for (int i = 0; i < 2; ++i)
+            v += (i ? w : -w) * nuc_sum<NC, NBC>(s, i, S.nat, S.cat, S.zan, false);
+        v -= w * coul<NC, NBC>(s, 0, 1);
+        ansSs += w * (ov * G2_TO_PI3);
+    };
     for (int k = 0; k < S.ngtg; ++k) {
-        double gv = S.gamma[k], bv = S.bcoef[k];
-        if constexpr (!MULT) {
-            Sys s1 = mksys(S, 2, e, p, 0, 0, gv, 0, 0);  // (e, p): hub = p
-            // the electron's and the proton's kinetic operators on the same
-            // two-particle star: one pass serves both
-            double ke[2], kp[2], ov, vp;
-            kin_pair<NL, NC, NBC, true>(s1, KinOp{0, 1, 2, {0.0, gv}, 1.0}, KinOp{1, 0, 2, {0.0, gv}, S.pmass}, PI_G2,
-                                        ke, kp, &ov, &vp, S.nat, S.cat, S.zan, false);
-            tegx += bv * ke[0];
-            texg += bv * ke[1];
-            tpgx += bv * kp[0];
-            tpxg += bv * kp[1];
-            vcegx += bv * nuc_sum<NC, NBC>(s1, 0, S.nat, S.cat, S.zan, false);
-            vcpgx += bv * vp;
-            vmgx += bv * coul<NC, NBC>(s1, 0, 1);
-            ogx += bv * (ov * G2_TO_PI3);
-        }
-        // (k,l) and (l,k) share the configuration gamma_k + gamma_l; their
-        // kinetic terms differ only in the ket-geminal exponent (gamma_l,
-        // gamma_k), two variants of one kinetic call
-        for (int l = k; l < S.ngtg; ++l) {
-            double gw = S.gamma[l], bb = bv * S.bcoef[l];
-            Sys s2 = mksys(S, 2, e, p, 0, 0, gv + gw, 0, 0);
-            int nv = (l == k) ? 1 : 2;
-            double ke[2], kp[2], ov, vp;
-            kin_pair<NL, NC, NBC, true>(s2, KinOp{0, 1, nv, {gw, gv}, 1.0}, KinOp{1, 0, nv, {gw, gv}, S.pmass}, PI_G2,
-                                        ke, kp, &ov, &vp, S.nat, S.cat, S.zan, false);
-            tegg += (l == k) ? bb * ke[0] : bb * ke[0] + bb * ke[1];
-            tpgg += (l == k) ? bb * kp[0] : bb * kp[0] + bb * kp[1];
-            double w = (l == k) ? bb : 2.0 * bb;
-            vcegg += w * nuc_sum<NC, NBC>(s2, 0, S.nat, S.cat, S.zan, false);
-            vcpgg += w * vp;
-            vmgg += w * coul<NC, NBC>(s2, 0, 1);
-            ogg += w * (ov * G2_TO_PI3);
+        const double gk = S.gamma[k], bk = S.bcoef[k];
+        for (int l = MULT ? k : k - 1; l < S.ngtg; ++l) {
+            const bool one = l < k; // the one-geminal term of k
+            const double gl = one ? 0.0 : S.gamma[l];
+            const double w = one ? 2.0 * bk : (l == k ? 1.0 : 2.0) * (bk * S.bcoef[l]);
+            config(gk + gl, 2.0 * gk * gl * (1.0 + im), w);
         }
     }
-    double te = tegx + texg + tegg, tp = tpgx + tpxg + tpgg;
-    double vce = 2.0 * vcegx + vcegg, vcp = 2.0 * vcpgx + vcpgg, vmx = 2.0 * vmgx + vmgg;
-    ansE = te + tp - vce + vcp - vmx;
-    ansS = 2.0 * ogx + ogg;
+    ansE = te + v;
+    ansS = ansSs;
 }
 
 // xcalc_GAM2_MD (gam_2_OMP.f:546-1077).  With MULT set: RXCHFmult_GAM2_MD
@@ -1275,24 +1296,26 @@ NRX_HD void gam2_core(const SysParams &S, const PairRec *e1, const PairRec *e2, 
         gVEP += bk * xgVEP;
         gVEE += bk * xgVEE;
     }
-    double gTPg = 0, gTEg1 = 0, gTEg2 = 0, gTEg3 = 0, gVPCg = 0, gVECg1 = 0, gVECg2 = 0;
+    double gTg = 0, gTEg3 = 0, gVPCg = 0, gVECg1 = 0, gVECg2 = 0;
     double gVEPg1 = 0, gVEPg2 = 0, gVEEg1 = 0, gVEEg2 = 0, gsg = 0;
+    const double im = 1.0 / S.pmass;
     for (int ik = 0; ik < S.ngtg; ++ik)
         for (int il = 0; il < S.ngtg; ++il) {
             double gk = S.gamma[ik], gl = S.gamma[il];
             double bb = S.bcoef[ik] * S.bcoef[il];
-            // sb: g(e1,p)=gk, g(e2,p)=gl.  The reference's xgTEg2 of the pair
-            // (il,ik) (bra g(e2,p)=gl, ket g(e1,p)=gk) is the kinetic operator
-            // on this configuration with ket partner exponent gk.
+            // sb: g(e1,p)=gk, g(e2,p)=gl.  One star_kin gives gTPg (bra
+            // g(e1,p), ket g(e2,p)) and gTEg1 + gTEg2, the kinetic operator of
+            // e1 on its ket and, for the ket geminal of gTEg2, on its bra.
             Sys sb = mksys(S, 3, e1, e2, p, 0, gk, gl, 0);
-            double kk[2], kq[2], ov, vp;
-            kin_pair<NL, NC, NBC, true>(sb, KinOp{0, 2, 2, {0.0, gk}, 1.0}, KinOp{2, 1, 1, {gl, gl}, S.pmass}, PI, kk,
-                                        kq, &ov, &vp, S.nat, S.cat, S.zan, true);
-            gTEg1 += bb * kk[0];
-            gTEg2 += bb * kk[1];
-            gTPg += bb * kq[0];
-            gVPCg += bb * vp;
-            gVECg1 -= bb * nuc_sum<NC, NBC>(sb, 0, S.nat, S.cat, S.zan, true);
+            double ov;
+            gTg += bb * star_kin<NL>(sb, StarKin{{1.0, 0.0, 0.5 * im}, {1.0, 0.0, 0.5 * im}, 2.0 * gk * gl * im,
+                                                 -0.5 * gk * im, 0.5 * gl * im}, PI, ov);
+            // one copy of the code for the proton's attraction and e1's
+            NRX_DIRS for (int i = 0; i < 2; ++i) {
+                const double x = bb * nuc_sum<NC, NBC>(sb, 2 * i, S.nat, S.cat, S.zan, true);
+                gVPCg += i ? x : 0.0;
+                gVECg1 -= i ? 0.0 : x;
+            }
             double v = coul<NC, NBC>(sb, 0, 2);
             underflow(v);
             gVEPg1 -= bb * v;
@@ -1314,8 +1337,8 @@ NRX_HD void gam2_core(const SysParams &S, const PairRec *e1, const PairRec *e2, 
             underflow(v);
             gVEEg1 += w * v;
         }
-    ansE = 2.0 * (gTE + gVEC + gVEP) + 4.0 * gVEE * 0.5 + gTPg + gVPCg + gTEg1 + gTEg3 + 2.0 * (gVEPg1 + gVECg1) +
-           gTEg2 + gVEPg2 + gVECg2 + 2.0 * gVEEg1 * 0.5 + 2.0 * gVEEg2 * 0.5;
+    ansE = 2.0 * (gTE + gVEC + gVEP) + 4.0 * gVEE * 0.5 + gTg + gVPCg + gTEg3 + 2.0 * (gVEPg1 + gVECg1) +
+           gVEPg2 + gVECg2 + 2.0 * gVEEg1 * 0.5 + 2.0 * gVEEg2 * 0.5;
     ansS = gsg;
     ansE2 = gVEPg2 + gVEEg1;
     ansE3 = gVEEg2;
@@ -1448,24 +1471,22 @@ NRX_HD void rxchf2_tuple(const SysParams &S, const PairRec *e1, const PairRec *e
         Sys s1p = mksys(S, 2, e1, p, 0, 0, g, 0, 0);
         return ovl<NC>(s1p);
     };
-    double gTPg = 0, gTEg1 = 0, gTEg2 = 0, gTEg3 = 0, gVPCg = 0, gVECg1 = 0, gVECg2 = 0, gVECg3 = 0;
+    double gTg = 0, gTEg3 = 0, gVPCg = 0, gVECg1 = 0, gVECg2 = 0, gVECg3 = 0;
     double gVEPg1 = 0, gVEPg2 = 0, gVEPg3 = 0, gVEEg1 = 0, gVEEg2 = 0, gsg = 0;
+    const double im = 1.0 / S.pmass;
     for (int ik = 0; ik < S.ngtg; ++ik)
         for (int il = 0; il < S.ngtg; ++il) {
             const double gk = S.gamma[ik], gl = S.gamma[il];
             const double bb = S.bcoef[ik] * S.bcoef[il];
             Sys sb = mksys(S, 3, e1, e2, p, 0, gk, gl, 0);
-            // e1's kinetic energy (no ket geminal on e1) and the proton's (ket
-            // geminal gl to e2) share the configuration's pass, with the
-            // proton's nuclear attraction and the overlap
-            double kk[2], kq[2], ov, vp;
-            kin_pair<NL, NC, NBC, true>(sb, KinOp{0, 2, 1, {0.0, 0.0}, 1.0}, KinOp{2, 1, 1, {gl, gl}, S.pmass}, PI, kk,
-                                        kq, &ov, &vp, S.nat, S.cat, S.zan, true);
-            gTEg1 += bb * kk[0];
-            gTPg += bb * kq[0];
-            gVPCg += bb * vp;
+            // e1's kinetic energy (both geminals on the bra side: on its ket),
+            // e2's (ket geminal gl: on its bra) and the proton's (ket geminal
+            // gl to e2)
+            double ov;
+            gTg += bb * star_kin<NL>(sb, StarKin{{1.0, 0.0, 0.5 * im}, {0.0, 1.0, 0.5 * im}, 2.0 * gk * gl * im,
+                                                 -0.5 * gk * im, 0.5 * gl * im}, PI, ov);
+            gVPCg += bb * nuc_sum<NC, NBC>(sb, 2, S.nat, S.cat, S.zan, true);
             gsg += bb * ov;
-            gTEg2 += bb * kin<NL>(sb, 1, 2, gl, 1.0); // e2, ket geminal gl to p
             gVECg1 -= bb * nuc_sum<NC, NBC>(sb, 0, S.nat, S.cat, S.zan, true);
             gVECg2 -= bb * nuc_sum<NC, NBC>(sb, 1, S.nat, S.cat, S.zan, true);
             double v = coul<NC, NBC>(sb, 0, 2);
@@ -1491,7 +1512,7 @@ NRX_HD void rxchf2_tuple(const SysParams &S, const PairRec *e1, const PairRec *e
             gVEEg1 += w * v;
         }
     ansE1 = gTEg3 + gVECg3 + gVEPg3 + gVEEg1;
-    ansE2 = gTPg + gVPCg + gTEg1 + gVECg1 + gTEg2 + gVECg2 + gVEPg1 + gVEPg2 + gVEEg2;
+    ansE2 = gTg + gVPCg + gVECg1 + gVECg2 + gVEPg1 + gVEPg2 + gVEEg2;
     ansS = gsg;
 }
 
