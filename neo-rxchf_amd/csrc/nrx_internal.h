@@ -86,6 +86,14 @@ struct System {
 NRX_HIDDEN System *get_sys(i64 h);
 
 // ------------------------------------------------------------------
+// primitive tuples (nrx_prims.hip)
+// ------------------------------------------------------------------
+// values of tuples start .. start + ntup - 1 of class cls 1..10 from source src
+// (nrx_tuples.h), up to four outputs (os, ox, oy may be null)
+NRX_HIDDEN int nrx_prims(int cls, int src, const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os,
+                         double *ox, double *oy, hipStream_t st);
+
+// ------------------------------------------------------------------
 // the l <= 3 build of the engine (nrx_wide.hip)
 // ------------------------------------------------------------------
 // Tuples beyond the l <= 2 capacities (an f function on some particle) are
@@ -188,12 +196,14 @@ NRX_HIDDEN int nrx_gam1_launch(System *s, double *d_g1, double *d_g1s, hipStream
 // row before the DP(ip,jp) weight, part[blk][ne] = its DE-weighted sum / 3;
 // g of storage type dtype
 NRX_HIDDEN int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype, double *part,
-                             hipStream_t st);
+                             double *split, hipStream_t st);
+// doubles of the split scratch of such a launch (0: not used)
+NRX_HIDDEN i64 nrx_eg3_split_doubles(i64 ne, i64 nblk);
 // the same rows as the symmetric bilinear form T(X, Y) of two densities (X on
 // the (i2,j2) pair, Y on the (i3,j3) pair; T(DE, DE) are EG3IC1's rows), and
 // part[blk][ne] = sum_x Z(i1,x) F[x] / 3, or 0 when d_z is null
 NRX_HIDDEN int nrx_eg3_slabs2(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g,
-                              int dtype, double *part, hipStream_t st);
+                              int dtype, double *part, double *split, hipStream_t st);
 // EG2IC1 slab partials of nblk slabs (ip,jp,i1): part[blk][4][ne] = dir, ex,
 // dirS, exS (gs may be NULL: the S rows stay zero)
 NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double *g, const double *gs, double *part,

@@ -443,221 +443,12 @@ extern "C" int neorx_system_order(int64_t handle, int64_t *eorder, int64_t *pord
     return NEORX_OK;
 }
 
-// Tuples of a launch are sorted by bin, a counting sort in two passes:
-// k_prim_bin gives each tuple its bin (capacity tier tuple_tier, and for the
-// classes whose Coulomb terms take the hub-cycle path also the proton pair's
-// largest per-direction degree, which bounds that path's series) and counts
-// the bins, one atomic per wave and bin; k_prim_scatter writes the tuple
-// positions bin by bin into one list; k_prim_tiers evaluates every bin with
-// its tier's capacities, one lane per listed tuple, so that every wave runs
-// at the capacity its tuples need.  Both passes count in LDS per block and
-// touch each global counter once per block.  Out-of-range list entries are
-// flagged (NaN results) and left out.
-template <int CLS> constexpr int hub_bins() { return (CLS == 2 || CLS == 4 || CLS == 5 || CLS == 9) ? 5 : 1; }
-template <int CLS> constexpr int n_bins() { return Tier<CLS>::N * hub_bins<CLS>(); }
-
-template <int CLS> NRX_DI int tuple_bin(const PairRec *const *q)
-{
-    int k = tuple_tier<CLS>(q);
-    if (k == Tier<CLS>::N) return n_bins<CLS>(); // the wide bin (l <= 3 build)
-    if constexpr (hub_bins<CLS>() == 1) {
-        return k;
-    } else {
-        const PairRec &P = *q[nel<CLS>()];
-        int m = 0;
-        NRX_UNROLL for (int d = 0; d < 3; ++d) m = max(m, P.la[d] + P.lb[d]);
-        return k * hub_bins<CLS>() + min(m, hub_bins<CLS>() - 1);
-    }
-}
-
-template <int CLS, int SRC>
-__global__ void __launch_bounds__(256) k_prim_bin(DevSys S, i64 start, i64 ntup, const i64 *__restrict__ idx,
-                                                  double *__restrict__ outE, double *__restrict__ outS,
-                                                  double *__restrict__ outX, double *__restrict__ outY,
-                                                  unsigned char *__restrict__ code, unsigned *__restrict__ counts)
-{
-    __shared__ unsigned lc[32];
-    if (threadIdx.x < 32) lc[threadIdx.x] = 0u;
-    __syncthreads();
-    i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-    int bin = -1;
-    if (t < ntup) {
-        i64 x[2 * nel<CLS>() + 2];
-        bool ok = true;
-        if constexpr (SRC == SRC_LIST)
-            ok = load_tuple<CLS>(S, idx, t, x);
-        else
-            range_tuple<CLS, SRC == SRC_SORTED>(S, start + t, x);
-        if (ok) {
-            const PairRec *q[nel<CLS>() + 1];
-            tuple_pairs<CLS>(S, x, q);
-            bin = tuple_bin<CLS>(q);
-        } else { // out-of-range primitive index: flag the entry
-            outE[t] = __builtin_nan("");
-            if (outS) outS[t] = __builtin_nan("");
-            if (outX) outX[t] = __builtin_nan("");
-            if (outY) outY[t] = __builtin_nan("");
-        }
-        code[t] = (unsigned char)(bin < 0 ? 255 : bin);
-    }
-    if (bin >= 0) atomicAdd(&lc[bin], 1u);
-    __syncthreads();
-    if (threadIdx.x < n_bins<CLS>() + 1 && lc[threadIdx.x]) atomicAdd(&counts[threadIdx.x], lc[threadIdx.x]);
-}
-
-template <int CLS>
-__global__ void __launch_bounds__(256) k_prim_scatter(i64 ntup, const unsigned char *__restrict__ code,
-                                                      const unsigned *__restrict__ counts,
-                                                      unsigned *__restrict__ cursors, unsigned *__restrict__ list)
-{
-    __shared__ unsigned lc[32], lbase[32];
-    if (threadIdx.x < 32) lc[threadIdx.x] = 0u;
-    __syncthreads();
-    i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-    int bin = -1;
-    if (t < ntup) {
-        int c = code[t];
-        bin = (c == 255) ? -1 : c;
-    }
-    unsigned loc = 0;
-    if (bin >= 0) loc = atomicAdd(&lc[bin], 1u); // rank within the block's share of the bin
-    __syncthreads();
-    if (threadIdx.x < n_bins<CLS>() + 1)
-        lbase[threadIdx.x] = bin_offset(counts, threadIdx.x) +
-                             (lc[threadIdx.x] ? atomicAdd(&cursors[threadIdx.x], lc[threadIdx.x]) : 0u);
-    __syncthreads();
-    if (bin >= 0) list[lbase[bin] + loc] = (unsigned)t;
-}
-
-// Lanes per block of the tier kernel: one wavefront, so that blocks are
-// scheduled per SIMD (the kernels run at one wave per SIMD), measured ~1 %
-// faster than 256-lane blocks.
-constexpr int TIER_BS = 64;
-
-// One listed tuple of tier K: its pair records are staged in LDS (the
-// evaluation reads them many times; at one wave per SIMD, the register use
-// of these kernels, the LDS footprint costs no occupancy), then it is
-// evaluated with the tier's capacities.
-template <int CLS, int SRC, int K>
-NRX_DI void tier_item(const DevSys &S, i64 start, const i64 *__restrict__ idx, double *__restrict__ outE,
-                      double *__restrict__ outS, double *__restrict__ outX, double *__restrict__ outY, i64 t,
-                      PairRec (*stage)[TIER_BS])
-{
-    constexpr int NP = nel<CLS>() + 1;
-    i64 x[2 * NP];
-    src_tuple<CLS, SRC>(S, idx, start, t, x); // a list was validated by k_prim_bin
-    const PairRec *q[NP];
-    tuple_pairs<CLS>(S, x, q);
-    NRX_UNROLL for (int i = 0; i < NP; ++i) {
-        stage[i][threadIdx.x] = *q[i];
-        q[i] = &stage[i][threadIdx.x];
-    }
-    double e, s, xx, yy;
-    tuple_eval<CLS, Tier<CLS>::NL[K], Tier<CLS>::NB[K]>(d_params(S), q, e, s, xx, yy);
-    outE[t] = e;
-    if (outS) outS[t] = s;
-    if (outX) outX[t] = xx;
-    if (outY) outY[t] = yy;
-}
-
-// block b of the fused launch: the bins are laid out from the last tier and
-// the highest proton degree down (their tuples take longest, so they start
-// first).  Locates the block's bin; -1 past the last bin.
-template <int CLS> NRX_DI int block_bin(const unsigned *__restrict__ counts, i64 b, i64 &k0)
-{
-    for (int bin = n_bins<CLS>() - 1; bin >= 0; --bin) {
-        i64 nb = ((i64)counts[bin] + TIER_BS - 1) / TIER_BS;
-        if (b < nb) {
-            k0 = b * TIER_BS;
-            return bin;
-        }
-        b -= nb;
-    }
-    return -1;
-}
-
-// one inlined evaluation per tier: tier K of the bin's tuple
-template <int CLS, int SRC, int K>
-NRX_DI void tier_eval(int tier, const DevSys &S, i64 start, const i64 *__restrict__ idx, double *__restrict__ outE,
-                      double *__restrict__ outS, double *__restrict__ outX, double *__restrict__ outY, i64 t,
-                      PairRec (*stage)[TIER_BS])
-{
-    if constexpr (K >= 0) {
-        if (tier == K) {
-            tier_item<CLS, SRC, K>(S, start, idx, outE, outS, outX, outY, t, stage);
-            return;
-        }
-        tier_eval<CLS, SRC, K - 1>(tier, S, start, idx, outE, outS, outX, outY, t, stage);
-    }
-}
-
-// Every bin of a launch in one kernel, so that the bins' tails overlap:
-// lane per listed tuple, blocks past the bins exit.
-template <int CLS, int SRC>
-__global__ void __launch_bounds__(TIER_BS) k_prim_tiers(DevSys S, i64 start, const i64 *__restrict__ idx,
-                                                    double *__restrict__ outE, double *__restrict__ outS,
-                                                    double *__restrict__ outX, double *__restrict__ outY,
-                                                    const unsigned *__restrict__ list,
-                                                    const unsigned *__restrict__ counts)
-{
-    __shared__ PairRec stage[nel<CLS>() + 1][TIER_BS];
-    i64 k0 = 0;
-    const int bin = block_bin<CLS>(counts, (i64)blockIdx.x, k0);
-    if (bin < 0) return;
-    const i64 k = k0 + threadIdx.x;
-    if (k >= (i64)counts[bin]) return;
-    const i64 t = (i64)list[bin_offset(counts, bin) + k];
-    tier_eval<CLS, SRC, Tier<CLS>::N - 1>(bin / hub_bins<CLS>(), S, start, idx, outE, outS, outX, outY, t, stage);
-}
-
-__global__ void k_zero_u32n(unsigned *p, int n)
-{
-    if ((int)threadIdx.x < n) p[threadIdx.x] = 0u;
-}
-
-
-// tuples per launch of the primitive kernels (bounds the sorted list, whose
-// entries are 32-bit positions, and the bin counters)
-static const i64 PRIM_CHUNK = (i64)1 << 24;
-
+// primitive tuples of class CLS from tuple source SRC
 template <int CLS, int SRC>
 static int launch_prims(const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os, hipStream_t st,
                         double *ox = nullptr, double *oy = nullptr)
 {
-    constexpr int NBN = n_bins<CLS>();
-    static_assert(NBN + 1 <= 32, "bin counters (with the wide bin) and cursors fit the 256-byte header");
-    if constexpr (two_basis<CLS>())
-        if (SRC != SRC_LIST && (d.npebf1 <= 0 || d.npebf1 >= d.npebf))
-            return fail(NEORX_E_ARG, "class %d enumerates two electron bases; this handle has one", CLS);
-    if (ntup <= 0) return NEORX_OK;
-    i64 cap = std::min(ntup, PRIM_CHUNK);
-    // stream-ordered scratch: bin counters, the sorted tuple list and the bin codes
-    StreamBuf ws; // header: counts[32], cursors[32]; list: cap x u32; codes: cap x u8
-    int rc = ws.alloc(256 + cap * sizeof(unsigned) + cap, st);
-    if (rc) return rc;
-    unsigned *counts = (unsigned *)ws.p, *cursors = counts + 32, *list = (unsigned *)((char *)ws.p + 256);
-    unsigned char *code = (unsigned char *)(list + cap);
-    for (i64 off = 0; off < ntup; off += PRIM_CHUNK) {
-        i64 n = std::min(ntup - off, PRIM_CHUNK);
-        const i64 *ix = SRC == SRC_LIST ? idx + off * (2 * nel<CLS>() + 2) : nullptr;
-        double *e = oe + off, *s = os ? os + off : nullptr, *x = ox ? ox + off : nullptr;
-        double *y = oy ? oy + off : nullptr;
-        hipLaunchKernelGGL(k_zero_u32n, dim3(1), dim3(64), 0, st, counts, 64);
-        hipLaunchKernelGGL((k_prim_bin<CLS, SRC>), dim3(nblocks(n, 256)), dim3(256), 0, st, d, start + off, n, ix, e, s,
-                           x, y, code, counts);
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL((k_prim_scatter<CLS>), dim3(nblocks(n, 256)), dim3(256), 0, st, n, code, counts, cursors,
-                           list);
-        HIPCHK(hipGetLastError());
-        hipLaunchKernelGGL((k_prim_tiers<CLS, SRC>), dim3(nblocks(n, TIER_BS) + NBN), dim3(TIER_BS), 0, st, d, start + off, ix,
-                           e, s, x, y, list, counts);
-        HIPCHK(hipGetLastError());
-        if (d.lmax > 2) { // tuples with f functions: the wide bin
-            rc = nrx_wide_prims(CLS, SRC, d, start + off, ix, e, s, x, y, list, counts, NBN, n, st);
-            if (rc) return rc;
-        }
-    }
-    return NEORX_OK;
+    return nrx_prims(CLS, SRC, d, start, ntup, idx, oe, os, ox, oy, st);
 }
 
 static int prim_list(int64_t handle, int64_t cls, int64_t ntup, const int64_t *d_idx, double *d_ansE, double *d_ansS,
@@ -1614,10 +1405,19 @@ NRX_DI unsigned short buf_ld(const bf16_t *, __amdgpu_buffer_rsrc_t r, unsigned 
 // the scheduler issued narrow loads one at a time, each followed by a wait).
 #define NRX_LOADS_ISSUED() asm volatile("" ::: "memory")
 
-// loads in flight per lane in the EG3 slab loop when no tuned value is
-// recorded: 16 for FP64 storage and 12 for FP32 (both measured best at
-// nebf = 24), 16 for BF16
-template <class T> constexpr int eg3_unroll() { return sizeof(T) == 4 ? 12 : 16; }
+// Loads in flight per lane in the EG3 slab loop when no tuned value is
+// recorded, from sweeps over nebf 7 .. 32 (us, 8 / 12 / 16 / 24 in flight):
+//   FP64  20/6 3049 3005 3027 2817; 24/4 3622 3589 3584 3785; 28/2 3602 3455 3056 3295
+//   FP32  17/5 568 537 544 534; 19/4 693 647 658 688; 24/4 2226 2013 1975 1882; 28/2 3306 3043 2434 2714
+//   BF16  17/5 389 357 478 475; 20/6 1140 1019 1064 1051; 24/4 945 984 1413 2002; 28/2 843 877 844 1017
+template <class T> constexpr int eg3_unroll(i64 ne)
+{
+    if (ne <= 8) return 8;
+    if (sizeof(T) == 2) return ne <= 20 ? 12 : 8;
+    if (ne <= 12) return 12;
+    if (ne <= 16 || ne > 20) return 16;
+    return sizeof(T) == 4 ? 12 : 24;
+}
 
 // most lanes of one EG3 slab block (its launch bound)
 constexpr unsigned EG3_MAX_THREADS = 512;
@@ -1708,8 +1508,23 @@ NRX_DI void eg3_rows(__amdgpu_buffer_rsrc_t rb, unsigned row_d, unsigned row_c, 
     }
 }
 
+// the last r < R + 1 rows, c = c0 .., in one batch of their own
+template <class T, int R, int P, class A>
+NRX_DI void eg3_tail(unsigned r, __amdgpu_buffer_rsrc_t rb, unsigned row_d, unsigned row_c, unsigned voff, unsigned c0,
+                     const A *__restrict__ xd, const A *__restrict__ xb, const A *const *xf, A *s1, A *s2, A *s3)
+{
+    if constexpr (R > 0) {
+        if (r == R)
+            eg3_rows<T, R, P, A>(rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
+        else
+            eg3_tail<T, R - 1, P, A>(r, rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
+    }
+}
+
 // X, Y: the two densities (column-major ne x ne); Z: the density of the
-// nuclear-row term, or null.  P columns per lane (P divides ne).
+// nuclear-row term, or null.  P columns per lane (P divides ne).  With
+// gridDim.y splits a block takes its share of the b rows and writes the sums
+// F of that share to part[split][blk][x] (k_eg3_combine adds them in order).
 template <class T, int U, int P>
 __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const double *__restrict__ X,
                                                               const double *__restrict__ Y, const double *__restrict__ Z,
@@ -1730,6 +1545,7 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
     const unsigned nw = blockDim.x >> 6;
     double *Fw = sm + (threadIdx.x >> 6) * ne, *Ff = sm + nw * ne, *Xf = Ff + ne2, *Yt = Xf + ne * xs;
     float *Xs = (float *)(Yt + ne2);
+    const unsigned ns = gridDim.y, b0 = blockIdx.y * ne / ns, b1 = (blockIdx.y + 1) * ne / ns;
     const T *g = G + blk * (i64)ne4 * ne;
     for (unsigned k = threadIdx.x; k < nw * ne + ne2; k += blockDim.x) sm[k] = 0.0;
     for (unsigned k = threadIdx.x; k < ne2; k += blockDim.x) {
@@ -1760,7 +1576,7 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
             accf[p] = 0.0;
         }
         const unsigned voff = ef * (unsigned)sizeof(T);
-        for (unsigned b = 0; b < ne; ++b) {
+        for (unsigned b = b0; b < b1; ++b) {
             const double y_eb = on ? Ye[b] : 0.0;
             // row block b of the slab: ne^4 entries, at most 2^31 bytes for
             // nebf <= EG3_MAX_NE
@@ -1776,16 +1592,14 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
                     const unsigned row_d = d * ne2 * (unsigned)sizeof(T), row_c = ne3 * (unsigned)sizeof(T);
                     const A *xd = Xa + d * xstride;
                     unsigned c = 0;
-                    // U (then eight) independent loads in flight per lane
+                    // U (then the rest) independent loads in flight per lane
                     // before the FMAs; the slab is read once, so the loads are
-                    // nontemporal
+                    // nontemporal.  The rest goes as one batch: as an eight and
+                    // singles, each with its own wait, 17 functions in FP32
+                    // ran at 1.9 TB/s.
                     for (; c + U <= ne; c += U)
                         eg3_rows<T, U, P, A>(rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
-                    if (c + 8 <= ne) {
-                        eg3_rows<T, 8, P, A>(rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
-                        c += 8;
-                    }
-                    for (; c < ne; ++c) eg3_rows<T, 1, P, A>(rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
+                    eg3_tail<T, U - 1, P, A>(ne - c, rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
                 }
                 double vd = 0.0;
 #pragma unroll
@@ -1813,12 +1627,28 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
             double fx = 0.0;
             for (unsigned w = 0; w < nw; ++w) fx += sm[w * ne + x];
             for (unsigned e = 0; e < ne; ++e) fx += Ff[e * ne + x];
-            part[blk * (ne + 1) + x] = fx;
+            part[((i64)blockIdx.y * gridDim.x + blk) * (ne + 1) + x] = fx;
             if (Z) p += Z[x * ne + a] * fx;
         }
         p = wave_sum(p);
-        if (threadIdx.x == 0) part[blk * (ne + 1) + ne] = p / 3.0;
+        if (threadIdx.x == 0 && ns == 1) part[blk * (ne + 1) + ne] = p / 3.0;
     }
+}
+
+// the rows of every slab from its splits, and the Z-weighted sum; a wave per slab
+__global__ void __launch_bounds__(64) k_eg3_combine(i64 ne, int ns, const double *__restrict__ Z,
+                                                    const double *__restrict__ split, double *__restrict__ part)
+{
+    const i64 blk = blockIdx.x, a = blk % ne;
+    double p = 0.0;
+    for (i64 x = threadIdx.x; x < ne; x += 64) {
+        double fx = 0.0;
+        for (int s = 0; s < ns; ++s) fx += split[((i64)s * gridDim.x + blk) * (ne + 1) + x];
+        part[blk * (ne + 1) + x] = fx;
+        if (Z) p += Z[x * ne + a] * fx;
+    }
+    p = wave_sum(p);
+    if (threadIdx.x == 0) part[blk * (ne + 1) + ne] = p / 3.0;
 }
 
 // LDS bytes of k_eg3_slab: per-wavefront rows, per-column partials and the
@@ -1867,12 +1697,23 @@ struct Eg3Dens {
     const double *X, *Y, *Z;
 };
 
+// Splits of the b rows per slab: a launch of few slabs (small bases, odd
+// numbers of blocks over the 256 CUs) is cut until it has about 2048 blocks.
+// One pass with splits and whole last batches: 7/4 FP64 112 -> 12 us, 17/5 FP32
+// 1.17 -> 0.54 ms (4.5 TB/s), 20/8 FP64 5.75 -> 5.2 ms (6.3 TB/s).
+static int eg3_splits(i64 ne, i64 nblk) { return (int)std::max<i64>(1, std::min<i64>(ne, (2047 + nblk) / nblk)); }
+i64 nrx_eg3_split_doubles(i64 ne, i64 nblk)
+{
+    const int ns = eg3_splits(ne, nblk);
+    return ns > 1 ? ns * nblk * (ne + 1) : 0;
+}
+
 template <class T, int P>
-static int eg3_launch_u(int u, i64 ne, i64 nblk, Eg3Dens D, const T *g, double *part, hipStream_t st)
+static int eg3_launch_u(int u, i64 ne, i64 nblk, int ns, Eg3Dens D, const T *g, double *part, hipStream_t st)
 {
     const unsigned nt = eg3_threads_n(ne * ne / P);
     const size_t lds = eg3_lds(ne, nt);
-    const dim3 grid((unsigned)nblk), blk(nt);
+    const dim3 grid((unsigned)nblk, (unsigned)ns), blk(nt);
     switch (u) {
     case 8: hipLaunchKernelGGL((k_eg3_slab<T, 8, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
     case 12: hipLaunchKernelGGL((k_eg3_slab<T, 12, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
@@ -1884,32 +1725,47 @@ static int eg3_launch_u(int u, i64 ne, i64 nblk, Eg3Dens D, const T *g, double *
     return NEORX_OK;
 }
 
-static int eg3_launch(int dtype, int u, i64 ne, i64 nblk, Eg3Dens D, const void *g, double *part, hipStream_t st)
+// split: scratch of nrx_eg3_split_doubles (unused when that is 0)
+static int eg3_launch(int dtype, int u, i64 ne, i64 nblk, Eg3Dens D, const void *g, double *part, double *split,
+                      hipStream_t st)
 {
+    const int ns = eg3_splits(ne, nblk);
+    double *out = ns > 1 ? split : part;
+    int rc;
     switch (dtype) {
     case NRX_F64:
-        return eg3_launch_u<double, 1>(u ? u : eg3_unroll<double>(), ne, nblk, D, (const double *)g, part, st);
-    case NRX_F32: return eg3_launch_u<float, 1>(u ? u : eg3_unroll<float>(), ne, nblk, D, (const float *)g, part, st);
+        rc = eg3_launch_u<double, 1>(u ? u : eg3_unroll<double>(ne), ne, nblk, ns, D, (const double *)g, out, st);
+        break;
+    case NRX_F32:
+        rc = eg3_launch_u<float, 1>(u ? u : eg3_unroll<float>(ne), ne, nblk, ns, D, (const float *)g, out, st);
+        break;
     case NRX_BF16:
         if (eg3_pack(dtype, ne) == 2)
-            return eg3_launch_u<bf16_t, 2>(u ? u : eg3_unroll<bf16_t>(), ne, nblk, D, (const bf16_t *)g, part, st);
-        return eg3_launch_u<bf16_t, 1>(u ? u : eg3_unroll<bf16_t>(), ne, nblk, D, (const bf16_t *)g, part, st);
+            rc = eg3_launch_u<bf16_t, 2>(u ? u : eg3_unroll<bf16_t>(ne), ne, nblk, ns, D, (const bf16_t *)g, out, st);
+        else
+            rc = eg3_launch_u<bf16_t, 1>(u ? u : eg3_unroll<bf16_t>(ne), ne, nblk, ns, D, (const bf16_t *)g, out, st);
+        break;
     default: return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
     }
+    if (rc || ns == 1) return rc;
+    hipLaunchKernelGGL(k_eg3_combine, dim3((unsigned)nblk), dim3(64), 0, st, ne, ns, D.Z, split, part);
+    HIPCHK(hipGetLastError());
+    return NEORX_OK;
 }
 
 int nrx_eg3_slabs2(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g, int dtype,
-                   double *part, hipStream_t st)
+                   double *part, double *split, hipStream_t st)
 {
     if (ne <= 0 || ne > EG3_MAX_NE) return fail(NEORX_E_UNSUPPORTED, "EG3 slabs: nebf=%lld not in 1..%lld",
                                                 (long long)ne, (long long)EG3_MAX_NE);
     if (dtype < 0 || dtype > 2) return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
-    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, Eg3Dens{d_x, d_y, d_z}, g, part, st);
+    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, Eg3Dens{d_x, d_y, d_z}, g, part, split, st);
 }
 
-int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype, double *part, hipStream_t st)
+int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype, double *part, double *split,
+                  hipStream_t st)
 {
-    return nrx_eg3_slabs2(ne, nblk, d_de, d_de, d_de, g, dtype, part, st);
+    return nrx_eg3_slabs2(ne, nblk, d_de, d_de, d_de, g, dtype, part, split, st);
 }
 
 extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype, const double *d_de, const void *d_gm3,
@@ -1923,8 +1779,10 @@ extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype,
     if (!d_de || !d_gm3 || reps < 1) return fail(NEORX_E_ARG, "autotune EG3: bad arguments");
     const i64 nblk = np * np * ne;
     DevBuf part;
-    rc = part.alloc(nblk * (ne + 1) * 8);
+    const i64 nsp = nrx_eg3_split_doubles(ne, nblk);
+    rc = part.alloc((nblk * (ne + 1) + nsp) * 8);
     if (rc) return rc;
+    double *split = part.d() + nblk * (ne + 1);
     hipStream_t st = nullptr;
     HIPCHK(hipStreamCreate(&st));
     hipEvent_t e0, e1;
@@ -1934,10 +1792,10 @@ extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype,
     float bt = 0.0f;
     for (int k = 0; k < 4 && !rc; ++k) {
         const int u = EG3_UNROLLS[k];
-        rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), st); // warm-up
+        rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), split, st); // warm-up
         if (!rc) rc = hipEventRecord(e0, st) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventRecord failed");
         for (i64 r = 0; r < reps && !rc; ++r)
-            rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), st);
+            rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), split, st);
         if (!rc) rc = hipEventRecord(e1, st) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventRecord failed");
         if (!rc) rc = hipEventSynchronize(e1) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventSynchronize failed");
         float ms = 0.0f;
@@ -1993,10 +1851,10 @@ static int eg3_dev(int64_t nebf, int64_t npbf, const double *d_de, const double 
     i64 nblk = np * np * ne;
     Work W(st);
     double *part;
-    rc = W.get(part, nblk * (ne + 1) + np * np);
+    rc = W.get(part, nblk * (ne + 1) + np * np + nrx_eg3_split_doubles(ne, nblk));
     if (rc) return rc;
-    double *fpd = part + nblk * (ne + 1);
-    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, sizeof(T) == 8 ? NRX_F64 : NRX_F32, part, st);
+    double *fpd = part + nblk * (ne + 1), *split = fpd + np * np;
+    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, sizeof(T) == 8 ? NRX_F64 : NRX_F32, part, split, st);
     if (rc) return rc;
     hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + np * np, 256)), dim3(256), 0, st, ne, np, d_dp, part,
                        d_fe, fpd);
@@ -2042,9 +1900,12 @@ extern "C" int neorx_eg3ic1_noalloc_dev(int64_t nebf, int64_t npbf, const double
     HIPCHK(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEVICES || !g_scratch[dev])
         return fail(NEORX_E_NODEVICE, "neorx_eg3ic1_noalloc_dev: device %d was not set up by neorx_init", dev);
-    double *part = g_scratch[dev], *fpd = part + nblk * (ne + 1);
+    // splits exist for at most 2047 slabs: with their sums no more than
+    // 3 * 4094 * (nebf + 1) doubles, far inside the array
+    double *part = g_scratch[dev], *fpd = part + nblk * (ne + 1), *split = fpd + np * np;
+    static_assert((i64)3 * 4094 * (EG3_MAX_NE + 1) <= SCRATCH_DOUBLES, "the split sums fit the scratch array");
     hipStream_t st = (hipStream_t)stream;
-    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, NRX_F64, part, st);
+    rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, NRX_F64, part, split, st);
     if (rc) return rc;
     hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + np * np, 256)), dim3(256), 0, st, ne, np, d_dp, part,
                        d_fe, fpd);
@@ -2361,18 +2222,17 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     if (!rc && !pairs) rc = W.get(X, nb * ne6);
     if (!rc && !pairs) rc = W.get(Y, slab_cap(s, 3));
     if (!rc && pairs) rc = W.get(partq, s->plan.nq * ne * (ne + 1));
-    if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp);
+    // splits of any launch: their slab counts differ, each has at most 4094
+    if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp + 4094 * (ne + 1));
     if (rc) return rc;
-    double *fpd = part + npp * ne * (ne + 1);
+    double *fpd = part + npp * ne * (ne + 1), *split = fpd + npp;
     if (pairs) {
         for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
             const i64 q1 = std::min(s->plan.nq, q0 + nb);
             rc = nrx_gam3_pairs(s, false, q0, q1, 0, G, W);
             if (rc) return rc;
-            hipLaunchKernelGGL((k_eg3_slab<double, 16, 1>), dim3((unsigned)((q1 - q0) * ne)), dim3(eg3_threads(ne)),
-                               eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G,
-                               partq + q0 * ne * (ne + 1));
-            HIPCHK(hipGetLastError());
+            rc = nrx_eg3_slabs(ne, (q1 - q0) * ne, d_de, G, NRX_F64, partq + q0 * ne * (ne + 1), split, st);
+            if (rc) return rc;
         }
         hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * (ne + 1), 256)), dim3(256), 0, st, np,
                            ne * (ne + 1), partq, part);
@@ -2383,9 +2243,8 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
         rc = build3_block(s, p0, p1, X, Y, st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_gam3_symm, dim3(grid_blocks(n, 256)), dim3(256), 0, st, ne, n, X, G);
-        hipLaunchKernelGGL((k_eg3_slab<double, 16, 1>), dim3((unsigned)((p1 - p0) * ne)), dim3(eg3_threads(ne)),
-                           eg3_lds(ne, eg3_threads(ne)), st, ne, d_de, d_de, d_de, G, part + p0 * ne * (ne + 1));
-        HIPCHK(hipGetLastError());
+        rc = nrx_eg3_slabs(ne, (p1 - p0) * ne, d_de, G, NRX_F64, part + p0 * ne * (ne + 1), split, st);
+        if (rc) return rc;
     }
     hipLaunchKernelGGL(k_eg3_reduce, dim3(nblocks(ne * ne + npp, 256)), dim3(256), 0, st, ne, np, d_dp, part, d_fe,
                        fpd);

@@ -1032,6 +1032,7 @@ struct Xchf {
     double *zpart = nullptr, *rows = nullptr;
     // incremental EG3 builds: rows of the reference density, the reference
     // density and the pass's two densities
+    double *part3s = nullptr; // split sums of the EG3 pass
     double *part3ref = nullptr, *DEref = nullptr, *DXi = nullptr, *DYi = nullptr;
     i64 nz_fe = 1, nch_fp = 1, nz_dot = 1;
     double *FEs = nullptr, *SEs = nullptr, *FP23 = nullptr, *SP2 = nullptr;
@@ -1189,12 +1190,12 @@ int phase_a(Xchf *x, const double *DE, int dtype, int pass = G3_FULL)
     if (pass == G3_INC) {
         hipLaunchKernelGGL(k_inc_dens, dim3(nblocks(ne * ne, 256)), dim3(256), 0, st, ne * ne, DE, x->DEref, x->DXi,
                            x->DYi);
-        rc = nrx_eg3_slabs2(ne, nblk, x->DXi, x->DYi, nullptr, g, dtype, x->part3, st);
+        rc = nrx_eg3_slabs2(ne, nblk, x->DXi, x->DYi, nullptr, g, dtype, x->part3, x->part3s, st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_inc_rows, dim3((unsigned)nblk), dim3(64), 0, st, ne, nblk, DE, x->part3ref, x->part3);
         HIPCHK(hipGetLastError());
     } else {
-        rc = nrx_eg3_slabs(ne, nblk, DE, g, dtype, x->part3, st);
+        rc = nrx_eg3_slabs(ne, nblk, DE, g, dtype, x->part3, x->part3s, st);
         if (rc) return rc;
         if (pass == G3_REFRESH) {
             hipLaunchKernelGGL(k_copy, dim3(nblocks(nblk * (ne + 1), 256)), dim3(256), 0, st, nblk * (ne + 1),
@@ -1374,6 +1375,7 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
     x->nz_dot = 256;
     rc |= x->alloc(x->part2, x->nelec > 1 ? np2 * ne * 4 * ne : 1);
     rc |= x->alloc(x->part3, x->nelec > 2 ? np2 * ne * (ne + 1) : 1);
+    rc |= x->alloc(x->part3s, x->nelec > 2 ? nrx_eg3_split_doubles(ne, np2 * ne) : 1);
     rc |= x->alloc(x->part3ref, x->nelec > 2 ? np2 * ne * (ne + 1) : 1);
     rc |= x->alloc(x->DEref, ne2);
     rc |= x->alloc(x->DXi, ne2);
