@@ -520,8 +520,9 @@ int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype, const doub
  * the 5-particle contraction is evaluated in factorized form from GAM_ee and
  * GAM_2s, with the same result as EG4ICR on the in-core tensor.
  * store: bit mask of the storage types GAM_3 is kept in (1 FP64, 2 FP32,
- * 4 BF16); 0 means FP64; bit 8 also autotunes the EG3 contraction for each
- * stored type (neorx_autotune_eg3_dev).  The integrals are only built here:
+ * 4 BF16); 0 means FP64; bit 8 also autotunes the context's EG3 contraction
+ * for each stored type.  GAM_3 is held over its distinct nuclear pairs and
+ * distinct (i3,j3) pairs.  The integrals are only built here:
  * these entry points read no .ufm file.
  * Each context owns a non-blocking stream; neorx_xchf_scf on different
  * contexts may run from different host threads at once (graph capture is

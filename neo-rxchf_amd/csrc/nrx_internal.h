@@ -199,11 +199,15 @@ NRX_HIDDEN int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g
                              double *split, hipStream_t st);
 // doubles of the split scratch of such a launch (0: not used)
 NRX_HIDDEN i64 nrx_eg3_split_doubles(i64 ne, i64 nblk);
-// the same rows as the symmetric bilinear form T(X, Y) of two densities (X on
-// the (i2,j2) pair, Y on the (i3,j3) pair; T(DE, DE) are EG3IC1's rows), and
-// part[blk][ne] = sum_x Z(i1,x) F[x] / 3, or 0 when d_z is null
-NRX_HIDDEN int nrx_eg3_slabs2(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g,
-                              int dtype, double *part, double *split, hipStream_t st);
+// the rows of the symmetric bilinear form T(X, Y) of two densities (X on the
+// (i2,j2) pair, Y on the (i3,j3) pair; T(DE, DE) are EG3IC1's rows), and
+// part[blk][ne] = sum_x Z(i1,x) F[x] / 3, or 0 when d_z is null, over tensors
+// packed in the (i3,j3) pair (nrx_gam3_pairs with pack), slabs (q,i1); u:
+// loads in flight per lane, 0 for the default
+NRX_HIDDEN int nrx_eg3_packed(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g,
+                              int dtype, int u, double *part, double *split, hipStream_t st);
+// doubles of scratch it takes in `split`
+NRX_HIDDEN i64 nrx_eg3_packed_split_doubles(i64 ne, i64 nblk);
 // EG2IC1 slab partials of nblk slabs (ip,jp,i1): part[blk][4][ne] = dir, ex,
 // dirS, exS (gs may be NULL: the S rows stay zero)
 NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double *g, const double *gs, double *part,
@@ -215,8 +219,9 @@ NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double 
 // ------------------------------------------------------------------
 // GAM3_IC1 (mult: RXCHFmult_GAM3_XCHF) of the distinct nuclear pairs
 // [q0, q1).  npbf > 0: into the full tensor G, both orders of each pair;
-// npbf = 0: one block of nebf^6 per pair, from G on.
-NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, Work &W);
+// npbf = 0: one block of nebf^6 per pair, from G on.  pack: the third
+// electron's index pair over its distinct values only, [i1 j1][i2 j2][J(J+1)/2 + I].
+NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, Work &W, bool pack = false);
 // GAM2_IC1 (G = GM2ICR, Gs = GM2sICR) or, with rxne, RXCHFne_GAM2_IC1 (GM2ICR,
 // GM2exICR), nuclear pairs and blocks as above
 NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 npbf, double *G, double *Gs, Work &W);

@@ -1419,8 +1419,20 @@ template <class T> constexpr int eg3_unroll(i64 ne)
     return sizeof(T) == 4 ? 12 : 24;
 }
 
+// The same for the packed form (nebf, distinct nuclear pairs: us at 8 / 12 / 16 / 24):
+//   FP64  8,10 14 14 14 15; 10,55 66 55 59 60; 16,10 129 134 139 128; 18,1 45 43 44 41
+//   FP32  8,10 14 14 14 15; 10,55 43 46 47 49; 16,10 77 97 91 89; 18,1 43 39 40 34
+//   BF16  8,10 13 13 14 14; 10,55 39 35 45 49; 16,10 59 58 63 56; 18,1 39 36 44 35
+template <class T> constexpr int eg3p_unroll(i64 ne)
+{
+    if (sizeof(T) == 2) return ne <= 20 ? 12 : 8;
+    if (sizeof(T) == 4) return ne <= 16 ? 8 : 24;
+    return ne <= 12 ? 12 : 24;
+}
+
 // most lanes of one EG3 slab block (its launch bound)
 constexpr unsigned EG3_MAX_THREADS = 512;
+constexpr unsigned EG3P_THREADS = 256; // and of the packed form
 
 // P adjacent (e,f) columns of one stored row in one buffer load: P = 1 for
 // every storage type, P = 2 for BF16 (a 4-byte load, so a wavefront keeps
@@ -1635,7 +1647,156 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
     }
 }
 
-// the rows of every slab from its splits, and the Z-weighted sum; a wave per slab
+// The EG3 rows over a tensor that is symmetric in (e,f) and holds e >= f only
+// (packed at C = e(e+1)/2 + f): an entry stands for (e,f) and (f,e), so the
+// sums over c gain X(c,e) beside X(c,f), and each entry's terms are those of
+// k_eg3_slab in both orders (the second left out where e = f).  Half the
+// bytes and four FMAs an entry instead of three: the GM3 pass of a
+// device-resident context, which also keeps the distinct nuclear pairs only.
+// Lanes run over (d,C), which is contiguous in memory: d is then fixed in a
+// lane, F[d] needs no sum over the wavefront inside the loop over d, and few
+// lanes of a wavefront idle at any nebf.  Bound by HBM in FP64 (16 functions,
+// 10 pairs: 713 MB in 128 us, 5.6 TB/s; the full tensor is 3.8 times that)
+// and by the latency of load, LDS and FP32 chains in BF16 (178 MB in 57 us;
+// lanes over C alone, a wavefront sum per d: 118 us; split over b only, so
+// that set-up and closing sums are paid for one or two b: 156 us).
+template <class T, int R, int P, class A>
+NRX_DI void eg3p_rows(__amdgpu_buffer_rsrc_t rb, unsigned row_c, unsigned voff, unsigned c0, const A *xd,
+                      const A *__restrict__ xb, const A *const *xf, const A *const *xe, A (*s)[P])
+{
+    typename Pack<T, P>::raw r[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) r[k] = Pack<T, P>::ld(rb, voff, row_c * (c0 + k));
+    NRX_LOADS_ISSUED();
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+        const A xdk = xd[c0 + k], xbk = xb[c0 + k];
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            const A gv = (A)Pack<T, P>::get(r[k], p);
+            s[0][p] += xdk * gv;           // X(c,d)
+            s[1][p] += xbk * gv;           // X(c,b)
+            s[2][p] += xf[p][c0 + k] * gv; // X(c,f)
+            s[3][p] += xe[p][c0 + k] * gv; // X(c,e)
+        }
+    }
+}
+template <class T, int R, int P, class A>
+NRX_DI void eg3p_tail(unsigned r, __amdgpu_buffer_rsrc_t rb, unsigned row_c, unsigned voff, unsigned c0, const A *xd,
+                      const A *__restrict__ xb, const A *const *xf, const A *const *xe, A (*s)[P])
+{
+    if constexpr (R > 0) {
+        if (r == R)
+            eg3p_rows<T, R, P, A>(rb, row_c, voff, c0, xd, xb, xf, xe, s);
+        else
+            eg3p_tail<T, R - 1, P, A>(r, rb, row_c, voff, c0, xd, xb, xf, xe, s);
+    }
+}
+
+// A slab is split over cs groups of wpb wavefronts' columns, and those over b
+// where that is still few (Eg3Split).  LDS: Fw[nw][ne], Xf, Yt and Xs as in
+// k_eg3_slab
+template <class T, int U, int P>
+__global__ void __launch_bounds__(EG3P_THREADS) k_eg3_packed(i64 ne_, unsigned cs, unsigned wpb,
+                                                             const double *__restrict__ X,
+                                                             const double *__restrict__ Y,
+                                                             const double *__restrict__ Z, const T *__restrict__ G,
+                                                             double *__restrict__ part)
+{
+    using A = typename SlabAcc<T>::type;
+    constexpr bool F32 = sizeof(A) == 4;
+    extern __shared__ double sm[];
+    const unsigned ne = (unsigned)ne_, xs = ne + 1, nc = ne * (ne + 1) / 2, ncol = ne * nc / P;
+    const unsigned yc = blockIdx.y % cs, yb = blockIdx.y / cs, bs = gridDim.y / cs;
+    const unsigned wend = min(ncol, (yc + 1) * wpb * 64);
+    const i64 blk = blockIdx.x;
+    const unsigned a = (unsigned)(blk % ne), ne2 = ne * ne, nw = blockDim.x >> 6;
+    double *Fw = sm + (threadIdx.x >> 6) * ne, *Xf = sm + nw * ne, *Yt = Xf + ne * xs;
+    float *Xs = (float *)(Yt + ne2);
+    const size_t bsz = (size_t)ne2 * nc; // entries of one b: [c][d][C]
+    const unsigned b0 = yb * ne / bs, b1 = (yb + 1) * ne / bs;
+    const T *g = G + (size_t)blk * ne * bsz;
+    for (unsigned k = threadIdx.x; k < nw * ne; k += blockDim.x) sm[k] = 0.0;
+    for (unsigned k = threadIdx.x; k < ne2; k += blockDim.x) {
+        const unsigned r = k / ne, q = k % ne;
+        Xf[r * xs + q] = X[k]; // X(q, r)
+        Xs[r * xs + q] = (float)X[k];
+        Yt[k] = Y[q * ne + r]; // Y(r, q)
+    }
+    __syncthreads();
+    const A *Xa = F32 ? (const A *)(const void *)Xs : (const A *)(const void *)X; // columns shared by a wavefront
+    const A *Xc = F32 ? (const A *)(const void *)Xs : (const A *)(const void *)Xf;
+    const unsigned xstride = F32 ? xs : ne, row_c = ne * nc * (unsigned)sizeof(T);
+    const unsigned lane = threadIdx.x & 63;
+    for (unsigned w0 = yc * wpb * 64 + __builtin_amdgcn_readfirstlane(threadIdx.x & ~63u); w0 < wend; w0 += blockDim.x) {
+        const bool on = w0 + lane < ncol;
+        const unsigned w = on ? (w0 + lane) * P : 0, d = w / nc, C = w - d * nc;
+        unsigned e[P], f[P];
+        const A *xf[P], *xe[P], *xd = Xc + d * xs;
+        double y1[P], yed[P], yfd[P], accf[P], acce[P], accd = 0.0;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            e[p] = (unsigned)((__fsqrt_rn(8.0f * (float)(C + p) + 1.0f) - 1.0f) * 0.5f);
+            while (e[p] * (e[p] + 1) / 2 > C + p) --e[p];
+            while ((e[p] + 1) * (e[p] + 2) / 2 <= C + p) ++e[p];
+            f[p] = C + p - e[p] * (e[p] + 1) / 2;
+            xf[p] = Xc + f[p] * xs;
+            xe[p] = Xc + e[p] * xs;
+            const double wf = e[p] != f[p] ? 1.0 : 0.0;
+            y1[p] = Yt[e[p] * ne + f[p]] + wf * Yt[f[p] * ne + e[p]];
+            yed[p] = Yt[e[p] * ne + d];
+            yfd[p] = wf * Yt[f[p] * ne + d];
+            accf[p] = acce[p] = 0.0;
+        }
+        const unsigned voff = w * (unsigned)sizeof(T);
+        for (unsigned b = b0; b < b1; ++b) {
+            const __amdgpu_buffer_rsrc_t rb = buf_rsrc(g + b * bsz, (unsigned)(bsz * sizeof(T)));
+            const A *xb = Xa + b * xstride;
+            A s[4][P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) s[0][p] = s[1][p] = s[2][p] = s[3][p] = (A)0;
+            if (on) { // the other lanes' sums stay zero, and their terms with them
+                unsigned c = 0;
+                for (; c + U <= ne; c += U) eg3p_rows<T, U, P, A>(rb, row_c, voff, c, xd, xb, xf, xe, s);
+                eg3p_tail<T, U - 1, P, A>(ne - c, rb, row_c, voff, c, xd, xb, xf, xe, s);
+            }
+            double accb = 0.0;
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                const double yeb = Yt[e[p] * ne + b], yfb = e[p] != f[p] ? Yt[f[p] * ne + b] : 0.0;
+                const double t1 = s[0][p], t2 = s[1][p], t3 = s[2][p], t4 = s[3][p];
+                accb += y1[p] * t1 - 0.5 * (yed[p] * t3 + yfd[p] * t4);
+                accf[p] += 0.25 * yed[p] * t2 - 0.5 * yeb * t1;
+                acce[p] += 0.25 * yfd[p] * t2 - 0.5 * yfb * t1;
+                accd += -0.5 * y1[p] * t2 + 0.25 * (yeb * t3 + yfb * t4);
+            }
+            accb = wave_sum(accb);
+            if (lane == 0) Fw[b] += 3.0 * accb;
+        }
+        for (unsigned x = 0; x < ne; ++x) { // the lanes' F[d], F[e] and F[f]
+            double v = d == x ? accd : 0.0;
+#pragma unroll
+            for (int p = 0; p < P; ++p) v += (e[p] == x ? acce[p] : 0.0) + (f[p] == x ? accf[p] : 0.0);
+            v = wave_sum(v);
+            if (lane == 0) Fw[x] += 3.0 * v;
+        }
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        double p = 0.0;
+        for (unsigned x = threadIdx.x; x < ne; x += 64) {
+            double fx = 0.0;
+            for (unsigned w = 0; w < nw; ++w) fx += sm[w * ne + x];
+            part[((i64)blockIdx.y * gridDim.x + blk) * (ne + 1) + x] = fx;
+            if (Z) p += Z[x * ne + a] * fx;
+        }
+        p = wave_sum(p);
+        if (threadIdx.x == 0 && gridDim.y == 1) part[blk * (ne + 1) + ne] = p / 3.0;
+    }
+}
+
+// the rows of every slab from its splits, and the Z-weighted sum; a wave per
+// slab (unrolled: the splits' loads wait together, their sum keeps its order)
 __global__ void __launch_bounds__(64) k_eg3_combine(i64 ne, int ns, const double *__restrict__ Z,
                                                     const double *__restrict__ split, double *__restrict__ part)
 {
@@ -1643,6 +1804,7 @@ __global__ void __launch_bounds__(64) k_eg3_combine(i64 ne, int ns, const double
     double p = 0.0;
     for (i64 x = threadIdx.x; x < ne; x += 64) {
         double fx = 0.0;
+#pragma unroll 16
         for (int s = 0; s < ns; ++s) fx += split[((i64)s * gridDim.x + blk) * (ne + 1) + x];
         part[blk * (ne + 1) + x] = fx;
         if (Z) p += Z[x * ne + a] * fx;
@@ -1753,19 +1915,78 @@ static int eg3_launch(int dtype, int u, i64 ne, i64 nblk, Eg3Dens D, const void 
     return NEORX_OK;
 }
 
-int nrx_eg3_slabs2(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g, int dtype,
-                   double *part, double *split, hipStream_t st)
+// Blocks of a packed slab: wpb wavefronts' columns each (a wavefront takes
+// all b of its columns, which pays for its set-up and its closing sums), cs
+// of them, times bs ranges of b where the columns alone leave the chip idle.
+// 2048 blocks are aimed at (us for 1024 / 2048 / 4096: BF16 16,10 56 58 56;
+// FP64 18,1 58 43 47; FP64 8,10 15 14 15)
+struct Eg3Split {
+    i64 wpb, cs, bs;
+    Eg3Split(i64 ne, i64 nblk, i64 P)
+    {
+        const i64 ns = (2047 + nblk) / nblk, nwave = (ne * (ne * (ne + 1) / 2) / P + 63) / 64;
+        wpb = (nwave + ns - 1) / ns;
+        cs = (nwave + wpb - 1) / wpb;
+        bs = std::max<i64>(1, std::min(ne, ns / cs));
+    }
+};
+i64 nrx_eg3_packed_split_doubles(i64 ne, i64 nblk)
+{
+    const i64 ns = (2047 + nblk) / nblk; // no fewer than cs * bs
+    return ns > 1 ? ns * nblk * (ne + 1) : 0;
+}
+
+template <class T, int P>
+static int eg3_packed_u(int u, i64 ne, i64 nblk, int *ns, Eg3Dens D, const T *g, double *part, double *split,
+                        hipStream_t st)
+{
+    const Eg3Split S(ne, nblk, P);
+    const i64 passes = (S.wpb * 64 + EG3P_THREADS - 1) / EG3P_THREADS; // shared evenly by the block's wavefronts
+    const unsigned nt = 64u * (unsigned)((S.wpb + passes - 1) / passes);
+    *ns = (int)(S.cs * S.bs);
+    double *out = *ns > 1 ? split : part;
+    const size_t lds = (size_t)((nt / 64) * ne + ne * ne + ne * (ne + 1)) * 8 + (size_t)ne * (ne + 1) * 4;
+    const dim3 grid((unsigned)nblk, (unsigned)*ns), blk(nt);
+    const unsigned cs = (unsigned)S.cs, wpb = (unsigned)S.wpb;
+    switch (u) {
+    case 8: hipLaunchKernelGGL((k_eg3_packed<T, 8, P>), grid, blk, lds, st, ne, cs, wpb, D.X, D.Y, D.Z, g, out); break;
+    case 12: hipLaunchKernelGGL((k_eg3_packed<T, 12, P>), grid, blk, lds, st, ne, cs, wpb, D.X, D.Y, D.Z, g, out); break;
+    case 16: hipLaunchKernelGGL((k_eg3_packed<T, 16, P>), grid, blk, lds, st, ne, cs, wpb, D.X, D.Y, D.Z, g, out); break;
+    case 24: hipLaunchKernelGGL((k_eg3_packed<T, 24, P>), grid, blk, lds, st, ne, cs, wpb, D.X, D.Y, D.Z, g, out); break;
+    default: return fail(NEORX_E_ARG, "EG3 slabs: no variant with %d loads in flight", u);
+    }
+    HIPCHK(hipGetLastError());
+    return NEORX_OK;
+}
+
+int nrx_eg3_packed(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g, int dtype,
+                   int u, double *part, double *split, hipStream_t st)
 {
     if (ne <= 0 || ne > EG3_MAX_NE) return fail(NEORX_E_UNSUPPORTED, "EG3 slabs: nebf=%lld not in 1..%lld",
                                                 (long long)ne, (long long)EG3_MAX_NE);
-    if (dtype < 0 || dtype > 2) return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
-    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, Eg3Dens{d_x, d_y, d_z}, g, part, split, st);
+    const Eg3Dens D{d_x, d_y, d_z};
+    int rc, ns = 1;
+    if (dtype == NRX_F64)
+        rc = eg3_packed_u<double, 1>(u ? u : eg3p_unroll<double>(ne), ne, nblk, &ns, D, (const double *)g, part, split, st);
+    else if (dtype == NRX_F32)
+        rc = eg3_packed_u<float, 1>(u ? u : eg3p_unroll<float>(ne), ne, nblk, &ns, D, (const float *)g, part, split, st);
+    else if (ne * (ne + 1) / 2 % 2 == 0) // two columns per 4-byte load: every row starts on 4 bytes
+        rc = eg3_packed_u<bf16_t, 2>(u ? u : eg3p_unroll<bf16_t>(ne), ne, nblk, &ns, D, (const bf16_t *)g, part, split, st);
+    else
+        rc = eg3_packed_u<bf16_t, 1>(u ? u : eg3p_unroll<bf16_t>(ne), ne, nblk, &ns, D, (const bf16_t *)g, part, split, st);
+    if (rc || ns == 1) return rc;
+    hipLaunchKernelGGL(k_eg3_combine, dim3((unsigned)nblk), dim3(64), 0, st, ne, ns, D.Z, split, part);
+    HIPCHK(hipGetLastError());
+    return NEORX_OK;
 }
 
 int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype, double *part, double *split,
                   hipStream_t st)
 {
-    return nrx_eg3_slabs2(ne, nblk, d_de, d_de, d_de, g, dtype, part, split, st);
+    if (ne <= 0 || ne > EG3_MAX_NE) return fail(NEORX_E_UNSUPPORTED, "EG3 slabs: nebf=%lld not in 1..%lld",
+                                                (long long)ne, (long long)EG3_MAX_NE);
+    if (dtype < 0 || dtype > 2) return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
+    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, Eg3Dens{d_de, d_de, d_de}, g, part, split, st);
 }
 
 extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype, const double *d_de, const void *d_gm3,

@@ -410,11 +410,18 @@ __global__ void __launch_bounds__(64) k_fock_ee(i64 ne, const double *__restrict
 // ------------------------------------------------------------------
 // phase B: weighting by DP and the assembly of xchf1_fock
 // ------------------------------------------------------------------
+// number of the distinct nuclear pair of pq = ip*npbf + jp
+NRX_DI i64 nuc_pair(i64 pq, i64 np)
+{
+    const i64 ip = pq / np, jp = pq % np, a = min(ip, jp), b = max(ip, jp);
+    return b * (b + 1) / 2 + a;
+}
 // a wavefront per (a,b) of the electronic matrices (lanes over (ip,jp)) and
 // per (ip,jp) of the nuclear ones (lanes over (a,b)), fixed-order wave sums:
 //   FEs(a,b) = sum_pq DP(pq) [GAM_ep + GAM_1][pq][a][b] + EG2 + EG3 rows,
 //   SEs(a,b) = sum_pq DP(pq) GAM_1s[pq][a][b] + 2 SE2 (se1 + 2 se2),
-//   FPs(pq) = EG2 + EG3 nuclear sums; SP2(pq)
+//   FPs(pq) = EG2 + EG3 nuclear sums; SP2(pq);
+// the EG3 rows (part3) are those of the distinct nuclear pairs
 __global__ void __launch_bounds__(64) k_phaseB_rows(i64 ne, i64 np, const double *__restrict__ DE,
                                                     const double *__restrict__ DP, const double *__restrict__ Gep,
                                                     const double *__restrict__ G1, const double *__restrict__ G1s,
@@ -437,7 +444,7 @@ __global__ void __launch_bounds__(64) k_phaseB_rows(i64 ne, i64 np, const double
                     f2 += dp * 2.0 * (pr[b] - 0.5 * pr[ne + b]);
                     s2 += dp * (pr[2 * ne + b] - 0.5 * pr[3 * ne + b]);
                 }
-                if (has3) f3 += dp * part3[(pq * ne + a) * (ne + 1) + b];
+                if (has3) f3 += dp * part3[(nuc_pair(pq, np) * ne + a) * (ne + 1) + b];
             }
             f = wsum(f);
             s1 = wsum(s1);
@@ -459,7 +466,7 @@ __global__ void __launch_bounds__(64) k_phaseB_rows(i64 ne, i64 np, const double
                     f += dab * (pr[b] - 0.5 * pr[ne + b]);
                     fs += dab * (pr[2 * ne + b] - 0.5 * pr[3 * ne + b]);
                 }
-                if (has3 && b == 0) f3 += part3[(pq * ne + a) * (ne + 1) + ne];
+                if (has3 && b == 0) f3 += part3[(nuc_pair(pq, np) * ne + a) * (ne + 1) + ne];
             }
             f = wsum(f);
             fs = wsum(fs);
@@ -1022,7 +1029,11 @@ struct Xchf {
     // integrals (HBM)
     double *Se = nullptr, *Sp = nullptr, *He = nullptr, *Hp = nullptr, *Gep = nullptr, *Gee = nullptr;
     double *G1 = nullptr, *G1s = nullptr, *G2 = nullptr, *G2s = nullptr, *G3 = nullptr;
+    // GAM_3 (and its FP32 and BF16 copies) of the distinct nuclear pairs, the
+    // third electron's index pair over its distinct values: 0.29 of the full
+    // tensor, which is symmetric in both
     void *G3f = nullptr, *G3h = nullptr;
+    int u3[3] = {0, 0, 0}; // tuned loads in flight of the GM3 pass per storage type
     double *GeeU = nullptr, *G2sU = nullptr, *Xe = nullptr, *Xp = nullptr;
     // Fock-build workspace
     double *part2 = nullptr, *part3 = nullptr, *FPx = nullptr, *FEee = nullptr;
@@ -1179,23 +1190,23 @@ int phase_a_rest(Xchf *x, const double *DE)
 int phase_a(Xchf *x, const double *DE, int dtype, int pass = G3_FULL)
 {
     hipStream_t st = x->st;
-    const i64 ne = x->ne, np = x->np, np2 = np * np;
+    const i64 ne = x->ne;
     if (x->nelec <= 2) return phase_a_rest(x, DE);
     const void *g = dtype == NRX_F64 ? (const void *)x->G3 : dtype == NRX_F32 ? x->G3f : x->G3h;
     if (!g) return fail(NEORX_E_ARG, "GAM_3 is not held in storage type %d (see neorx_xchf_create store)", dtype);
     int rc = phase_a_rest(x, DE);
     if (rc) return rc;
     // the GM3 pass
-    const i64 nblk = np2 * ne;
+    const i64 nblk = x->s->plan.nq * ne;
     if (pass == G3_INC) {
         hipLaunchKernelGGL(k_inc_dens, dim3(nblocks(ne * ne, 256)), dim3(256), 0, st, ne * ne, DE, x->DEref, x->DXi,
                            x->DYi);
-        rc = nrx_eg3_slabs2(ne, nblk, x->DXi, x->DYi, nullptr, g, dtype, x->part3, x->part3s, st);
+        rc = nrx_eg3_packed(ne, nblk, x->DXi, x->DYi, nullptr, g, dtype, x->u3[dtype], x->part3, x->part3s, st);
         if (rc) return rc;
         hipLaunchKernelGGL(k_inc_rows, dim3((unsigned)nblk), dim3(64), 0, st, ne, nblk, DE, x->part3ref, x->part3);
         HIPCHK(hipGetLastError());
     } else {
-        rc = nrx_eg3_slabs(ne, nblk, DE, g, dtype, x->part3, x->part3s, st);
+        rc = nrx_eg3_packed(ne, nblk, DE, DE, DE, g, dtype, x->u3[dtype], x->part3, x->part3s, st);
         if (rc) return rc;
         if (pass == G3_REFRESH) {
             hipLaunchKernelGGL(k_copy, dim3(nblocks(nblk * (ne + 1), 256)), dim3(256), 0, st, nblk * (ne + 1),
@@ -1255,12 +1266,53 @@ int copy_on(hipStream_t st, void *dst, const void *src, size_t bytes, hipMemcpyK
     return NEORX_OK;
 }
 
+// loads in flight of the GM3 pass per held storage type, from timed launches
+int tune_g3(Xchf *x)
+{
+    const i64 ne = x->ne, nblk = x->s->plan.nq * ne;
+    Work W(x->st);
+    double *part;
+    int rc = W.get(part, nblk * (ne + 1) + nrx_eg3_packed_split_doubles(ne, nblk));
+    if (rc) return rc;
+    double *split = part + nblk * (ne + 1);
+    hipEvent_t ev[2];
+    HIPCHK(hipEventCreate(&ev[0]));
+    if (hipEventCreate(&ev[1]) != hipSuccess) {
+        (void)hipEventDestroy(ev[0]);
+        return fail(NEORX_E_HIP, "hipEventCreate failed");
+    }
+    const void *g[3] = {x->G3, x->G3f, x->G3h};
+    constexpr int depths[4] = {8, 12, 16, 24}, reps = 3;
+    for (int t = 0; t < 3 && !rc; ++t) {
+        float best = 0.0f;
+        for (int k = 0; k < 4 && g[t] && !rc; ++k) {
+            for (int r = 0; r <= reps && !rc; ++r) { // the first one warms up
+                if (r == 1) (void)hipEventRecord(ev[0], x->st);
+                rc = nrx_eg3_packed(ne, nblk, x->Se, x->Se, x->Se, g[t], t, depths[k], part, split, x->st);
+            }
+            float ms = 0.0f;
+            if (!rc && (hipEventRecord(ev[1], x->st) != hipSuccess || hipEventSynchronize(ev[1]) != hipSuccess ||
+                        hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess))
+                rc = fail(NEORX_E_HIP, "timing the GM3 pass failed");
+            if (!rc && (best == 0.0f || ms < best)) {
+                best = ms;
+                x->u3[t] = depths[k];
+            }
+        }
+        if (g_verbose && g[t] && !rc)
+            fprintf(stderr, "neorx: GM3 pass depth for storage %d: %d (%.3f ms)\n", t, x->u3[t], best / reps);
+    }
+    (void)hipEventDestroy(ev[0]);
+    (void)hipEventDestroy(ev[1]);
+    return rc;
+}
+
 int xchf_build(Xchf *x, i64 handle, i64 store)
 {
     System *s = x->s;
     hipStream_t st = x->st;
     const i64 ne = x->ne, np = x->np, ne2 = ne * ne, np2 = np * np, ne4 = ne2 * ne2;
-    const i64 ng1 = ne2 * np2, ng2 = ne4 * np2, ng3 = ne4 * ne2 * np2;
+    const i64 ng1 = ne2 * np2, ng2 = ne4 * np2, nq = s->plan.nq, ng3 = nq * ne4 * (ne * (ne + 1) / 2);
     int rc = 0;
     rc |= x->alloc(x->Se, ne2);
     rc |= x->alloc(x->Sp, np2);
@@ -1320,7 +1372,8 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
     if (x->nelec > 2) {
         rc = x->alloc(x->G3, ng3);
         if (rc) return rc;
-        rc = neorx_gam3_ic1_dev(handle, x->G3, st);
+        Work W(st);
+        rc = nrx_gam3_pairs(s, false, 0, s->plan.nq, 0, x->G3, W, true);
         if (rc) return rc;
         if (store & 2) {
             float *f = nullptr;
@@ -1338,21 +1391,10 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
         }
         HIPCHK(hipGetLastError());
         if (store & 8) {
-            // autotune the EG3 contraction on the stored tensors (the timing
-            // does not depend on the density; the overlap stands in for it)
-            HIPCHK(hipStreamSynchronize(st));
-            const void *g[3] = {x->G3, x->G3f, x->G3h};
-            for (int t = 0; t < 3; ++t)
-                if (g[t]) {
-                    int64_t best = 0;
-                    double bms = 0.0, all[4] = {};
-                    rc = neorx_autotune_eg3_dev(ne, np, t, x->Se, g[t], 3, &best, &bms, all);
-                    if (rc) return rc;
-                    if (g_verbose)
-                        fprintf(stderr, "neorx: EG3 slab depth for storage %d: %lld (%.3f ms; 8/12/16/24: %.3f %.3f %.3f "
-                                        "%.3f ms)\n",
-                                t, (long long)best, bms, all[0], all[1], all[2], all[3]);
-                }
+            // autotune the GM3 pass on the stored tensors (the timing does not
+            // depend on the density; the overlap stands in for it)
+            rc = tune_g3(x);
+            if (rc) return rc;
         }
         if (!(store & 1)) {
             HIPCHK(hipStreamSynchronize(st));
@@ -1374,9 +1416,9 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
     x->nch_fp = std::max<i64>(1, std::min<i64>(64, (ne4 + 4095) / 4096));
     x->nz_dot = 256;
     rc |= x->alloc(x->part2, x->nelec > 1 ? np2 * ne * 4 * ne : 1);
-    rc |= x->alloc(x->part3, x->nelec > 2 ? np2 * ne * (ne + 1) : 1);
-    rc |= x->alloc(x->part3s, x->nelec > 2 ? nrx_eg3_split_doubles(ne, np2 * ne) : 1);
-    rc |= x->alloc(x->part3ref, x->nelec > 2 ? np2 * ne * (ne + 1) : 1);
+    rc |= x->alloc(x->part3, x->nelec > 2 ? nq * ne * (ne + 1) : 1);
+    rc |= x->alloc(x->part3s, x->nelec > 2 ? nrx_eg3_packed_split_doubles(ne, nq * ne) : 1);
+    rc |= x->alloc(x->part3ref, x->nelec > 2 ? nq * ne * (ne + 1) : 1);
     rc |= x->alloc(x->DEref, ne2);
     rc |= x->alloc(x->DXi, ne2);
     rc |= x->alloc(x->DYi, ne2);

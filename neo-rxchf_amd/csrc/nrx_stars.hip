@@ -401,6 +401,7 @@ struct Gam3Out {
     double *G;        // full tensor, or the first block
     i64 blk;          // entries of one (ip,jp) block
     i64 np;           // > 0: block of nuclear pair (i,j) at i*np + j and j*np + i; 0: at q
+    int pack;         // the last index over the distinct pairs only
 };
 
 __global__ void __launch_bounds__(256) k_gam3_expand(PairPlan P, i64 ne, i64 q0, const double *__restrict__ T,
@@ -434,14 +435,15 @@ __global__ void __launch_bounds__(256) k_gam3_expand(PairPlan P, i64 ne, i64 q0,
         b[1] = jp * O.np + ip;
         nb = ip == jp ? 1 : 2;
     }
-    for (i64 x = threadIdx.x; x < ne2; x += blockDim.x) {
-        const double v = row[tri_index(x / ne, x % ne)];
+    const i64 len = O.pack ? nc : ne2;
+    for (i64 x = threadIdx.x; x < len; x += blockDim.x) {
+        const double v = row[O.pack ? x : tri_index(x / ne, x % ne)];
         for (int k = 0; k < nb; ++k)
             for (int u = 0; u < n1; ++u)
                 for (int w = 0; w < n2; ++w)
                     for (int z = 0; z < sw; ++z) {
                         const i64 P1 = z ? r2[w] : r1[u], P2 = z ? r1[u] : r2[w];
-                        O.G[b[k] * O.blk + (P1 * ne2 + P2) * ne2 + x] = v;
+                        O.G[b[k] * O.blk + (P1 * ne2 + P2) * len + x] = v;
                     }
     }
 }
@@ -770,7 +772,7 @@ int rec_ne(int deg) { return (deg <= 4 ? deg : deg <= 6 ? 6 : deg <= 8 ? 8 : 12)
 
 // V, X and T of the distinct nuclear pairs, then G (see Gam3Out).  mult: the
 // RXCHFmult form, without the one-geminal terms.
-int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G, Work &W)
+int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G, Work &W, bool pack)
 {
     hipStream_t st = W.st;
     const DevSys &d = s->d;
@@ -844,7 +846,8 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
                 }
             }
         }
-        Gam3Out O{np_full > 0 ? G : G + (q - q0) * ne * ne * ne * ne * ne * ne, ne * ne * ne * ne * ne * ne, np_full};
+        const i64 blk = ne * ne * ne * ne * (pack ? nc : ne * ne);
+        Gam3Out O{np_full > 0 ? G : G + (q - q0) * blk, blk, np_full, pack};
         hipLaunchKernelGGL(k_gam3_expand, dim3((unsigned)ntri, (unsigned)nqp), dim3(256), nc * 8, st, P, ne, q, T, V,
                            X + (q - q0) * nc, O);
         HIPCHK(hipGetLastError());
