@@ -69,6 +69,25 @@ NRX_DI double block_sum(double v, double *red)
     return t;
 }
 
+// N sums over the block at once, each as block_sum makes it; red holds >= 16 N
+template <int N> NRX_DI void block_sums(double (&v)[N], double *red)
+{
+    const int w = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+#pragma unroll
+    for (int k = 0; k < N; ++k) v[k] = wsum(v[k]);
+    __syncthreads();
+    if ((threadIdx.x & 63) == 0)
+        for (int k = 0; k < N; ++k) red[k * 16 + w] = v[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < N; ++k) {
+        double t = 0.0;
+        for (int i = 0; i < nw; ++i) t += red[k * 16 + i];
+        v[k] = t;
+    }
+    __syncthreads();
+}
+
 NRX_DI double block_max(double v, double *red)
 {
     v = wmax(v);
@@ -186,36 +205,51 @@ __global__ void k_to_f32s(i64 n, const double *__restrict__ x, float *__restrict
 // ------------------------------------------------------------------
 // FP64 MFMA GEMM: C[z] = sum_{k in chunk z} A(m,k) B(k,n) for the density
 // transforms of the factorized 5-particle term.  A(m,k) = A[m*sam + k*sak],
-// B(k,n) = B[k*sbk + n*sbn], C row-major with leading dimension ldc, chunk z
-// at C + z*zstride.  One wavefront per 16x16 tile of C with
-// v_mfma_f64_16x16x4_f64: lane l supplies A(m0 + l%16, k + l/16) and
+// B(k,n) = B[k*sbk + col(n)*sbn], C(m,n) at m*ldc + col(n), chunk z at
+// C + z*zstride; col(n) = (n / nin)*nout + n % nin runs a column index over
+// the rows of a higher tensor (col(n) = n with nin = N), so that an inner
+// index is carried without a transposed copy.  One wavefront per 16x16 tile
+// of C with v_mfma_f64_16x16x4_f64: lane l supplies A(m0 + l%16, k + l/16) and
 // B(k + l/16, n0 + l%16) and holds C(m0 + l/16 + 4i, n0 + l%16) in its i-th
-// accumulator, i < 4.
+// accumulator, i < 4.  Bound by the latency of its loads at these sizes: they
+// go GEMM_KB k-steps at a time (clamped inside the operands, the values beyond
+// k1, M and N selected to 0).
 // ------------------------------------------------------------------
 typedef double d4_t __attribute__((ext_vector_type(4)));
 
+constexpr int GEMM_KB = 4;
 __global__ void __launch_bounds__(256) k_gemm_f64(i64 M, i64 N, i64 K, i64 kchunk, const double *__restrict__ A,
                                                   i64 sam, i64 sak, const double *__restrict__ B, i64 sbk, i64 sbn,
-                                                  double *__restrict__ C, i64 ldc, i64 zstride)
+                                                  double *__restrict__ C, i64 ldc, i64 zstride, i64 nin, i64 nout)
 {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const i64 n0 = ((i64)blockIdx.x * (blockDim.x >> 6) + w) * 16, m0 = (i64)blockIdx.y * 16;
     if (n0 >= N) return; // the whole wavefront leaves together
     const i64 k0 = (i64)blockIdx.z * kchunk, k1 = std::min<i64>(K, k0 + kchunk);
     const int r = lane & 15, kq = lane >> 4;
-    const i64 am = m0 + r, bn = n0 + r;
-    const bool aon = am < M, bon = bn < N;
+    const i64 am = std::min<i64>(m0 + r, M - 1), bn = std::min<i64>(n0 + r, N - 1);
+    const i64 col = nin == N ? bn : bn / nin * nout + bn % nin;
+    const bool aon = m0 + r < M, bon = n0 + r < N;
+    const double *Ap = A + am * sam, *Bp = B + col * sbn;
     d4_t acc = {0.0, 0.0, 0.0, 0.0};
-    for (i64 k = k0; k < k1; k += 4) {
-        const i64 kk = k + kq;
-        const double a = (aon && kk < k1) ? A[am * sam + kk * sak] : 0.0;
-        const double b = (bon && kk < k1) ? B[kk * sbk + bn * sbn] : 0.0;
-        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, acc, 0, 0, 0);
+    for (i64 k = k0; k < k1; k += 4 * GEMM_KB) {
+        double a[GEMM_KB], b[GEMM_KB];
+#pragma unroll
+        for (int u = 0; u < GEMM_KB; ++u) {
+            const i64 kk = std::min<i64>(k + 4 * u + kq, k1 - 1);
+            a[u] = Ap[kk * sak];
+            b[u] = Bp[kk * sbk];
+        }
+#pragma unroll
+        for (int u = 0; u < GEMM_KB; ++u) {
+            const bool kon = k + 4 * u + kq < k1;
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(aon && kon ? a[u] : 0.0, bon && kon ? b[u] : 0.0, acc, 0, 0, 0);
+        }
     }
     double *Cz = C + (i64)blockIdx.z * zstride;
     for (int i = 0; i < 4; ++i) {
         const i64 m = m0 + kq + 4 * i;
-        if (m < M && bon) Cz[m * ldc + bn] = acc[i];
+        if (m < M && bon) Cz[m * ldc + col] = acc[i];
     }
 }
 
@@ -225,19 +259,9 @@ __global__ void k_sum_chunks(i64 n, i64 nz, const double *__restrict__ Cz, doubl
     GRID_LOOP(t, n)
     {
         double s = 0.0;
+#pragma unroll 8
         for (i64 z = 0; z < nz; ++z) s += Cz[z * n + t];
         C[t] = s;
-    }
-}
-
-// Y[(c,d)][(a,b)] = X[(a,b)][(c,d)] over pairs of an ne^4 tensor
-__global__ void k_pair_transpose(i64 ne, const double *__restrict__ X, double *__restrict__ Y)
-{
-    const i64 n2 = ne * ne;
-    GRID_LOOP(t, n2 * n2)
-    {
-        const i64 ab = t / n2, cd = t % n2;
-        Y[cd * n2 + ab] = X[t];
     }
 }
 
@@ -351,6 +375,7 @@ __global__ void k_sum_rows(i64 nrow, i64 ncol, const double *__restrict__ part, 
     GRID_LOOP(t, nrow)
     {
         double s = 0.0;
+#pragma unroll 16
         for (i64 c = 0; c < ncol; ++c) s += part[t * ncol + c];
         out[t] = s;
     }
@@ -497,8 +522,7 @@ __global__ void __launch_bounds__(1024) k_assemble(i64 ne, i64 np, int nelec, do
                                                    const double *__restrict__ E4, double *__restrict__ FE,
                                                    double *__restrict__ FP, double *__restrict__ comps)
 {
-    __shared__ double red[16];
-    __shared__ double sc[4];
+    __shared__ double red[16 * 9];
     const i64 ne2 = ne * ne, np2 = np * np;
     double ecore = 0.0, eee = 0.0;
     for (i64 t = threadIdx.x; t < ne2; t += blockDim.x) {
@@ -521,15 +545,10 @@ __global__ void __launch_bounds__(1024) k_assemble(i64 ne, i64 np, int nelec, do
         }
         if (nelec > 2) eg3 += dp * FP23[2 * np2 + t];
     }
-    ecore = block_sum(ecore, red);
-    eee = 0.5 * block_sum(eee, red);
-    pcore = block_sum(pcore, red);
-    eep = block_sum(eep, red);
-    eg1 = block_sum(eg1, red);
-    sg1 = block_sum(sg1, red);
-    eg2 = block_sum(eg2, red);
-    sg2 = block_sum(sg2, red);
-    eg3 = block_sum(eg3, red);
+    double sum[9] = {ecore, eee, pcore, eep, eg1, sg1, eg2, sg2, eg3};
+    block_sums(sum, red);
+    ecore = sum[0], eee = 0.5 * sum[1], pcore = sum[2], eep = sum[3], eg1 = sum[4];
+    sg1 = sum[5], eg2 = sum[6], sg2 = sum[7], eg3 = sum[8];
     const double eg4 = nelec > 2 ? E4[0] : 0.0;
     const double S = 1.0 + sg1 + sg2;
     const double psi = (ecore + pcore + eep + eee + eg1 + eg2 + eg3 + eg4) / S;
@@ -1093,52 +1112,45 @@ Xchf *get_x(i64 h)
 }
 
 // C (M x N) = A(M x K) B(K x N) through the MFMA GEMM, split over K when the
-// output is small; zpart holds the chunks
+// output is small, in chunks of 64 products: four load batches of the kernel.
+// (The 12 products of an SCF iteration at 8 functions: 8.0 us each in the mean
+// with chunks of 256 and one k-step of loads at a time, 3.2 us so.)  zpart
+// holds the chunks.  nin, nout: the GEMM's column map, with rows of C ldc apart
 int gemm(hipStream_t st, i64 M, i64 N, i64 K, const double *A, i64 sam, i64 sak, const double *B, i64 sbk, i64 sbn,
-         double *C, double *zpart, i64 zcap)
+         double *C, double *zpart, i64 zcap, i64 ldc = 0, i64 nin = 0, i64 nout = 0)
 {
     const i64 tm = (M + 15) / 16, tn = (N + 15) / 16;
     const i64 wpb = std::min<i64>(4, tn);
     i64 nz = 1;
-    if (tm * tn < 64 && K > 256) nz = std::min<i64>(zcap, (K + 255) / 256);
+    if (tm * tn < 64 && K > 256 && !nin) nz = std::min<i64>(zcap, (K + 63) / 64);
     const i64 kchunk = ((K + nz - 1) / nz + 3) / 4 * 4;
     nz = (K + kchunk - 1) / kchunk;
     dim3 grid((unsigned)((tn + wpb - 1) / wpb), (unsigned)tm, (unsigned)nz);
-    if (nz == 1) {
-        hipLaunchKernelGGL(k_gemm_f64, grid, dim3((unsigned)(64 * wpb)), 0, st, M, N, K, kchunk, A, sam, sak, B, sbk, sbn,
-                           C, N, (i64)0);
-    } else {
-        hipLaunchKernelGGL(k_gemm_f64, grid, dim3((unsigned)(64 * wpb)), 0, st, M, N, K, kchunk, A, sam, sak, B, sbk, sbn,
-                           zpart, N, M * N);
+    hipLaunchKernelGGL(k_gemm_f64, grid, dim3((unsigned)(64 * wpb)), 0, st, M, N, K, kchunk, A, sam, sak, B, sbk, sbn,
+                       nz == 1 ? C : zpart, ldc ? ldc : N, nz == 1 ? (i64)0 : M * N, nin ? nin : N, nout);
+    if (nz > 1)
         hipLaunchKernelGGL(k_sum_chunks, dim3(nblocks(M * N, 256)), dim3(256), 0, st, M * N, nz, zpart, C);
-    }
     HIPCHK(hipGetLastError());
     return NEORX_OK;
 }
 
-// Y[c][r] = sum_i D(i,c) X[i][r] over the leading index of an ne x R tensor
-// (D column-major: D(i,c) = D[c*ne + i], read row-major as [c][i])
-int lead_transform(Xchf *x, const double *D, const double *X, double *Y, i64 R)
+// an ne^4 tensor X[i0][b0][i1][b1] with one bra index carried by D
+// (column-major: D(i,c) = D[c*ne + i]): sum_i D(i,c) X[.. i ..], or with inv
+// sum_c D(i,c) X[.. c ..]; the index i0, or i1 (inner) as ne^2 products of
+// ne x ne matrices whose columns the GEMM walks as one index
+int bra_transform(Xchf *x, const double *D, bool inv, bool inner, const double *X, double *Y)
 {
-    return gemm(x->st, x->ne, R, x->ne, D, 1 * x->ne, 1, X, R, 1, Y, x->zpart, 1);
-}
-
-// the inverse direction: Y[i][r] = sum_c D(i,c) X[c][r]
-int lead_transform_inv(Xchf *x, const double *D, const double *X, double *Y, i64 R)
-{
-    return gemm(x->st, x->ne, R, x->ne, D, 1, x->ne, X, R, 1, Y, x->zpart, 1);
+    const i64 ne = x->ne, ne2 = ne * ne, ne3 = ne2 * ne, sam = inv ? 1 : ne, sak = inv ? ne : 1;
+    if (inner) return gemm(x->st, ne, ne3, ne, D, sam, sak, X, ne, 1, Y, x->zpart, 1, ne, ne, ne2);
+    return gemm(x->st, ne, ne3, ne, D, sam, sak, X, ne3, 1, Y, x->zpart, 1);
 }
 
 // both bra indices of an ne^4 tensor [i0][b0][i1][b1] carried by D:
-//   H = slot i1 only, T = both slots (t4: scratch)
+//   H = slot i1 only, T = both slots
 int both_bras(Xchf *x, const double *D, const double *G, double *H, double *T)
 {
-    const i64 ne = x->ne, ne3 = ne * ne * ne, ne4 = ne3 * ne;
-    hipLaunchKernelGGL(k_pair_transpose, dim3(grid_blocks(ne4, 256)), dim3(256), 0, x->st, ne, G, x->t4);
-    int rc = lead_transform(x, D, x->t4, T, ne3); // T[(c1 b1)][(i0 b0)]
-    if (rc) return rc;
-    hipLaunchKernelGGL(k_pair_transpose, dim3(grid_blocks(ne4, 256)), dim3(256), 0, x->st, ne, T, H);
-    return lead_transform(x, D, H, T, ne3);
+    const int rc = bra_transform(x, D, false, true, G, H);
+    return rc ? rc : bra_transform(x, D, false, false, H, T);
 }
 
 // how one phase A reads GAM_3
@@ -1172,11 +1184,8 @@ int phase_a_rest(Xchf *x, const double *DE)
         hipLaunchKernelGGL(k_g4_traces, dim3(grid_blocks(4 * ne * ne, 256)), dim3(256), 0, st, ne, x->A4, x->R4);
         hipLaunchKernelGGL(k_g4_adjoint, dim3(grid_blocks(ne4, 256)), dim3(256), 0, st, ne, x->A4, x->R4, x->Bb4);
         // GPbar(i2,b2,i3,b3) = sum D(i2,c2) D(i3,c3) Bbar(c2,b2,c3,b3)
-        hipLaunchKernelGGL(k_pair_transpose, dim3(grid_blocks(ne4, 256)), dim3(256), 0, st, ne, x->Bb4, x->t4);
-        rc = lead_transform_inv(x, DE, x->t4, x->GPb4, ne * ne * ne);
-        if (rc) return rc;
-        hipLaunchKernelGGL(k_pair_transpose, dim3(grid_blocks(ne4, 256)), dim3(256), 0, st, ne, x->GPb4, x->t4);
-        rc = lead_transform_inv(x, DE, x->t4, x->GPb4, ne * ne * ne);
+        rc = bra_transform(x, DE, true, true, x->Bb4, x->t4);
+        if (!rc) rc = bra_transform(x, DE, true, false, x->t4, x->GPb4);
         if (rc) return rc;
         const i64 chunk = (ne4 + x->nch_fp - 1) / x->nch_fp;
         hipLaunchKernelGGL(k_gemv_rows, dim3((unsigned)x->nch_fp, (unsigned)np2), dim3(256), 0, st, ne4, chunk, x->G2sU,
@@ -1414,7 +1423,7 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
     // workspace
     x->nz_fe = 64;
     x->nch_fp = std::max<i64>(1, std::min<i64>(64, (ne4 + 4095) / 4096));
-    x->nz_dot = 256;
+    x->nz_dot = std::max<i64>(1, std::min<i64>(256, (ne4 + 1023) / 1024));
     rc |= x->alloc(x->part2, x->nelec > 1 ? np2 * ne * 4 * ne : 1);
     rc |= x->alloc(x->part3, x->nelec > 2 ? nq * ne * (ne + 1) : 1);
     rc |= x->alloc(x->part3s, x->nelec > 2 ? nrx_eg3_packed_split_doubles(ne, nq * ne) : 1);
