@@ -1039,9 +1039,9 @@ __global__ void __launch_bounds__(64) k_inc_rows(i64 ne, i64 nblk, const double 
 // ------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------
+// (keeps nothing of its System, which the caller may destroy before it)
 struct Xchf {
-    System *s = nullptr;
-    i64 ne = 0, np = 0;
+    i64 ne = 0, np = 0, nq = 0; // functions; distinct nuclear pairs
     int nelec = 0;
     double enuc = 0.0;
     std::vector<void *> allocs;
@@ -1206,7 +1206,7 @@ int phase_a(Xchf *x, const double *DE, int dtype, int pass = G3_FULL)
     int rc = phase_a_rest(x, DE);
     if (rc) return rc;
     // the GM3 pass
-    const i64 nblk = x->s->plan.nq * ne;
+    const i64 nblk = x->nq * ne;
     if (pass == G3_INC) {
         hipLaunchKernelGGL(k_inc_dens, dim3(nblocks(ne * ne, 256)), dim3(256), 0, st, ne * ne, DE, x->DEref, x->DXi,
                            x->DYi);
@@ -1278,7 +1278,7 @@ int copy_on(hipStream_t st, void *dst, const void *src, size_t bytes, hipMemcpyK
 // loads in flight of the GM3 pass per held storage type, from timed launches
 int tune_g3(Xchf *x)
 {
-    const i64 ne = x->ne, nblk = x->s->plan.nq * ne;
+    const i64 ne = x->ne, nblk = x->nq * ne;
     Work W(x->st);
     double *part;
     int rc = W.get(part, nblk * (ne + 1) + nrx_eg3_packed_split_doubles(ne, nblk));
@@ -1316,12 +1316,11 @@ int tune_g3(Xchf *x)
     return rc;
 }
 
-int xchf_build(Xchf *x, i64 handle, i64 store)
+int xchf_build(Xchf *x, System *s, i64 handle, i64 store)
 {
-    System *s = x->s;
     hipStream_t st = x->st;
     const i64 ne = x->ne, np = x->np, ne2 = ne * ne, np2 = np * np, ne4 = ne2 * ne2;
-    const i64 ng1 = ne2 * np2, ng2 = ne4 * np2, nq = s->plan.nq, ng3 = nq * ne4 * (ne * (ne + 1) / 2);
+    const i64 ng1 = ne2 * np2, ng2 = ne4 * np2, nq = x->nq, ng3 = nq * ne4 * (ne * (ne + 1) / 2);
     int rc = 0;
     rc |= x->alloc(x->Se, ne2);
     rc |= x->alloc(x->Sp, np2);
@@ -1382,7 +1381,7 @@ int xchf_build(Xchf *x, i64 handle, i64 store)
         rc = x->alloc(x->G3, ng3);
         if (rc) return rc;
         Work W(st);
-        rc = nrx_gam3_pairs(s, false, 0, s->plan.nq, 0, x->G3, W, true);
+        rc = nrx_gam3_pairs(s, false, 0, nq, 0, x->G3, W, true);
         if (rc) return rc;
         if (store & 2) {
             float *f = nullptr;
@@ -1556,9 +1555,9 @@ extern "C" int neorx_xchf_create(int64_t handle, int64_t nelec, int64_t store, i
     if (s->d.nebf > RH_MAXN || s->d.npbf > RH_MAXN)
         return fail(NEORX_E_UNSUPPORTED, "ROOTHAN on the device supports at most %d basis functions", RH_MAXN);
     Xchf *x = new Xchf();
-    x->s = s;
     x->ne = s->d.nebf;
     x->np = s->d.npbf;
+    x->nq = x->np * (x->np + 1) / 2;
     x->nelec = (int)nelec;
     // Non-blocking: a context's stream takes no implicit dependency on the
     // legacy stream, so another thread's legacy-stream work cannot
@@ -1569,7 +1568,7 @@ extern "C" int neorx_xchf_create(int64_t handle, int64_t nelec, int64_t store, i
         delete x;
         return fail(NEORX_E_HIP, "hipStreamCreateWithFlags failed");
     }
-    rc = xchf_build(x, handle, store ? store : 1);
+    rc = xchf_build(x, s, handle, store ? store : 1);
     if (rc) {
         delete x;
         return rc;

@@ -334,3 +334,40 @@ def test_scf_batch_concurrent(torch_dev):
         x.close()
     for h in hs:
         h.close()
+
+
+def test_context_outlives_system(torch_dev):
+    """A context holds every integral, so its System may go first: the Fock
+    build and the SCF of contexts whose System was destroyed, with Systems of
+    other sizes created in its place, bit for bit those of a context whose
+    System is there."""
+    torch = torch_dev
+    s = _small(4, seed=82, n_e_centres=1, e_shells=(0, 1), contract=(1, 2), p_shells=(0, 1))
+    ne, npb = s["nebf"], s["npbf"]
+    print(f"case context outlives system nebf={ne} npbf={npb}", flush=True)
+    de = _dev(torch, synth.density(ne, 4.0, 5).ravel(order="F"))
+    dp = _dev(torch, synth.density(npb, 1.0, 6).ravel(order="F"))
+
+    def results(X):
+        o = [torch.zeros(n, dtype=torch.float64, device="cuda") for n in (ne * ne, npb * npb, 14)]
+        X.fock_dev(de.data_ptr(), dp.data_ptr(), "f64", *[x.data_ptr() for x in o])
+        torch.cuda.synchronize()
+        r = X.scf(tole=1e6, tolp=1e6)  # converged after its first iterations
+        return [x.cpu().numpy() for x in o] + [np.array(list(r["comps"].values())), r["CE"], r["CP"]]
+
+    S = neorx.System(s)
+    X = xchf.XCHF(S, 4)
+    want = results(X)
+    X.close()
+    X = xchf.XCHF(S, 4)
+    S.close()
+    others = [neorx.System(_small(4, seed=k, n_e_centres=1, e_shells=(0,), p_shells=(0,) * k)) for k in (3, 5, 7)]
+    for a, b in zip(results(X), want):
+        assert np.array_equal(a, b)
+    for o in others:
+        o.close()
+    X.close()
+    X = xchf.XCHF(neorx.System(s), 4)  # nothing but the context is kept
+    for a, b in zip(results(X), want):
+        assert np.array_equal(a, b)
+    X.close()
