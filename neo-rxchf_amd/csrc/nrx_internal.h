@@ -12,6 +12,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -217,11 +218,17 @@ NRX_HIDDEN int nrx_eg2_slabs(i64 ne, i64 nblk, const double *d_de, const double 
 // tensors from distinct pairs (nrx_stars.hip), l <= 2.  Enqueued on W's
 // stream, with scratch from W.
 // ------------------------------------------------------------------
-// GAM3_IC1 (mult: RXCHFmult_GAM3_XCHF) of the distinct nuclear pairs
-// [q0, q1).  npbf > 0: into the full tensor G, both orders of each pair;
-// npbf = 0: one block of nebf^6 per pair, from G on.  pack: the third
-// electron's index pair over its distinct values only, [i1 j1][i2 j2][J(J+1)/2 + I].
-NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 npbf, double *G, Work &W, bool pack = false);
+// GAM3_IC1 (mult: RXCHFmult_GAM3_XCHF) of every distinct nuclear pair.  npbf
+// > 0: into the full tensor G, both orders of each pair; npbf = 0: one block
+// of nebf^6 per pair, from G on.  nb > 0 (with npbf = 0): at most nb pairs at
+// a time, each batch [q0, q1) from the start of G, and sink called after it --
+// the scratch of one batch serves them all, and what does not depend on the
+// nuclear pair is formed once.  pack: the third electron's index pair over its
+// distinct values only, [i1 j1][i2 j2][J(J+1)/2 + I].
+using PairSink = std::function<int(i64 q0, i64 q1)>;
+NRX_HIDDEN int nrx_gam3_pairs(System *s, bool mult, i64 npbf, double *G, Work &W, bool pack = false, i64 nb = 0,
+                              const PairSink &sink = {});
 // GAM2_IC1 (G = GM2ICR, Gs = GM2sICR) or, with rxne, RXCHFne_GAM2_IC1 (GM2ICR,
-// GM2exICR), nuclear pairs and blocks as above
-NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 npbf, double *G, double *Gs, Work &W);
+// GM2exICR), nuclear pairs, blocks and batches as above
+NRX_HIDDEN int nrx_gam2_pairs(System *s, bool rxne, i64 npbf, double *G, double *Gs, Work &W, i64 nb = 0,
+                              const PairSink &sink = {});

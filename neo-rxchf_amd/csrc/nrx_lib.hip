@@ -885,7 +885,7 @@ extern "C" int neorx_gam2_ic1_dev(int64_t handle, double *d_gm2, double *d_gm2s,
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
         Work W(st);
-        int r = nrx_gam2_pairs(s, false, 0, s->plan.nq, np, d_gm2, d_gm2s, W);
+        int r = nrx_gam2_pairs(s, false, np, d_gm2, d_gm2s, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }
@@ -911,7 +911,7 @@ template <int CLS> static int gam3_build_dev(System *s, double *d_gm3, void *str
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
         Work W(st);
-        int r = nrx_gam3_pairs(s, CLS == 7, 0, s->plan.nq, np, d_gm3, W);
+        int r = nrx_gam3_pairs(s, CLS == 7, np, d_gm3, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }
@@ -2373,8 +2373,8 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
         return fail(NEORX_E_ARG, "null argument");
     i64 ne = s->d.nebf, np = s->d.npbf, ne4 = ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
-    i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne4));
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
+    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->plan.nq : npp, BLOCK_CAP / ne4));
     Work W(st);
     double *X = nullptr, *Xs = nullptr, *Y = nullptr, *Ys = nullptr, *partq = nullptr, *G, *Gs, *part, *fpd;
     i64 cap = slab_cap(s, 2);
@@ -2396,13 +2396,10 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     if (pairs) {
         // (underflow() of a primitive value, below 1e-100, is no part of this
         // form: the values never exist one by one)
-        for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
-            const i64 q1 = std::min(s->plan.nq, q0 + nb);
-            rc = nrx_gam2_pairs(s, false, q0, q1, 0, G, Gs, W);
-            if (!rc)
-                rc = eg2_slab_launch<double>(ne, (q1 - q0) * ne, d_de, G, Gs, partq + q0 * ne * 4 * ne, st);
-            if (rc) return rc;
-        }
+        rc = nrx_gam2_pairs(s, false, 0, G, Gs, W, nb, [&](i64 q0, i64 q1) {
+            return eg2_slab_launch<double>(ne, (q1 - q0) * ne, d_de, G, Gs, partq + q0 * ne * 4 * ne, st);
+        });
+        if (rc) return rc;
         hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * 4 * ne, 256)), dim3(256), 0, st, np, ne * 4 * ne,
                            partq, part);
         HIPCHK(hipGetLastError());
@@ -2435,8 +2432,8 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     if (!d_de || !d_dp || !d_fe || !d_fp || !d_e) return fail(NEORX_E_ARG, "null argument");
     i64 ne = s->d.nebf, np = s->d.npbf, ne6 = ne * ne * ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
-    i64 nb = std::max<i64>(1, std::min<i64>(npp, BLOCK_CAP / ne6));
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
+    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->plan.nq : npp, BLOCK_CAP / ne6));
     Work W(st);
     double *X = nullptr, *Y = nullptr, *partq = nullptr, *G, *part;
     int rc = W.get(G, nb * ne6);
@@ -2448,13 +2445,10 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     if (rc) return rc;
     double *fpd = part + npp * ne * (ne + 1), *split = fpd + npp;
     if (pairs) {
-        for (i64 q0 = 0; q0 < s->plan.nq; q0 += nb) {
-            const i64 q1 = std::min(s->plan.nq, q0 + nb);
-            rc = nrx_gam3_pairs(s, false, q0, q1, 0, G, W);
-            if (rc) return rc;
-            rc = nrx_eg3_slabs(ne, (q1 - q0) * ne, d_de, G, NRX_F64, partq + q0 * ne * (ne + 1), split, st);
-            if (rc) return rc;
-        }
+        rc = nrx_gam3_pairs(s, false, 0, G, W, false, nb, [&](i64 q0, i64 q1) {
+            return nrx_eg3_slabs(ne, (q1 - q0) * ne, d_de, G, NRX_F64, partq + q0 * ne * (ne + 1), split, st);
+        });
+        if (rc) return rc;
         hipLaunchKernelGGL(k_unfold_pairs, dim3(grid_blocks(npp * ne * (ne + 1), 256)), dim3(256), 0, st, np,
                            ne * (ne + 1), partq, part);
         HIPCHK(hipGetLastError());
@@ -3021,7 +3015,7 @@ extern "C" int neorx_rxchfne_gam2_ic1_dev(int64_t handle, double *d_gm2, double 
     hipStream_t st = (hipStream_t)stream;
     if (s->maxl <= 2) {
         Work W(st);
-        int r = nrx_gam2_pairs(s, true, 0, s->plan.nq, np, d_gm2, d_gm2ex, W);
+        int r = nrx_gam2_pairs(s, true, np, d_gm2, d_gm2ex, W);
         if (!r) HIPCHK(hipStreamSynchronize(st));
         return r;
     }

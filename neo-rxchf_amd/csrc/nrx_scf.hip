@@ -1381,7 +1381,7 @@ int xchf_build(Xchf *x, System *s, i64 handle, i64 store)
         rc = x->alloc(x->G3, ng3);
         if (rc) return rc;
         Work W(st);
-        rc = nrx_gam3_pairs(s, false, 0, nq, 0, x->G3, W, true);
+        rc = nrx_gam3_pairs(s, false, 0, x->G3, W, true);
         if (rc) return rc;
         if (store & 2) {
             float *f = nullptr;

@@ -772,7 +772,7 @@ int rec_ne(int deg) { return (deg <= 4 ? deg : deg <= 6 ? 6 : deg <= 8 ? 8 : 12)
 
 // V, X and T of the distinct nuclear pairs, then G (see Gam3Out).  mult: the
 // RXCHFmult form, without the one-geminal terms.
-int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G, Work &W, bool pack)
+int nrx_gam3_pairs(System *s, bool mult, i64 np_full, double *G, Work &W, bool pack, i64 nb, const PairSink &sink)
 {
     hipStream_t st = W.st;
     const DevSys &d = s->d;
@@ -780,19 +780,19 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
     const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2;
     const int ng = (int)d.ngtg, nt = ng * ng;
     double *lone, *T, *rec;
-    int rc = W.get(lone, LONE_F * P.nslot + nc * nc + nc * (q1 - q0) + nc * P.npl);
+    int rc = W.get(lone, LONE_F * P.nslot + nc * nc + nc * P.nq + nc * P.npl);
     if (rc) return rc;
-    double *V = lone + LONE_F * P.nslot, *X = V + nc * nc, *Vp = X + nc * (q1 - q0);
+    double *V = lone + LONE_F * P.nslot, *X = V + nc * nc, *Vp = X + nc * P.nq;
     hipLaunchKernelGGL(k_lone_prep, dim3((unsigned)(P.nslot / 64)), dim3(64), 0, st, d, P, lone);
     HIPCHK(hipGetLastError());
-    StarJob X1{0, P.npl, q0, q1 - q0, 0, 0, P.gx, nullptr, P.wx};
+    StarJob X1{0, P.npl, 0, P.nq, 0, 0, P.gx, nullptr, P.wx};
     X1.nterm = ng + ng * (ng + 1) / 2;
     if (mult) { // the two-geminal terms only: they follow the ng one-geminal ones
         X1.gk += ng;
         X1.w += ng;
         X1.nterm -= ng;
     }
-    hipLaunchKernelGGL(k_star_ovl, dim3(nblocks((q1 - q0) * nc, 64)), dim3(64), 0, st, d, P, X1, X);
+    hipLaunchKernelGGL(k_star_ovl, dim3(nblocks(P.nq * nc, 64)), dim3(64), 0, st, d, P, X1, X);
     HIPCHK(hipGetLastError());
     const int NE = rec_ne(4 * P.le + 2 * P.lp), NE1 = rec_ne(2 * P.le), RS = REC_HEAD + 3 * NE;
     const i64 star_b = (i64)nt * 3 * RS * 8;
@@ -806,7 +806,7 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
     };
     i64 nst = 0, nu = 0, big = 0;
     for (i64 B = 0; B < nc; ++B) big = std::max(big, span(B, B + 1, 1, nst, nu));
-    const i64 nqt = std::max<i64>(1, std::min<i64>({q1 - q0, T_BYTES / (ntri * nc * 8), (i64)32768})); // nuclear pairs T holds
+    const i64 nqt = std::max<i64>(1, std::min<i64>({nb ? nb : P.nq, P.nq, T_BYTES / (ntri * nc * 8), (i64)32768})); // nuclear pairs T holds
     const i64 nqr = std::max<i64>(1, std::min<i64>(nqt, REC_BYTES / big));               // and one launch takes
     const i64 vcap = P.npl * (REC_HEAD + 3 * NE1) * 8;
     if ((rc = W.get(T, nqt * ntri * nc))) return rc;
@@ -821,8 +821,8 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
         hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nc * nc, 256)), dim3(256), 0, st, P, nc, (i64)1, nc, Vp, V);
         HIPCHK(hipGetLastError());
     }
-    for (i64 q = q0; q < q1; q += nqt) {
-        const i64 nqp = std::min(nqt, q1 - q);
+    for (i64 q = 0; q < P.nq; q += nqt) {
+        const i64 nqp = std::min(nqt, P.nq - q);
         for (i64 k = 0; k < nqp; k += nqr) {
             const i64 nq = std::min(nqr, nqp - k);
             for (i64 B0 = 0, B1; B0 < nc; B0 = B1) {
@@ -847,22 +847,22 @@ int nrx_gam3_pairs(System *s, bool mult, i64 q0, i64 q1, i64 np_full, double *G,
             }
         }
         const i64 blk = ne * ne * ne * ne * (pack ? nc : ne * ne);
-        Gam3Out O{np_full > 0 ? G : G + (q - q0) * blk, blk, np_full, pack};
+        Gam3Out O{np_full > 0 || nb ? G : G + q * blk, blk, np_full, pack};
         hipLaunchKernelGGL(k_gam3_expand, dim3((unsigned)ntri, (unsigned)nqp), dim3(256), nc * 8, st, P, ne, q, T, V,
-                           X + (q - q0) * nc, O);
+                           X + q * nc, O);
         HIPCHK(hipGetLastError());
+        if (nb && (rc = sink(q, q + nqp))) return rc;
     }
     return NEORX_OK;
 }
 
-// GAM_2 and its overlaps (rxne: the RXCHF-ne tensors) of the distinct nuclear
-// pairs [q0, q1)
-int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G, double *Gs, Work &W)
+// GAM_2 and its overlaps (rxne: the RXCHF-ne tensors) of the distinct nuclear pairs
+int nrx_gam2_pairs(System *s, bool rxne, i64 np_full, double *G, double *Gs, Work &W, i64 nb, const PairSink &sink)
 {
     hipStream_t st = W.st;
     const DevSys &d = s->d;
     const PairPlan &P = s->plan;
-    const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2, nqa = q1 - q0;
+    const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2, nqa = nb ? std::min(nb, P.nq) : P.nq;
     const int ng = (int)d.ngtg, nt = ng * ng, nx = ng * (ng + 1) / 2 + (rxne ? 0 : ng);
     const int NE2 = rec_ne(2 * P.le + 2 * P.lp), nterms = rxne ? 1 : BT_OVL;
     const i64 nrows = (i64)nt * (rxne ? 1 : BT_ROWS);
@@ -891,53 +891,58 @@ int nrx_gam2_pairs(System *s, bool rxne, i64 q0, i64 q1, i64 np_full, double *G,
     const i64 nqr = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / big));
     const i64 nql = std::max<i64>(1, std::min<i64>(nqa, REC_BYTES / lone_b));
     if ((rc = W.get(rec, (std::max({nql * lone_b, nqr * big, std::min(nqr * all, REC_BYTES)}) + 7) / 8))) return rc;
-    for (i64 q = q0; q < q1; q += nql) { // L
-        const i64 nq = std::min(nql, q1 - q);
-        StarJob J{0, P.npl, q, nq, nx, NE2, P.gx + (rxne ? ng : 0), P.gx, P.wx + (rxne ? ng : 0)};
-        LoneJob Lj{0, nc, q, 0, P.npl, nx, NE2, nc, rxne ? 0.0 : 1.0};
-        double *part = rec + nq * P.npl * nx * 2 * (REC_HEAD + 3 * NE2), *o = L + (q - q0) * nc * nc;
-        rc = star_launch<2>(d, P, J, rec, st);
-        if (!rc) rc = lone_launch<2>(d, P, Lj, nq, rec, lone, P.npl > nc ? part : o, st);
-        if (rc) return rc;
-        if (P.npl > nc)
-            hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nc * nq * nc, 256)), dim3(256), 0, st, P, nc, nq, nc, part, o);
-        HIPCHK(hipGetLastError());
-    }
     const int dmax = 4 * P.le + 2 * P.lp; // per direction and in total
-    for (i64 q = q0; q < q1; q += nqr) { // B, Y
-        const i64 nq = std::min(nqr, q1 - q);
-        for (i64 B0 = 0, B1; B0 < nc; B0 = B1) {
-            B1 = B0 + 1;
-            while (B1 < nc && nq * span(B0, B1 + 1, nst, nu) <= REC_BYTES) ++B1;
-            span(B0, B1, nst, nu);
-            const i64 s0 = s->cp_start[B0], n = nst * nq;
-            StarJob J{s0 * (s0 + 1) / 2, nst, q, nq, nt, 0, P.gk, P.gl, P.wkl};
-            LoneJob U{B0 * (B0 + 1) / 2, nu, q, 0, 0, 0, 0, ntri, 0.0};
-            unsigned *list = (unsigned *)(rec + std::max<i64>(nrows, 2) * n);
-            hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, counts);
-            hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 0, counts, list);
-            hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 1, counts, list);
-            const dim3 g((unsigned)std::min<i64>(BOND_BLOCKS, (n * nt + 63) / 64), (unsigned)nterms);
+    for (i64 q0 = 0; q0 < P.nq; q0 += nqa) {
+        const i64 q1 = std::min(P.nq, q0 + nqa);
+        for (i64 q = q0; q < q1; q += nql) { // L
+            const i64 nq = std::min(nql, q1 - q);
+            StarJob J{0, P.npl, q, nq, nx, NE2, P.gx + (rxne ? ng : 0), P.gx, P.wx + (rxne ? ng : 0)};
+            LoneJob Lj{0, nc, q, 0, P.npl, nx, NE2, nc, rxne ? 0.0 : 1.0};
+            double *part = rec + nq * P.npl * nx * 2 * (REC_HEAD + 3 * NE2), *o = L + (q - q0) * nc * nc;
+            rc = star_launch<2>(d, P, J, rec, st);
+            if (!rc) rc = lone_launch<2>(d, P, Lj, nq, rec, lone, P.npl > nc ? part : o, st);
+            if (rc) return rc;
+            if (P.npl > nc)
+                hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nc * nq * nc, 256)), dim3(256), 0, st, P, nc, nq, nc, part,
+                                   o);
+            HIPCHK(hipGetLastError());
+        }
+        for (i64 q = q0; q < q1; q += nqr) { // B, Y
+            const i64 nq = std::min(nqr, q1 - q);
+            for (i64 B0 = 0, B1; B0 < nc; B0 = B1) {
+                B1 = B0 + 1;
+                while (B1 < nc && nq * span(B0, B1 + 1, nst, nu) <= REC_BYTES) ++B1;
+                span(B0, B1, nst, nu);
+                const i64 s0 = s->cp_start[B0], n = nst * nq;
+                StarJob J{s0 * (s0 + 1) / 2, nst, q, nq, nt, 0, P.gk, P.gl, P.wkl};
+                LoneJob U{B0 * (B0 + 1) / 2, nu, q, 0, 0, 0, 0, ntri, 0.0};
+                unsigned *list = (unsigned *)(rec + std::max<i64>(nrows, 2) * n);
+                hipLaunchKernelGGL(k_zero_counts, dim3(1), dim3(64), 0, st, counts);
+                hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 0, counts, list);
+                hipLaunchKernelGGL(k_bond_bin, dim3(nblocks(n, 256)), dim3(256), 0, st, P, J, 1, counts, list);
+                const dim3 g((unsigned)std::min<i64>(BOND_BLOCKS, (n * nt + 63) / 64), (unsigned)nterms);
 #define NRX_BOND(K)                                                                                                   \
     if (K == 0 || dmax >= BTIER_NL[K ? K - 1 : 0] || dmax >= BTIER_NB[K ? K - 1 : 0])                                 \
     hipLaunchKernelGGL((k_bond<K>), g, dim3(64), 0, st, d, P, J, (int)rxne, kt, counts, list, rec)
-            NRX_BOND(4);
-            NRX_BOND(3);
-            NRX_BOND(2);
-            NRX_BOND(1);
-            NRX_BOND(0);
+                NRX_BOND(4);
+                NRX_BOND(3);
+                NRX_BOND(2);
+                NRX_BOND(1);
+                NRX_BOND(0);
 #undef NRX_BOND
-            hipLaunchKernelGGL(k_bond_rows, dim3(grid_blocks(n, 256)), dim3(256), 0, st, n, (i64)nterms * nt,
-                               (i64)BT_OVL * nt, rxne ? (i64)0 : (i64)nt, rec);
-            const i64 o = (q - q0) * ntri + U.u0;
-            hipLaunchKernelGGL(k_bond_sum, dim3(grid_blocks(nu * nq, 256)), dim3(256), 0, st, P, J, U, rec,
-                               B + o, rxne ? nullptr : Y + o);
-            HIPCHK(hipGetLastError());
+                hipLaunchKernelGGL(k_bond_rows, dim3(grid_blocks(n, 256)), dim3(256), 0, st, n, (i64)nterms * nt,
+                                   (i64)BT_OVL * nt, rxne ? (i64)0 : (i64)nt, rec);
+                const i64 o = (q - q0) * ntri + U.u0;
+                hipLaunchKernelGGL(k_bond_sum, dim3(grid_blocks(nu * nq, 256)), dim3(256), 0, st, P, J, U, rec,
+                                   B + o, rxne ? nullptr : Y + o);
+                HIPCHK(hipGetLastError());
+            }
         }
+        const i64 nout = (np_full > 0 ? np_full * np_full : q1 - q0) * ne * ne * ne * ne;
+        hipLaunchKernelGGL(k_gam2_expand, dim3(grid_blocks(nout, 256)), dim3(256), 0, st, ne, nc, q0, q1 - q0, np_full,
+                           (int)rxne, L, B, Y, G, Gs);
+        HIPCHK(hipGetLastError());
+        if (nb && (rc = sink(q0, q1))) return rc;
     }
-    const i64 nout = (np_full > 0 ? np_full * np_full : nqa) * ne * ne * ne * ne;
-    hipLaunchKernelGGL(k_gam2_expand, dim3(grid_blocks(nout, 256)), dim3(256), 0, st, ne, nc, q0, nqa, np_full, (int)rxne,
-                       L, B, Y, G, Gs);
-    HIPCHK(hipGetLastError());
     return NEORX_OK;
 }
