@@ -1406,9 +1406,15 @@ NRX_DI unsigned short buf_ld(const bf16_t *, __amdgpu_buffer_rsrc_t r, unsigned 
 #define NRX_LOADS_ISSUED() asm volatile("" ::: "memory")
 
 // Loads in flight per lane in the EG3 slab loop when no tuned value is
-// recorded, from sweeps over nebf 7 .. 32 (us, 8 / 12 / 16 / 24 in flight):
-//   FP64  20/6 3049 3005 3027 2817; 24/4 3622 3589 3584 3785; 28/2 3602 3455 3056 3295
-//   FP32  17/5 568 537 544 534; 19/4 693 647 658 688; 24/4 2226 2013 1975 1882; 28/2 3306 3043 2434 2714
+// recorded, from a sweep over 35 sizes of nebf 6 .. 32 at the splits of
+// eg3_splits (us, 8 / 12 / 16 / 24 in flight).  Split that far the depth
+// matters little; the lines lie where one does:
+//   FP64   8/8 33 33 33 34;  10/8 100 97 98 98;  13/6 255 258 253 254;  16/6 701 694 700 697;
+//         17/8 2141 2205 2209 2200;  20/8 4986 4932 4953 4797;  21/4 1912 1935 1937 1927;
+//         24/8 14140 14257 14265 14291;  28/3 5512 5382 5186 5366
+//   FP32   8/8 22 21 22 23;  10/8 72 62 63 65;  13/6 147 150 145 145;  16/6 364 368 369 367;
+//         17/8 1252 1183 1187 1250;  20/8 2861 2893 2901 3002;  21/4 989 1053 1064 1114;
+//         24/8 7219 7227 7182 7205;  28/3 4810 4434 3636 3928
 //   BF16  17/5 389 357 478 475; 20/6 1140 1019 1064 1051; 24/4 945 984 1413 2002; 28/2 843 877 844 1017
 template <class T> constexpr int eg3_unroll(i64 ne)
 {
@@ -1859,11 +1865,18 @@ struct Eg3Dens {
     const double *X, *Y, *Z;
 };
 
-// Splits of the b rows per slab: a launch of few slabs (small bases, odd
-// numbers of blocks over the 256 CUs) is cut until it has about 2048 blocks.
-// One pass with splits and whole last batches: 7/4 FP64 112 -> 12 us, 17/5 FP32
-// 1.17 -> 0.54 ms (4.5 TB/s), 20/8 FP64 5.75 -> 5.2 ms (6.3 TB/s).
-static int eg3_splits(i64 ne, i64 nblk) { return (int)std::max<i64>(1, std::min<i64>(ne, (2047 + nblk) / nblk)); }
+// Splits of the b rows per slab: a launch of few slabs is cut until it has
+// about 8192 blocks (four to eight of them fit a CU, so fewer leave the last
+// round of a launch nearly empty).  2048 / 4096 / 8192 / 12288 blocks over
+// 70 launches (nebf 6 .. 32, FP64 and FP32): 11.7 / 6.4 / 3.1 / 2.8 % above
+// the fastest split of each in the mean; 24/8 FP64 14818 -> 14265 us, FP32
+// 7488 -> 7182; 17/5 FP64 931 -> 841, FP32 534 -> 464; 28/3 FP32 5563 -> 3636.
+// Two blocks a slab are slower than one at 24/8 (14495 and 7234 us).
+constexpr i64 EG3_BLOCKS = 8192;
+static int eg3_splits(i64 ne, i64 nblk)
+{
+    return (int)std::max<i64>(1, std::min<i64>(ne, (EG3_BLOCKS - 1 + nblk) / nblk));
+}
 i64 nrx_eg3_split_doubles(i64 ne, i64 nblk)
 {
     const int ns = eg3_splits(ne, nblk);
@@ -2121,10 +2134,11 @@ extern "C" int neorx_eg3ic1_noalloc_dev(int64_t nebf, int64_t npbf, const double
     HIPCHK(hipGetDevice(&dev));
     if (dev < 0 || dev >= MAX_DEVICES || !g_scratch[dev])
         return fail(NEORX_E_NODEVICE, "neorx_eg3ic1_noalloc_dev: device %d was not set up by neorx_init", dev);
-    // splits exist for at most 2047 slabs: with their sums no more than
-    // 3 * 4094 * (nebf + 1) doubles, far inside the array
+    // splits exist for at most EG3_BLOCKS - 1 slabs, of less than 2 EG3_BLOCKS
+    // blocks in all: with their sums no more than 3 (EG3_BLOCKS - 1) (nebf + 1)
+    // doubles and np*np of fpd, inside the array
     double *part = g_scratch[dev], *fpd = part + nblk * (ne + 1), *split = fpd + np * np;
-    static_assert((i64)3 * 4094 * (EG3_MAX_NE + 1) <= SCRATCH_DOUBLES, "the split sums fit the scratch array");
+    static_assert((3 * EG3_MAX_NE + 4) * (EG3_BLOCKS - 1) <= SCRATCH_DOUBLES, "the split sums fit the scratch array");
     hipStream_t st = (hipStream_t)stream;
     rc = nrx_eg3_slabs(ne, nblk, d_de, d_gm3, NRX_F64, part, split, st);
     if (rc) return rc;
@@ -2440,8 +2454,8 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     if (!rc && !pairs) rc = W.get(X, nb * ne6);
     if (!rc && !pairs) rc = W.get(Y, slab_cap(s, 3));
     if (!rc && pairs) rc = W.get(partq, s->plan.nq * ne * (ne + 1));
-    // splits of any launch: their slab counts differ, each has at most 4094
-    if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp + 4094 * (ne + 1));
+    // splits of any launch: their slab counts differ, each has less than 2 EG3_BLOCKS
+    if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp + 2 * EG3_BLOCKS * (ne + 1));
     if (rc) return rc;
     double *fpd = part + npp * ne * (ne + 1), *split = fpd + npp;
     if (pairs) {

@@ -13,7 +13,9 @@ from _util import check_close
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("ne,npb", [(1, 1), (2, 3), (7, 1), (9, 2), (13, 1), (17, 1), (21, 1)])
+@pytest.mark.parametrize("ne,npb", [(1, 1), (2, 3), (7, 1), (9, 2), (13, 1), (17, 1), (21, 1),
+                                    # 2400, 7938 and 8192 slabs: split into four, two and one
+                                    (6, 20), (2, 63), (2, 64)])
 def test_eg3_batches(ne, npb):
     import torch
 
