@@ -502,10 +502,14 @@ int neorx_rxchfmult_omg_dev(int64_t k, int64_t nebf, int64_t nebfbe, int64_t npb
                             double *d_fp, double *d_fbe, double *d_e, void *stream);
 
 /* ---- autotuner (no counterpart in the reference) ---------------------------
- * Times the EG3IC1 slab kernel with 8, 12, 16 and 24 loads in flight per lane
- * on the caller's tensor (dtype 0 FP64, 1 FP32, 2 BF16 storage; reps timed
- * launches each) and records the fastest for (dtype, nebf): every later EG3
- * contraction of that storage type and basis size in this process uses it.
+ * Times the EG3 passes with 8, 12, 16 and 24 loads in flight per lane on the
+ * caller's tensor (dtype 0 FP64, 1 FP32, 2 BF16 storage; reps timed launches
+ * each) and records the fastest for (dtype, nebf): every later EG3 contraction
+ * of that storage type and basis size in this process uses it -- EG3IC1 and
+ * GAM3_DSCF the depth of the in-core pass, an XCHF context that was not tuned
+ * by itself (store bit 8) that of its own pass, timed over as many entries of
+ * d_gm3 as its packed GAM_3 holds.  The results are those of the in-core pass;
+ * for BF16, which only contexts read, those of theirs.
  * best_unroll, best_ms and all_ms[4] (per candidate) may be NULL. */
 int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype, const double *d_de, const void *d_gm3,
                            int64_t reps, int64_t *best_unroll, double *best_ms, double *all_ms);

@@ -195,7 +195,7 @@ NRX_HIDDEN int nrx_gam_ee_launch(System *s, double *d_gee, hipStream_t st);
 NRX_HIDDEN int nrx_gam1_launch(System *s, double *d_g1, double *d_g1s, hipStream_t st);
 // EG3IC1 slab partials of nblk slabs (ip,jp,i1): part[blk][0..ne-1] = the FE
 // row before the DP(ip,jp) weight, part[blk][ne] = its DE-weighted sum / 3;
-// g of storage type dtype
+// g in FP64 or FP32
 NRX_HIDDEN int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype, double *part,
                              double *split, hipStream_t st);
 // doubles of the split scratch of such a launch (0: not used)
@@ -204,10 +204,14 @@ NRX_HIDDEN i64 nrx_eg3_split_doubles(i64 ne, i64 nblk);
 // (i2,j2) pair, Y on the (i3,j3) pair; T(DE, DE) are EG3IC1's rows), and
 // part[blk][ne] = sum_x Z(i1,x) F[x] / 3, or 0 when d_z is null, over tensors
 // packed in the (i3,j3) pair (nrx_gam3_pairs with pack), slabs (q,i1); u:
-// loads in flight per lane, 0 for the default
+// loads in flight per lane, 0 for the tuned or default one
 NRX_HIDDEN int nrx_eg3_packed(i64 ne, i64 nblk, const double *d_x, const double *d_y, const double *d_z, const void *g,
                               int dtype, int u, double *part, double *split, hipStream_t st);
-// doubles of scratch it takes in `split`
+// launch(u) at u = 8, 12, 16 and 24 loads in flight: ms a launch (the mean of
+// reps, after a first one) and the fastest u
+NRX_HIDDEN int nrx_time_depths(const std::function<int(int u)> &launch, i64 reps, hipStream_t st, int *best,
+                               double *ms);
+// doubles of scratch nrx_eg3_packed takes in `split`
 NRX_HIDDEN i64 nrx_eg3_packed_split_doubles(i64 ne, i64 nblk);
 // EG2IC1 slab partials of nblk slabs (ip,jp,i1): part[blk][4][ne] = dir, ex,
 // dirS, exS (gs may be NULL: the S rows stay zero)

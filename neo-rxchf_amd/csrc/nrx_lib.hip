@@ -1349,17 +1349,17 @@ extern "C" int neorx_eg2ic1(int64_t nebf, int64_t npbf, const double *de, const 
 // (e,f), the rows are a symmetric bilinear form T(X,Y) of the two densities,
 // so the difference of two Fock builds is one pass:
 //   T(D,D) - T(D0,D0) = T(D - D0, D + D0)
-// (the incremental build of the mixed-precision SCF).
+// (the incremental build of the mixed-precision SCF, over the packed tensor
+// of a context: k_eg3_packed; k_eg3_slab is the pass over a full one).
 // Each thread owns one (e,f) column pair, so every read of the slab is a
 // contiguous row of ne^2 values whose base is the same for the whole
 // wavefront (a scalar base plus the lane's 32-bit offset); the sums over c run
 // in registers.  F[b] and F[d] are wave-reduced and added by lane 0 into its
 // wavefront's own LDS row; F[f] is kept per (e,f) column; the rows and columns
 // are summed in a fixed order at the end, so the result does not depend on
-// wavefront timing.  T is the storage type of GM3 (double, float or BF16);
-// all arithmetic is FP64.
-// part[blk][0..ne-1] = F, part[blk][ne] = sum_x Z(a,x) F[x] / 3 (0 when Z is
-// null).
+// wavefront timing.  T is the storage type of GM3 (double or float); all
+// arithmetic is FP64.
+// part[blk][0..ne-1] = F, part[blk][ne] = sum_x DE(a,x) F[x] / 3.
 // BF16 storage: the upper 16 bits of the FP32 value (round to nearest even)
 struct bf16_t {
     uint16_t bits;
@@ -1415,11 +1415,9 @@ NRX_DI unsigned short buf_ld(const bf16_t *, __amdgpu_buffer_rsrc_t r, unsigned 
 //   FP32   8/8 22 21 22 23;  10/8 72 62 63 65;  13/6 147 150 145 145;  16/6 364 368 369 367;
 //         17/8 1252 1183 1187 1250;  20/8 2861 2893 2901 3002;  21/4 989 1053 1064 1114;
 //         24/8 7219 7227 7182 7205;  28/3 4810 4434 3636 3928
-//   BF16  17/5 389 357 478 475; 20/6 1140 1019 1064 1051; 24/4 945 984 1413 2002; 28/2 843 877 844 1017
 template <class T> constexpr int eg3_unroll(i64 ne)
 {
     if (ne <= 8) return 8;
-    if (sizeof(T) == 2) return ne <= 20 ? 12 : 8;
     if (ne <= 12) return 12;
     if (ne <= 16 || ne > 20) return 16;
     return sizeof(T) == 4 ? 12 : 24;
@@ -1440,9 +1438,9 @@ template <class T> constexpr int eg3p_unroll(i64 ne)
 constexpr unsigned EG3_MAX_THREADS = 512;
 constexpr unsigned EG3P_THREADS = 256; // and of the packed form
 
-// P adjacent (e,f) columns of one stored row in one buffer load: P = 1 for
-// every storage type, P = 2 for BF16 (a 4-byte load, so a wavefront keeps
-// twice the bytes in flight per load; the lower address is the low half)
+// P adjacent entries of one stored row in one buffer load: P = 1 for every
+// storage type, P = 2 for BF16 (a 4-byte load, so a wavefront keeps twice the
+// bytes in flight per load; the lower address is the low half)
 template <class T, int P> struct Pack;
 template <class T> struct Pack<T, 1> {
     using raw = raw_t<T>;
@@ -1503,140 +1501,111 @@ template <> struct SlabAcc<bf16_t> {
     using type = float;
 };
 
-// R rows of the slab, c = c0 .. c0+R-1, for one (b,d) and the lane's P
-// columns: raw loads first (the buffer covers row block b, each row's byte
-// offset is wave-uniform), then the widening and three FMAs per entry
-template <class T, int R, int P, class A>
+// R rows of the slab, c = c0 .. c0+R-1, for one (b,d) and the lane's column:
+// raw loads first (the buffer covers row block b, each row's byte offset is
+// wave-uniform), then the widening and three FMAs per entry
+template <class T, int R>
 NRX_DI void eg3_rows(__amdgpu_buffer_rsrc_t rb, unsigned row_d, unsigned row_c, unsigned voff, unsigned c0,
-                     const A *__restrict__ xd, const A *__restrict__ xb, const A *const *xf, A *s1, A *s2, A *s3)
+                     const double *__restrict__ xd, const double *__restrict__ xb, const double *xf, double &s1,
+                     double &s2, double &s3)
 {
-    typename Pack<T, P>::raw r[R];
+    typename Pack<T, 1>::raw r[R];
 #pragma unroll
-    for (int k = 0; k < R; ++k) r[k] = Pack<T, P>::ld(rb, voff, row_d + (c0 + k) * row_c);
+    for (int k = 0; k < R; ++k) r[k] = Pack<T, 1>::ld(rb, voff, row_d + (c0 + k) * row_c);
     NRX_LOADS_ISSUED();
 #pragma unroll
     for (int k = 0; k < R; ++k) {
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            const A gv = (A)Pack<T, P>::get(r[k], p);
-            s1[p] += xd[c0 + k] * gv;      // X(c,d)
-            s2[p] += xb[c0 + k] * gv;      // X(c,b)
-            s3[p] += xf[p][c0 + k] * gv;   // X(c,f)
-        }
+        const double gv = Pack<T, 1>::get(r[k], 0);
+        s1 += xd[c0 + k] * gv; // D(c,d)
+        s2 += xb[c0 + k] * gv; // D(c,b)
+        s3 += xf[c0 + k] * gv; // D(c,f)
     }
 }
 
 // the last r < R + 1 rows, c = c0 .., in one batch of their own
-template <class T, int R, int P, class A>
+template <class T, int R>
 NRX_DI void eg3_tail(unsigned r, __amdgpu_buffer_rsrc_t rb, unsigned row_d, unsigned row_c, unsigned voff, unsigned c0,
-                     const A *__restrict__ xd, const A *__restrict__ xb, const A *const *xf, A *s1, A *s2, A *s3)
+                     const double *__restrict__ xd, const double *__restrict__ xb, const double *xf, double &s1,
+                     double &s2, double &s3)
 {
     if constexpr (R > 0) {
         if (r == R)
-            eg3_rows<T, R, P, A>(rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
+            eg3_rows<T, R>(rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
         else
-            eg3_tail<T, R - 1, P, A>(r, rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
+            eg3_tail<T, R - 1>(r, rb, row_d, row_c, voff, c0, xd, xb, xf, s1, s2, s3);
     }
 }
 
-// X, Y: the two densities (column-major ne x ne); Z: the density of the
-// nuclear-row term, or null.  P columns per lane (P divides ne).  With
-// gridDim.y splits a block takes its share of the b rows and writes the sums
-// F of that share to part[split][blk][x] (k_eg3_combine adds them in order).
-template <class T, int U, int P>
-__global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const double *__restrict__ X,
-                                                              const double *__restrict__ Y, const double *__restrict__ Z,
+// DE: column-major ne x ne.  With gridDim.y splits a block takes its share of
+// the b rows and writes the sums F of that share to part[split][blk][x]
+// (k_eg3_combine adds them in order).
+template <class T, int U>
+__global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const double *__restrict__ DE,
                                                               const T *__restrict__ G, double *__restrict__ part)
 {
     // LDS: Fw[nw][ne] (per-wavefront rows), Ff[ne^2] (per-column partials),
-    // Xf[ne][ne+1] with Xf[f*(ne+1) + c] = X(c,f) (a lane reads its own
+    // Df[ne][ne+1] with Df[f*(ne+1) + c] = D(c,f) (a lane reads its own
     // column f at consecutive c; the odd stride spreads the lanes' columns
-    // over the banks), Yt[ne^2] with Yt[e*ne + x] = Y(e,x), and Xs, Xf in
-    // FP32 for the FP32 sums of BF16 storage
-    using A = typename SlabAcc<T>::type;
-    constexpr bool F32 = sizeof(A) == 4;
+    // over the banks), Dt[ne^2] with Dt[e*ne + x] = D(e,x).  The columns
+    // shared by a wavefront are scalar loads from DE.
     extern __shared__ double sm[];
     const unsigned ne = (unsigned)ne_, xs = ne + 1;
     const i64 blk = blockIdx.x;
     const unsigned a = (unsigned)(blk % ne);
-    const unsigned ne2 = ne * ne, ne3 = ne2 * ne, ne4 = ne3 * ne, ncol = ne2 / P;
+    const unsigned ne2 = ne * ne, ne3 = ne2 * ne, ne4 = ne3 * ne;
     const unsigned nw = blockDim.x >> 6;
-    double *Fw = sm + (threadIdx.x >> 6) * ne, *Ff = sm + nw * ne, *Xf = Ff + ne2, *Yt = Xf + ne * xs;
-    float *Xs = (float *)(Yt + ne2);
+    double *Fw = sm + (threadIdx.x >> 6) * ne, *Ff = sm + nw * ne, *Df = Ff + ne2, *Dt = Df + ne * xs;
     const unsigned ns = gridDim.y, b0 = blockIdx.y * ne / ns, b1 = (blockIdx.y + 1) * ne / ns;
     const T *g = G + blk * (i64)ne4 * ne;
     for (unsigned k = threadIdx.x; k < nw * ne + ne2; k += blockDim.x) sm[k] = 0.0;
     for (unsigned k = threadIdx.x; k < ne2; k += blockDim.x) {
         const unsigned r = k / ne, q = k % ne;
-        Xf[r * xs + q] = X[k];     // X(q, r)
-        Xs[r * xs + q] = (float)X[k];
-        Yt[k] = Y[q * ne + r];     // Y(r, q)
+        Df[r * xs + q] = DE[k];     // D(q,r)
+        Dt[k] = DE[q * ne + r];     // D(r,q)
     }
     __syncthreads();
-    // the X columns of the sums: global FP64 (wave-uniform, scalar loads) or
-    // LDS FP32
-    const A *Xa = F32 ? (const A *)(const void *)Xs : (const A *)(const void *)X;
-    const unsigned xstride = F32 ? xs : ne;
     const bool lead = (threadIdx.x & 63) == 0;
-    for (unsigned q0 = 0; q0 < ncol; q0 += blockDim.x) {
+    for (unsigned q0 = 0; q0 < ne2; q0 += blockDim.x) {
         const unsigned qc = q0 + threadIdx.x;
-        const bool on = qc < ncol;
-        const unsigned ef = on ? qc * P : 0;
-        const unsigned e = ef / ne, f = ef % ne; // the P columns share e
-        const double *Ye = Yt + e * ne;          // Ye[x] = Y(e,x)
-        const A *xf[P];
-        double y_ef[P], accf[P];
-#pragma unroll
-        for (int p = 0; p < P; ++p) {
-            // xf[p][c] = X(c,f+p)
-            xf[p] = F32 ? (const A *)(const void *)(Xs + (f + p) * xs) : (const A *)(const void *)(Xf + (f + p) * xs);
-            y_ef[p] = on ? Ye[f + p] : 0.0;
-            accf[p] = 0.0;
-        }
+        const bool on = qc < ne2;
+        const unsigned ef = on ? qc : 0;
+        const unsigned e = ef / ne, f = ef % ne;
+        const double *De = Dt + e * ne;  // De[x] = D(e,x)
+        const double *xf = Df + f * xs;  // xf[c] = D(c,f)
+        const double d_ef = on ? De[f] : 0.0;
+        double accf = 0.0;
         const unsigned voff = ef * (unsigned)sizeof(T);
         for (unsigned b = b0; b < b1; ++b) {
-            const double y_eb = on ? Ye[b] : 0.0;
+            const double d_eb = on ? De[b] : 0.0;
             // row block b of the slab: ne^4 entries, at most 2^31 bytes for
             // nebf <= EG3_MAX_NE
             const __amdgpu_buffer_rsrc_t rb = buf_rsrc(g + (size_t)b * ne4, ne4 * (unsigned)sizeof(T));
-            const A *xb = Xa + b * xstride;
+            const double *xb = DE + b * ne;
             double accb = 0.0;
             for (unsigned d = 0; d < ne; ++d) {
-                const double y_ed = on ? Ye[d] : 0.0;
-                A s1[P], s2[P], s3[P];
-#pragma unroll
-                for (int p = 0; p < P; ++p) s1[p] = s2[p] = s3[p] = (A)0;
+                const double d_ed = on ? De[d] : 0.0;
+                double s1 = 0.0, s2 = 0.0, s3 = 0.0;
                 if (on) {
                     const unsigned row_d = d * ne2 * (unsigned)sizeof(T), row_c = ne3 * (unsigned)sizeof(T);
-                    const A *xd = Xa + d * xstride;
+                    const double *xd = DE + d * ne;
                     unsigned c = 0;
                     // U (then the rest) independent loads in flight per lane
                     // before the FMAs; the slab is read once, so the loads are
                     // nontemporal.  The rest goes as one batch: as an eight and
                     // singles, each with its own wait, 17 functions in FP32
                     // ran at 1.9 TB/s.
-                    for (; c + U <= ne; c += U)
-                        eg3_rows<T, U, P, A>(rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
-                    eg3_tail<T, U - 1, P, A>(ne - c, rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
+                    for (; c + U <= ne; c += U) eg3_rows<T, U>(rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
+                    eg3_tail<T, U - 1>(ne - c, rb, row_d, row_c, voff, c, xd, xb, xf, s1, s2, s3);
                 }
-                double vd = 0.0;
-#pragma unroll
-                for (int p = 0; p < P; ++p) {
-                    const double t1 = s1[p], t2 = s2[p], t3 = s3[p];
-                    accb += y_ef[p] * t1 - 0.5 * y_ed * t3;
-                    accf[p] += 0.25 * y_ed * t2 - 0.5 * y_eb * t1;
-                    vd += -0.5 * y_ef[p] * t2 + 0.25 * y_eb * t3;
-                }
-                vd = wave_sum(vd);
+                accb += d_ef * s1 - 0.5 * d_ed * s3;
+                accf += 0.25 * d_ed * s2 - 0.5 * d_eb * s1;
+                const double vd = wave_sum(-0.5 * d_ef * s2 + 0.25 * d_eb * s3);
                 if (lead) Fw[d] += 3.0 * vd;
             }
             accb = wave_sum(accb);
             if (lead) Fw[b] += 3.0 * accb;
         }
-        if (on) {
-#pragma unroll
-            for (int p = 0; p < P; ++p) Ff[ef + p] = 3.0 * accf[p]; // each column belongs to one lane
-        }
+        if (on) Ff[ef] = 3.0 * accf; // each column belongs to one lane
     }
     __syncthreads();
     if (threadIdx.x < 64) {
@@ -1646,7 +1615,7 @@ __global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const dou
             for (unsigned w = 0; w < nw; ++w) fx += sm[w * ne + x];
             for (unsigned e = 0; e < ne; ++e) fx += Ff[e * ne + x];
             part[((i64)blockIdx.y * gridDim.x + blk) * (ne + 1) + x] = fx;
-            if (Z) p += Z[x * ne + a] * fx;
+            p += DE[x * ne + a] * fx;
         }
         p = wave_sum(p);
         if (threadIdx.x == 0 && ns == 1) part[blk * (ne + 1) + ne] = p / 3.0;
@@ -1700,8 +1669,9 @@ NRX_DI void eg3p_tail(unsigned r, __amdgpu_buffer_rsrc_t rb, unsigned row_c, uns
 }
 
 // A slab is split over cs groups of wpb wavefronts' columns, and those over b
-// where that is still few (Eg3Split).  LDS: Fw[nw][ne], Xf, Yt and Xs as in
-// k_eg3_slab
+// where that is still few (Eg3Split).  LDS: Fw[nw][ne] (per-wavefront rows),
+// Xf[ne][ne+1] with Xf[f*(ne+1) + c] = X(c,f), Yt[ne^2] with Yt[e*ne + x] =
+// Y(e,x), and Xs, Xf in FP32 for the FP32 sums of BF16 storage
 template <class T, int U, int P>
 __global__ void __launch_bounds__(EG3P_THREADS) k_eg3_packed(i64 ne_, unsigned cs, unsigned wpb,
                                                              const double *__restrict__ X,
@@ -1823,17 +1793,18 @@ __global__ void __launch_bounds__(64) k_eg3_combine(i64 ne, int ns, const double
 // two density layouts
 static inline size_t eg3_lds(i64 ne, unsigned threads)
 {
-    return (size_t)((threads / 64) * ne + 2 * ne * ne + ne * (ne + 1)) * 8 + (size_t)ne * (ne + 1) * 4;
+    return (size_t)((threads / 64) * ne + 2 * ne * ne + ne * (ne + 1)) * 8;
 }
 
 // largest nebf whose e-e-e-p slab (nebf^5 entries) has 32-bit offsets
 static const i64 EG3_MAX_NE = 73;
 
-// lanes per slab block for n lane columns: at most EG3_MAX_THREADS (the block
+// lanes per slab block (a lane per column): at most EG3_MAX_THREADS (the block
 // loops over its columns), the multiple of 64 that leaves the fewest idle
 // lanes in the last pass, the larger one on a tie
-static inline unsigned eg3_threads_n(i64 n)
+static inline unsigned eg3_threads(i64 ne)
 {
+    const i64 n = ne * ne;
     unsigned best = 64;
     i64 waste = ((n + 63) / 64) * 64 - n;
     for (unsigned t = 128; t <= EG3_MAX_THREADS; t += 64) {
@@ -1845,25 +1816,14 @@ static inline unsigned eg3_threads_n(i64 n)
     }
     return best;
 }
-static inline unsigned eg3_threads(i64 ne) { return eg3_threads_n(ne * ne); }
-
-// columns per lane: two for BF16 storage when nebf is even (the pair shares
-// e and its first entry lies on a 4-byte boundary), else one
-static inline int eg3_pack(int dtype, i64 ne) { return dtype == NRX_BF16 && ne % 2 == 0 ? 2 : 1; }
 
 // ------------------------------------------------------------------
-// autotuned EG3 slab launches: the loads-in-flight depth U of k_eg3_slab per
-// (storage type, nebf), chosen by neorx_autotune_eg3_dev from timed launches
-// on the caller's tensor; 0 = not tuned (eg3_unroll's default)
+// the loads-in-flight depth per (storage type, nebf) that
+// neorx_autotune_eg3_dev chose from timed launches on the caller's tensor, of
+// k_eg3_slab and of k_eg3_packed; 0 = not tuned (eg3_unroll, eg3p_unroll)
 // ------------------------------------------------------------------
 static const int EG3_UNROLLS[4] = {8, 12, 16, 24};
-static int g_eg3_tuned[3][EG3_MAX_NE + 1] = {};
-
-// the densities of one launch: X on the (c,d) pair, Y on the (e,f) pair, Z
-// for the nuclear-row term (or null)
-struct Eg3Dens {
-    const double *X, *Y, *Z;
-};
+static int g_eg3_tuned[2][EG3_MAX_NE + 1] = {}, g_eg3p_tuned[3][EG3_MAX_NE + 1] = {};
 
 // Splits of the b rows per slab: a launch of few slabs is cut until it has
 // about 8192 blocks (four to eight of them fit a CU, so fewer leave the last
@@ -1883,17 +1843,17 @@ i64 nrx_eg3_split_doubles(i64 ne, i64 nblk)
     return ns > 1 ? ns * nblk * (ne + 1) : 0;
 }
 
-template <class T, int P>
-static int eg3_launch_u(int u, i64 ne, i64 nblk, int ns, Eg3Dens D, const T *g, double *part, hipStream_t st)
+template <class T>
+static int eg3_launch_u(int u, i64 ne, i64 nblk, int ns, const double *d_de, const T *g, double *part, hipStream_t st)
 {
-    const unsigned nt = eg3_threads_n(ne * ne / P);
+    const unsigned nt = eg3_threads(ne);
     const size_t lds = eg3_lds(ne, nt);
     const dim3 grid((unsigned)nblk, (unsigned)ns), blk(nt);
     switch (u) {
-    case 8: hipLaunchKernelGGL((k_eg3_slab<T, 8, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
-    case 12: hipLaunchKernelGGL((k_eg3_slab<T, 12, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
-    case 16: hipLaunchKernelGGL((k_eg3_slab<T, 16, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
-    case 24: hipLaunchKernelGGL((k_eg3_slab<T, 24, P>), grid, blk, lds, st, ne, D.X, D.Y, D.Z, g, part); break;
+    case 8: hipLaunchKernelGGL((k_eg3_slab<T, 8>), grid, blk, lds, st, ne, d_de, g, part); break;
+    case 12: hipLaunchKernelGGL((k_eg3_slab<T, 12>), grid, blk, lds, st, ne, d_de, g, part); break;
+    case 16: hipLaunchKernelGGL((k_eg3_slab<T, 16>), grid, blk, lds, st, ne, d_de, g, part); break;
+    case 24: hipLaunchKernelGGL((k_eg3_slab<T, 24>), grid, blk, lds, st, ne, d_de, g, part); break;
     default: return fail(NEORX_E_ARG, "EG3 slabs: no variant with %d loads in flight", u);
     }
     HIPCHK(hipGetLastError());
@@ -1901,32 +1861,27 @@ static int eg3_launch_u(int u, i64 ne, i64 nblk, int ns, Eg3Dens D, const T *g, 
 }
 
 // split: scratch of nrx_eg3_split_doubles (unused when that is 0)
-static int eg3_launch(int dtype, int u, i64 ne, i64 nblk, Eg3Dens D, const void *g, double *part, double *split,
-                      hipStream_t st)
+static int eg3_launch(int dtype, int u, i64 ne, i64 nblk, const double *d_de, const void *g, double *part,
+                      double *split, hipStream_t st)
 {
     const int ns = eg3_splits(ne, nblk);
     double *out = ns > 1 ? split : part;
     int rc;
-    switch (dtype) {
-    case NRX_F64:
-        rc = eg3_launch_u<double, 1>(u ? u : eg3_unroll<double>(ne), ne, nblk, ns, D, (const double *)g, out, st);
-        break;
-    case NRX_F32:
-        rc = eg3_launch_u<float, 1>(u ? u : eg3_unroll<float>(ne), ne, nblk, ns, D, (const float *)g, out, st);
-        break;
-    case NRX_BF16:
-        if (eg3_pack(dtype, ne) == 2)
-            rc = eg3_launch_u<bf16_t, 2>(u ? u : eg3_unroll<bf16_t>(ne), ne, nblk, ns, D, (const bf16_t *)g, out, st);
-        else
-            rc = eg3_launch_u<bf16_t, 1>(u ? u : eg3_unroll<bf16_t>(ne), ne, nblk, ns, D, (const bf16_t *)g, out, st);
-        break;
-    default: return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
-    }
+    if (dtype == NRX_F64)
+        rc = eg3_launch_u<double>(u ? u : eg3_unroll<double>(ne), ne, nblk, ns, d_de, (const double *)g, out, st);
+    else
+        rc = eg3_launch_u<float>(u ? u : eg3_unroll<float>(ne), ne, nblk, ns, d_de, (const float *)g, out, st);
     if (rc || ns == 1) return rc;
-    hipLaunchKernelGGL(k_eg3_combine, dim3((unsigned)nblk), dim3(64), 0, st, ne, ns, D.Z, split, part);
+    hipLaunchKernelGGL(k_eg3_combine, dim3((unsigned)nblk), dim3(64), 0, st, ne, ns, d_de, split, part);
     HIPCHK(hipGetLastError());
     return NEORX_OK;
 }
+
+// the densities of one launch: X on the (c,d) pair, Y on the (e,f) pair, Z
+// for the nuclear-row term (or null)
+struct Eg3Dens {
+    const double *X, *Y, *Z;
+};
 
 // Blocks of a packed slab: wpb wavefronts' columns each (a wavefront takes
 // all b of its columns, which pays for its set-up and its closing sums), cs
@@ -1979,6 +1934,7 @@ int nrx_eg3_packed(i64 ne, i64 nblk, const double *d_x, const double *d_y, const
                                                 (long long)ne, (long long)EG3_MAX_NE);
     const Eg3Dens D{d_x, d_y, d_z};
     int rc, ns = 1;
+    if (!u) u = g_eg3p_tuned[dtype][ne];
     if (dtype == NRX_F64)
         rc = eg3_packed_u<double, 1>(u ? u : eg3p_unroll<double>(ne), ne, nblk, &ns, D, (const double *)g, part, split, st);
     else if (dtype == NRX_F32)
@@ -1998,8 +1954,34 @@ int nrx_eg3_slabs(i64 ne, i64 nblk, const double *d_de, const void *g, int dtype
 {
     if (ne <= 0 || ne > EG3_MAX_NE) return fail(NEORX_E_UNSUPPORTED, "EG3 slabs: nebf=%lld not in 1..%lld",
                                                 (long long)ne, (long long)EG3_MAX_NE);
-    if (dtype < 0 || dtype > 2) return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
-    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, Eg3Dens{d_de, d_de, d_de}, g, part, split, st);
+    if (dtype != NRX_F64 && dtype != NRX_F32) return fail(NEORX_E_ARG, "EG3 slabs: unknown storage type %d", dtype);
+    return eg3_launch(dtype, g_eg3_tuned[dtype][ne], ne, nblk, d_de, g, part, split, st);
+}
+
+int nrx_time_depths(const std::function<int(int u)> &launch, i64 reps, hipStream_t st, int *best, double *ms)
+{
+    hipEvent_t ev[2];
+    HIPCHK(hipEventCreate(&ev[0]));
+    if (hipEventCreate(&ev[1]) != hipSuccess) {
+        (void)hipEventDestroy(ev[0]);
+        return fail(NEORX_E_HIP, "hipEventCreate failed");
+    }
+    int rc = NEORX_OK, at = -1;
+    for (int k = 0; k < 4 && !rc; ++k) {
+        float t = 0.0f;
+        rc = launch(EG3_UNROLLS[k]); // warm-up
+        if (!rc && hipEventRecord(ev[0], st) != hipSuccess) rc = fail(NEORX_E_HIP, "hipEventRecord failed");
+        for (i64 r = 0; r < reps && !rc; ++r) rc = launch(EG3_UNROLLS[k]);
+        if (!rc && (hipEventRecord(ev[1], st) != hipSuccess || hipEventSynchronize(ev[1]) != hipSuccess ||
+                    hipEventElapsedTime(&t, ev[0], ev[1]) != hipSuccess))
+            rc = fail(NEORX_E_HIP, "timing the EG3 pass failed");
+        ms[k] = t / (float)reps;
+        if (!rc && (at < 0 || ms[k] < ms[at])) at = k;
+    }
+    (void)hipEventDestroy(ev[0]);
+    (void)hipEventDestroy(ev[1]);
+    if (!rc) *best = EG3_UNROLLS[at];
+    return rc;
 }
 
 extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype, const double *d_de, const void *d_gm3,
@@ -2011,43 +1993,38 @@ extern "C" int neorx_autotune_eg3_dev(int64_t nebf, int64_t npbf, int64_t dtype,
     if (ne <= 0 || ne > EG3_MAX_NE || np <= 0) return fail(NEORX_E_ARG, "autotune EG3: bad sizes");
     if (dtype < 0 || dtype > 2) return fail(NEORX_E_ARG, "autotune EG3: unknown storage type %lld", (long long)dtype);
     if (!d_de || !d_gm3 || reps < 1) return fail(NEORX_E_ARG, "autotune EG3: bad arguments");
-    const i64 nblk = np * np * ne;
+    const i64 nblk = np * np * ne, nblkp = np * (np + 1) / 2 * ne;
     DevBuf part;
-    const i64 nsp = nrx_eg3_split_doubles(ne, nblk);
-    rc = part.alloc((nblk * (ne + 1) + nsp) * 8);
+    rc = part.alloc((nblk * (ne + 1) +
+                     std::max(nrx_eg3_split_doubles(ne, nblk), nrx_eg3_packed_split_doubles(ne, nblkp))) * 8);
     if (rc) return rc;
     double *split = part.d() + nblk * (ne + 1);
     hipStream_t st = nullptr;
     HIPCHK(hipStreamCreate(&st));
-    hipEvent_t e0, e1;
-    HIPCHK(hipEventCreate(&e0));
-    HIPCHK(hipEventCreate(&e1));
-    int best = 0;
-    float bt = 0.0f;
-    for (int k = 0; k < 4 && !rc; ++k) {
-        const int u = EG3_UNROLLS[k];
-        rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), split, st); // warm-up
-        if (!rc) rc = hipEventRecord(e0, st) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventRecord failed");
-        for (i64 r = 0; r < reps && !rc; ++r)
-            rc = eg3_launch((int)dtype, u, ne, nblk, Eg3Dens{d_de, d_de, d_de}, d_gm3, part.d(), split, st);
-        if (!rc) rc = hipEventRecord(e1, st) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventRecord failed");
-        if (!rc) rc = hipEventSynchronize(e1) == hipSuccess ? 0 : fail(NEORX_E_HIP, "hipEventSynchronize failed");
-        float ms = 0.0f;
-        if (!rc) (void)hipEventElapsedTime(&ms, e0, e1);
-        ms /= (float)reps;
-        if (all_ms) all_ms[k] = ms;
-        if (!rc && (best == 0 || ms < bt)) {
-            best = u;
-            bt = ms;
-        }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
+    // A context's pass, over as many entries as its packed tensor holds: fewer
+    // than the full one, so that the first 4-byte boundary serves (BF16 pairs)
+    const void *g = dtype == NRX_BF16 && ne > 1 ? (const void *)(((uintptr_t)d_gm3 + 3) & ~(uintptr_t)3) : d_gm3;
+    int best = 0, bestp = 0;
+    double ms[4], msp[4];
+    rc = nrx_time_depths([&](int u) {
+        return nrx_eg3_packed(ne, nblkp, d_de, d_de, d_de, g, (int)dtype, u, part.d(), split, st);
+    }, reps, st, &bestp, msp);
+    if (!rc && dtype != NRX_BF16) // and of the in-core entry points
+        rc = nrx_time_depths([&](int u) {
+            return eg3_launch((int)dtype, u, ne, nblk, d_de, d_gm3, part.d(), split, st);
+        }, reps, st, &best, ms);
     (void)hipStreamDestroy(st);
     if (rc) return rc;
-    g_eg3_tuned[dtype][ne] = best;
+    g_eg3p_tuned[dtype][ne] = bestp;
+    if (dtype != NRX_BF16) {
+        g_eg3_tuned[dtype][ne] = best;
+    } else {
+        best = bestp;
+        std::copy(msp, msp + 4, ms);
+    }
     if (best_unroll) *best_unroll = best;
-    if (best_ms) *best_ms = bt;
+    if (best_ms) *best_ms = *std::min_element(ms, ms + 4);
+    if (all_ms) std::copy(ms, ms + 4, all_ms);
     return NEORX_OK;
 }
 

@@ -1284,35 +1284,17 @@ int tune_g3(Xchf *x)
     int rc = W.get(part, nblk * (ne + 1) + nrx_eg3_packed_split_doubles(ne, nblk));
     if (rc) return rc;
     double *split = part + nblk * (ne + 1);
-    hipEvent_t ev[2];
-    HIPCHK(hipEventCreate(&ev[0]));
-    if (hipEventCreate(&ev[1]) != hipSuccess) {
-        (void)hipEventDestroy(ev[0]);
-        return fail(NEORX_E_HIP, "hipEventCreate failed");
-    }
     const void *g[3] = {x->G3, x->G3f, x->G3h};
-    constexpr int depths[4] = {8, 12, 16, 24}, reps = 3;
     for (int t = 0; t < 3 && !rc; ++t) {
-        float best = 0.0f;
-        for (int k = 0; k < 4 && g[t] && !rc; ++k) {
-            for (int r = 0; r <= reps && !rc; ++r) { // the first one warms up
-                if (r == 1) (void)hipEventRecord(ev[0], x->st);
-                rc = nrx_eg3_packed(ne, nblk, x->Se, x->Se, x->Se, g[t], t, depths[k], part, split, x->st);
-            }
-            float ms = 0.0f;
-            if (!rc && (hipEventRecord(ev[1], x->st) != hipSuccess || hipEventSynchronize(ev[1]) != hipSuccess ||
-                        hipEventElapsedTime(&ms, ev[0], ev[1]) != hipSuccess))
-                rc = fail(NEORX_E_HIP, "timing the GM3 pass failed");
-            if (!rc && (best == 0.0f || ms < best)) {
-                best = ms;
-                x->u3[t] = depths[k];
-            }
-        }
-        if (g_verbose && g[t] && !rc)
-            fprintf(stderr, "neorx: GM3 pass depth for storage %d: %d (%.3f ms)\n", t, x->u3[t], best / reps);
+        if (!g[t]) continue;
+        double ms[4];
+        rc = nrx_time_depths([&](int u) {
+            return nrx_eg3_packed(ne, nblk, x->Se, x->Se, x->Se, g[t], t, u, part, split, x->st);
+        }, 3, x->st, &x->u3[t], ms);
+        if (g_verbose && !rc)
+            fprintf(stderr, "neorx: GM3 pass depth for storage %d: %d (8/12/16/24: %.3f %.3f %.3f %.3f ms)\n", t, x->u3[t],
+                    ms[0], ms[1], ms[2], ms[3]);
     }
-    (void)hipEventDestroy(ev[0]);
-    (void)hipEventDestroy(ev[1]);
     return rc;
 }
 
