@@ -13,6 +13,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -78,13 +79,23 @@ struct System {
     DevSys d;
     std::vector<void *> allocs;
     std::vector<i64> eord, pord;
-    std::vector<i64> kpestr; // host copy (1-based)
+    // host copies: contraction ranges (1-based), powers, coefficients, geminal
+    std::vector<i64> kpestr, kpeend, elcam, nucam;
+    std::vector<double> agebfcc, agnbfcc, bcoef, gamma;
     int maxl;
+    // the pair plan, formed by the first builder that works from pairs
+    // (nrx_plan): a handle that serves primitive tuples or two-basis routines
+    // never pays for it (neorx_system_create at 60 primitives 354 us, 237 so)
     PairPlan plan{};
     std::vector<i64> cp_start; // host copy
+    std::mutex plan_mu;
+    bool planned = false;
+    i64 nuc_pairs() const { return d.npbf * (d.npbf + 1) / 2; }
 };
 
 NRX_HIDDEN System *get_sys(i64 h);
+// forms s->plan if it is not there yet (l <= 2); any thread
+NRX_HIDDEN int nrx_plan(System *s);
 
 // ------------------------------------------------------------------
 // primitive tuples (nrx_prims.hip)

@@ -224,15 +224,16 @@ static void pair_table(i64 n, const double *ex, const i64 *am, const double *cen
         for (i64 j = 0; j < n; ++j) make_pair(host_prim(n, ex, am, cen, i), host_prim(n, ex, am, cen, j), tab[i * n + j]);
 }
 
-// PairPlan of a system from its pair tables (one device block, one copy)
-static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc, const double *agnbfcc,
-                     const double *bcoef, const double *gamma, const std::vector<PairRec> &ept,
-                     const std::vector<PairRec> &ppt)
+// PairPlan of a system (one device block, one copy)
+static int pair_plan(System *s)
 {
-    const i64 ne = s->d.nebf, pe = s->d.npebf, np = s->d.npbf;
-    auto deg = [](const PairRec &q) {
+    const i64 ne = s->d.nebf, pe = s->d.npebf, np = s->d.npbf, ng = s->d.ngtg;
+    const std::vector<i64> &kpeend = s->kpeend;
+    const std::vector<double> &agebfcc = s->agebfcc, &agnbfcc = s->agnbfcc, &bcoef = s->bcoef, &gamma = s->gamma;
+    // powers of a pair, bra and ket, per direction
+    auto deg = [](const std::vector<i64> &am, i64 n, i64 i, i64 j) {
         int m = 0;
-        for (int d = 0; d < 3; ++d) m |= (q.la[d] + q.lb[d]) << (8 * d);
+        for (int d = 0; d < 3; ++d) m |= (int)(am[d * n + i] + am[d * n + j]) << (8 * d);
         return m;
     };
     auto byte = [](int m, int d) { return (m >> (8 * d)) & 255; };
@@ -244,7 +245,7 @@ static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc
             for (i64 i = s->kpestr[I] - 1; i < kpeend[I]; ++i)
                 for (i64 j = I == J ? i : s->kpestr[J] - 1; j < kpeend[J]; ++j) {
                     idx.push_back((int)(i * pe + j));
-                    dg.push_back(deg(ept[i * pe + j]));
+                    dg.push_back(deg(s->elcam, pe, i, j));
                     cf.push_back(agebfcc[i] * agebfcc[j] * (I == J && i < j ? 2.0 : 1.0));
                 }
             cps.push_back((int)idx.size());
@@ -252,7 +253,7 @@ static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc
     for (i64 j = 0; j < np; ++j)
         for (i64 i = 0; i <= j; ++i) {
             pidx.push_back((int)(i * np + j));
-            pdg.push_back(deg(ppt[i * np + j]));
+            pdg.push_back(deg(s->nucam, np, i, j));
             pcf.push_back(agnbfcc[i] * agnbfcc[j]);
         }
     PairPlan &P = s->plan;
@@ -281,10 +282,10 @@ static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc
         gl.push_back(L);
     }
     P.le = P.lp = 0;
-    for (i64 i = 0; i < pe; ++i) P.le = std::max(P.le, total(dg.empty() ? 0 : deg(ept[i * pe + i])) / 2);
-    for (i64 i = 0; i < np; ++i) P.lp = std::max(P.lp, total(deg(ppt[i * np + i])) / 2);
+    for (i64 i = 0; i < pe; ++i) P.le = std::max(P.le, total(deg(s->elcam, pe, i, i)) / 2);
+    for (i64 i = 0; i < np; ++i) P.lp = std::max(P.lp, total(deg(s->nucam, np, i, i)) / 2);
     // geminal terms: gk, gl, wkl [ng^2]; gx, wx [ng + ng(ng+1)/2]; {1, 0}
-    std::vector<double> gk, gll, wkl, gx(gamma, gamma + ng), wx(bcoef, bcoef + ng);
+    std::vector<double> gk, gll, wkl, gx(gamma), wx(bcoef);
     for (i64 k = 0; k < ng; ++k)
         for (i64 l = 0; l < ng; ++l) {
             gk.push_back(gamma[k]);
@@ -320,6 +321,15 @@ static int pair_plan(System *s, i64 ng, const i64 *kpeend, const double *agebfcc
     for (int k = 0; k < 8; ++k) *ip[k] = (const int *)(b + off[7 + k]);
     s->cp_start.assign(cps.begin(), cps.end());
     return NEORX_OK;
+}
+
+int nrx_plan(System *s)
+{
+    std::lock_guard<std::mutex> lk(s->plan_mu);
+    if (s->planned) return NEORX_OK;
+    int rc = pair_plan(s);
+    if (!rc) s->planned = true;
+    return rc;
 }
 
 extern "C" int neorx_system_create(int64_t nebf, int64_t npebf, int64_t npbf, int64_t nat, int64_t ngtg, double pmass,
@@ -369,6 +379,13 @@ extern "C" int neorx_system_create(int64_t nebf, int64_t npebf, int64_t npbf, in
     s->maxl = maxl;
     s->d.lmax = maxl;
     s->kpestr.assign(kpestr, kpestr + nebf);
+    s->kpeend.assign(kpeend, kpeend + nebf);
+    s->elcam.assign(elcam, elcam + 3 * npebf);
+    s->nucam.assign(nucam, nucam + 3 * npbf);
+    s->agebfcc.assign(agebfcc, agebfcc + npebf);
+    s->agnbfcc.assign(agnbfcc, agnbfcc + npbf);
+    s->bcoef.assign(bcoef, bcoef + ngtg);
+    s->gamma.assign(gamma, gamma + ngtg);
     DevSys &d = s->d;
     d.nebf = nebf;
     d.npebf = npebf;
@@ -410,7 +427,6 @@ extern "C" int neorx_system_create(int64_t nebf, int64_t npebf, int64_t npbf, in
     r |= upload(s, s->pord.data(), npbf, &d.pord);
     r |= upload(s, ept.data(), ept.size(), &d.ep);
     r |= upload(s, ppt.data(), ppt.size(), &d.pp);
-    if (!r && maxl <= 2) r = pair_plan(s, ngtg, kpeend, agebfcc, agnbfcc, bcoef, gamma, ept, ppt);
     if (r) {
         for (void *p : s->allocs) (void)hipFree(p);
         delete s;
@@ -2365,7 +2381,7 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
     i64 ne = s->d.nebf, np = s->d.npbf, ne4 = ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
-    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->plan.nq : npp, BLOCK_CAP / ne4));
+    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->nuc_pairs() : npp, BLOCK_CAP / ne4));
     Work W(st);
     double *X = nullptr, *Xs = nullptr, *Y = nullptr, *Ys = nullptr, *partq = nullptr, *G, *Gs, *part, *fpd;
     i64 cap = slab_cap(s, 2);
@@ -2377,7 +2393,7 @@ extern "C" int neorx_gam2_dscf_dev(int64_t handle, const double *d_de, const dou
         if (!rc) rc = W.get(Y, cap);
         if (!rc) rc = W.get(Ys, cap);
     } else if (!rc) {
-        rc = W.get(partq, s->plan.nq * ne * 4 * ne);
+        rc = W.get(partq, s->nuc_pairs() * ne * 4 * ne);
     }
     if (!rc) rc = W.get(part, npp * ne * 4 * ne + 2 * npp);
     if (rc) return rc;
@@ -2424,13 +2440,13 @@ extern "C" int neorx_gam3_dscf_dev(int64_t handle, const double *d_de, const dou
     i64 ne = s->d.nebf, np = s->d.npbf, ne6 = ne * ne * ne * ne * ne * ne, npp = np * np;
     hipStream_t st = (hipStream_t)stream;
     const bool pairs = s->maxl <= 2; // blocks of the distinct nuclear pairs; else every (ip,jp)
-    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->plan.nq : npp, BLOCK_CAP / ne6));
+    i64 nb = std::max<i64>(1, std::min<i64>(pairs ? s->nuc_pairs() : npp, BLOCK_CAP / ne6));
     Work W(st);
     double *X = nullptr, *Y = nullptr, *partq = nullptr, *G, *part;
     int rc = W.get(G, nb * ne6);
     if (!rc && !pairs) rc = W.get(X, nb * ne6);
     if (!rc && !pairs) rc = W.get(Y, slab_cap(s, 3));
-    if (!rc && pairs) rc = W.get(partq, s->plan.nq * ne * (ne + 1));
+    if (!rc && pairs) rc = W.get(partq, s->nuc_pairs() * ne * (ne + 1));
     // splits of any launch: their slab counts differ, each has less than 2 EG3_BLOCKS
     if (!rc) rc = W.get(part, npp * ne * (ne + 1) + npp + 2 * EG3_BLOCKS * (ne + 1));
     if (rc) return rc;

@@ -1539,7 +1539,7 @@ extern "C" int neorx_xchf_create(int64_t handle, int64_t nelec, int64_t store, i
     Xchf *x = new Xchf();
     x->ne = s->d.nebf;
     x->np = s->d.npbf;
-    x->nq = x->np * (x->np + 1) / 2;
+    x->nq = s->nuc_pairs();
     x->nelec = (int)nelec;
     // Non-blocking: a context's stream takes no implicit dependency on the
     // legacy stream, so another thread's legacy-stream work cannot

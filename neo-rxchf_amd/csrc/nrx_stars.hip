@@ -774,13 +774,15 @@ int rec_ne(int deg) { return (deg <= 4 ? deg : deg <= 6 ? 6 : deg <= 8 ? 8 : 12)
 // RXCHFmult form, without the one-geminal terms.
 int nrx_gam3_pairs(System *s, bool mult, i64 np_full, double *G, Work &W, bool pack, i64 nb, const PairSink &sink)
 {
+    int rc = nrx_plan(s);
+    if (rc) return rc;
     hipStream_t st = W.st;
     const DevSys &d = s->d;
     const PairPlan &P = s->plan;
     const i64 ne = d.nebf, nc = P.ncp, ntri = nc * (nc + 1) / 2;
     const int ng = (int)d.ngtg, nt = ng * ng;
     double *lone, *T, *rec;
-    int rc = W.get(lone, LONE_F * P.nslot + nc * nc + nc * P.nq + nc * P.npl);
+    rc = W.get(lone, LONE_F * P.nslot + nc * nc + nc * P.nq + nc * P.npl);
     if (rc) return rc;
     double *V = lone + LONE_F * P.nslot, *X = V + nc * nc, *Vp = X + nc * P.nq;
     hipLaunchKernelGGL(k_lone_prep, dim3((unsigned)(P.nslot / 64)), dim3(64), 0, st, d, P, lone);
@@ -859,6 +861,8 @@ int nrx_gam3_pairs(System *s, bool mult, i64 np_full, double *G, Work &W, bool p
 // GAM_2 and its overlaps (rxne: the RXCHF-ne tensors) of the distinct nuclear pairs
 int nrx_gam2_pairs(System *s, bool rxne, i64 np_full, double *G, double *Gs, Work &W, i64 nb, const PairSink &sink)
 {
+    int rc = nrx_plan(s);
+    if (rc) return rc;
     hipStream_t st = W.st;
     const DevSys &d = s->d;
     const PairPlan &P = s->plan;
@@ -867,7 +871,7 @@ int nrx_gam2_pairs(System *s, bool rxne, i64 np_full, double *G, double *Gs, Wor
     const int NE2 = rec_ne(2 * P.le + 2 * P.lp), nterms = rxne ? 1 : BT_OVL;
     const i64 nrows = (i64)nt * (rxne ? 1 : BT_ROWS);
     double *lone, *rec;
-    int rc = W.get(lone, LONE_F * P.nslot + 3 * KT * (P.npl + P.nq) + nqa * (nc * nc + 2 * ntri) + 8);
+    rc = W.get(lone, LONE_F * P.nslot + 3 * KT * (P.npl + P.nq) + nqa * (nc * nc + 2 * ntri) + 8);
     if (rc) return rc;
     double *kt = lone + LONE_F * P.nslot, *L = kt + 3 * KT * (P.npl + P.nq),
            *B = L + nqa * nc * nc, *Y = B + nqa * ntri;
