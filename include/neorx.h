@@ -53,9 +53,11 @@ const char *neorx_device_arch(void);
  * a difference drops the copy.  Copies use at most 60 % of the device memory
  * (the oldest are released first).  NEORX_RESIDENT=0 in the environment
  * turns this off.  neorx_release_resident frees every copy (neorx_finalize
- * does too), and the scratch (at most 512 MiB) that the builders and Fock
- * contractions keep between calls.  neorx_transfer_bytes reports the bytes of tensors these entry
- * points copied host->device and device->host since the process started. */
+ * does too), and the scratch (at most 512 MiB in all) that the builders and
+ * Fock contractions keep between calls, which an allocation of this library
+ * that would fail otherwise does by itself.  neorx_transfer_bytes reports the
+ * bytes of tensors these entry points copied host->device and device->host
+ * since the process started. */
 int neorx_release_resident(void);
 int neorx_transfer_bytes(int64_t *h2d_bytes, int64_t *d2h_bytes);
 

@@ -131,6 +131,11 @@ static inline unsigned nblocks(i64 n, int bs) { return (unsigned)((n + bs - 1) /
 // entries).
 static inline unsigned grid_blocks(i64 n, int bs) { return (unsigned)std::min<i64>((n + bs - 1) / bs, g_grid_cap); }
 
+// hipMalloc that gives up the scratch kept between calls (Work) before it
+// fails; no error is left behind
+NRX_HIDDEN hipError_t nrx_malloc(void **p, size_t bytes);
+NRX_HIDDEN void nrx_release_work();
+
 // device buffer released when it goes out of scope
 struct DevBuf {
     void *p = nullptr;
@@ -141,7 +146,7 @@ struct DevBuf {
     }
     int alloc(size_t bytes)
     {
-        hipError_t e = hipMalloc(&p, bytes ? bytes : 8);
+        hipError_t e = nrx_malloc(&p, bytes ? bytes : 8);
         if (e != hipSuccess) {
             p = nullptr;
             return fail(NEORX_E_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
@@ -163,7 +168,13 @@ struct StreamBuf {
     {
         st = s;
         hipError_t e = hipMallocAsync(&p, bytes, s);
+        if (e != hipSuccess) { // as nrx_malloc
+            (void)hipGetLastError();
+            nrx_release_work();
+            e = hipMallocAsync(&p, bytes, s);
+        }
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             p = nullptr;
             return fail(NEORX_E_NOMEM, "hipMallocAsync(%zu) failed: %s", bytes, hipGetErrorString(e));
         }
@@ -172,10 +183,11 @@ struct StreamBuf {
 };
 
 // Scratch of one call that ends by synchronising its stream.  The blocks go
-// back to a process-wide free list (per device, at most WORK_KEEP bytes, the
-// oldest released first; larger blocks are freed) once the stream has drained,
+// back to a process-wide free list (at most WORK_KEEP bytes in all, the oldest
+// released first; larger blocks are freed) once the stream has drained,
 // so no two calls in flight share one, whatever their threads and streams.
-// neorx_release_resident and neorx_finalize empty the list.  A device
+// neorx_release_resident, neorx_finalize and an allocation of this library
+// that would fail otherwise empty the list.  A device
 // allocation costs 0.1 ms or more, as much as a small builder's kernels.
 struct Work {
     hipStream_t st;

@@ -68,7 +68,7 @@ template <class T> static int upload(System *s, const T *h, size_t n, const T **
 {
     void *p = nullptr;
     if (n == 0) n = 1;
-    HIPCHK(hipMalloc(&p, n * sizeof(T)));
+    HIPCHK(nrx_malloc(&p, n * sizeof(T)));
     s->allocs.push_back(p);
     if (h) HIPCHK(hipMemcpy(p, h, n * sizeof(T), hipMemcpyHostToDevice));
     *out = (const T *)p;
@@ -87,14 +87,25 @@ namespace {
 std::mutex g_work_mu;
 std::vector<Work::Block> g_work;
 constexpr size_t WORK_KEEP = (size_t)512 << 20;
+} // namespace
 
-void work_release()
+void nrx_release_work()
 {
     std::lock_guard<std::mutex> lk(g_work_mu);
     for (auto &b : g_work) (void)hipFree(b.p);
     g_work.clear();
 }
-} // namespace
+
+hipError_t nrx_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    (void)hipGetLastError();
+    nrx_release_work();
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
+}
 
 int Work::get(void **p, size_t bytes)
 {
@@ -115,12 +126,7 @@ int Work::get(void **p, size_t bytes)
     }
     if (!b.p) {
         b.n = (b.n + 65535) / 65536 * 65536;
-        hipError_t e = hipMalloc(&b.p, b.n);
-        if (e != hipSuccess) { // give the kept blocks up first
-            (void)hipGetLastError();
-            work_release();
-            e = hipMalloc(&b.p, b.n);
-        }
+        hipError_t e = nrx_malloc(&b.p, b.n);
         if (e != hipSuccess) return fail(NEORX_E_NOMEM, "hipMalloc(%zu) failed: %s", b.n, hipGetErrorString(e));
     }
     held.push_back(b);
@@ -781,7 +787,7 @@ void res_keep(DevBuf &b, const double *h, i64 n)
 
 extern "C" int neorx_release_resident(void)
 {
-    work_release();
+    nrx_release_work();
     std::lock_guard<std::mutex> lk(g_res_mu);
     while (!g_res.empty()) res_drop_locked(g_res.size() - 1);
     return NEORX_OK;

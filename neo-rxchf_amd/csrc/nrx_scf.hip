@@ -1083,7 +1083,7 @@ struct Xchf {
     template <class T> int alloc(T *&p, i64 n)
     {
         void *q = nullptr;
-        hipError_t e = hipMalloc(&q, (size_t)std::max<i64>(n, 1) * sizeof(T));
+        hipError_t e = nrx_malloc(&q, (size_t)std::max<i64>(n, 1) * sizeof(T));
         if (e != hipSuccess) return fail(NEORX_E_NOMEM, "hipMalloc(%lld x %zu) failed: %s", (long long)n, sizeof(T),
                                          hipGetErrorString(e));
         allocs.push_back(q);

@@ -94,3 +94,32 @@ def test_gam2_dscf_batches(torch_dev):
     for a, b, nm in zip(got, want, ("FE", "SE", "FP", "SP", "E", "S")):
         check_close(a.cpu().numpy(), b.cpu().numpy(), what=nm)
     S.close()
+
+
+def test_refused_allocation_gives_scratch_back(torch_dev):
+    """The scratch kept between calls does not stand in the way of another
+    allocation: one that fails (here for terabytes) has emptied the list
+    first."""
+    torch = torch_dev
+    s = synth.small(seed=61, n_e_centres=3, e_shells=(0, 0, 0, 1), contract=(1,), p_shells=(0, 1), ngtg=1)
+    ne, npb = s["nebf"], s["npbf"]
+    print(f"case refused allocation nebf={ne} npbf={npb}", flush=True)
+    S = neorx.System(s)
+    de, dp = densities(torch, ne, npb)
+    out = outputs(torch, (ne * ne, npb * npb, 1))
+    call = lambda: neorx.call_dev("neorx_gam3_dscf_dev", S.handle, de.data_ptr(), dp.data_ptr(),  # noqa: E731
+                                  *[x.data_ptr() for x in out], 0)
+    call()
+    torch.cuda.synchronize()
+    want = [x.clone() for x in out]
+    free = torch.cuda.mem_get_info()[0]
+    with pytest.raises(neorx.NeorxError, match="hipMalloc"):
+        neorx.autotune_eg3_dev(2, 200000, 0, de.data_ptr(), de.data_ptr(), reps=1)
+    assert torch.cuda.mem_get_info()[0] - free > 64 << 20  # 89 MB were kept
+    for x in out:
+        x.zero_()
+    call()
+    torch.cuda.synchronize()
+    for a, b in zip(out, want):
+        assert torch.equal(a, b)
+    S.close()
