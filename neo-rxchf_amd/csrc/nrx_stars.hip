@@ -56,6 +56,8 @@
 // nuclear: 12.6 ms, 0.96 ms.
 #include "nrx_tuples.h"
 
+#include <chrono>
+
 namespace {
 
 constexpr double TWO_PI_2P5 = 34.986836655249725; // 2 pi^(5/2)
@@ -823,6 +825,9 @@ int nrx_gam3_pairs(System *s, bool mult, i64 np_full, double *G, Work &W, bool p
         hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nc * nc, 256)), dim3(256), 0, st, P, nc, (i64)1, nc, Vp, V);
         HIPCHK(hipGetLastError());
     }
+    using clock = std::chrono::steady_clock;
+    const clock::time_point t0 = clock::now();
+    clock::time_point said = t0;
     for (i64 q = 0; q < P.nq; q += nqt) {
         const i64 nqp = std::min(nqt, P.nq - q);
         for (i64 k = 0; k < nqp; k += nqr) {
@@ -845,6 +850,17 @@ int nrx_gam3_pairs(System *s, bool mult, i64 np_full, double *G, Work &W, bool p
                     hipLaunchKernelGGL(k_lone_sum, dim3(grid_blocks(nu * nq * nc, 256)), dim3(256), 0, st, P, nu, nq,
                                        ntri, part, o);
                     HIPCHK(hipGetLastError());
+                }
+                if (g_verbose) { // a line every second, and at the end
+                    HIPCHK(hipStreamSynchronize(st));
+                    const clock::time_point t = clock::now();
+                    const bool last = B1 == nc && q + k + nq == P.nq;
+                    if (last || t - said > std::chrono::seconds(1)) {
+                        said = t;
+                        fprintf(stderr, "neorx: e-e-e-p build, row %lld of %lld, nuclear pair %lld of %lld in %.1f s\n",
+                                (long long)B1, (long long)nc, (long long)(q + k + nq), (long long)P.nq,
+                                std::chrono::duration<double>(t - t0).count());
+                    }
                 }
             }
         }

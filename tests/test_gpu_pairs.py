@@ -110,3 +110,21 @@ def test_gam2_from_pairs(torch_dev, name):
         assert np.isfinite(got).all()
         check_close(np.append(got[at], np.abs(got).max()), np.append(ref, np.abs(got).max()), what=what)
     S.close()
+
+
+def test_build_reports_progress(torch_dev, monkeypatch, capfd):
+    """NEORX_VERBOSE: a long e-e-e-p build says on stderr how far it is."""
+    s = synth.small(**SYSTEMS["sp-contracted"])
+    S = neorx.System(s)
+    nc, nq = s["nebf"] * (s["nebf"] + 1) // 2, s["npbf"] * (s["npbf"] + 1) // 2
+    try:
+        monkeypatch.setenv("NEORX_VERBOSE", "1")
+        neorx.init(0)
+        S.GAM3_IC1()
+        assert f"row {nc} of {nc}, nuclear pair {nq} of {nq}" in capfd.readouterr().err
+    finally:
+        monkeypatch.delenv("NEORX_VERBOSE")
+        neorx.init(0)
+    S.GAM3_IC1()
+    assert "e-e-e-p" not in capfd.readouterr().err
+    S.close()
