@@ -922,15 +922,18 @@ NRX_HD void rel_map(const PolyT<NF> &f, const PolyT<NM> &m, const LeafMap &g, Po
 struct StarKin {
     double wk[3], wb[3], cross, c0, c1;
 };
-// NL holds the star's degree + 2.
-template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double pic, double &ovl_out)
+// NL holds the star's degree + 2.  kp(i, x, k): the kinetic polynomial k of
+// particle i in direction x, weights included.
+template <int NL, class KP>
+NRX_HD double star_kin(const Sys &s, const StarKin &o, double pic, double &ovl_out, const KP &kp)
 {
     NRX_FENCE();
     double Pr = 1.0, R = 0.0;
     const int h = s.n - 1;
     constexpr int N = NL;
     NRX_DIRS for (int x = 0; x < 3; ++x) {
-        constexpr int FS = cmin(NS, N), FT = cmin(NS + 2, N), FR = cmin(NS + 1, N);
+        // one particle's polynomial, its kinetic one, and times (r_h - r_i)
+        constexpr int FS = cmin(NS, N - 2), FT = cmin(NS + 2, N), FR = cmin(NS + 1, N - 1);
         double w = s.q[h]->p, cq = 0.0, fac = 1.0;
         LeafMap g[2];
         NRX_UNROLL for (int i = 0; i < 2; ++i) {
@@ -954,7 +957,7 @@ template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double 
         fpoly(*s.q[0], x, f);
         to_hub(f, g[0], m0);
         rel_map(f, m0, g[0], r0);
-        pair_kin_poly(*s.q[0], x, o.wk[0], o.wb[0], k);
+        kp(0, x, k);
         to_hub(k, g[0], t);
         if (h == 1) {
             // (r_h - r_0)^2: (y - dl) r0 - M[y (r0's polynomial)], with
@@ -986,7 +989,7 @@ template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double 
             to_hub(f, g[1], m1);
             rel_map(f, m1, g[1], r1);
             p_mul(t, m1, u);
-            pair_kin_poly(*s.q[1], x, o.wk[1], o.wb[1], k);
+            kp(1, x, k);
             to_hub(k, g[1], t);
             p_mul(m0, t, q);
             p_add(u, q, u);
@@ -1010,7 +1013,7 @@ template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double 
         fpoly(*s.q[h], x, f);
         p_mul(u, f, u);
         if (h == 2) p_add(u, q, u);
-        pair_kin_poly(*s.q[h], x, o.wk[h], o.wb[h], k);
+        kp(h, x, k);
         p_mul(env, k, q);
         p_add(u, q, u);
         const double T = norm * close_expect(u, iw, cq);
@@ -1019,9 +1022,14 @@ template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double 
         R = R * S + Pr * T;
         Pr *= S;
     }
-    const double kp = Kprod(s);
-    ovl_out = kp * Pr;
-    return kp * R;
+    const double K = Kprod(s);
+    ovl_out = K * Pr;
+    return K * R;
+}
+template <int NL> NRX_HD double star_kin(const Sys &s, const StarKin &o, double pic, double &ovl_out)
+{
+    return star_kin<NL>(s, o, pic, ovl_out,
+                        [&](int i, int x, auto &k) { pair_kin_poly(*s.q[i], x, o.wk[i], o.wb[i], k); });
 }
 
 // hk[t+u] += ea[t] eb[u] (-1)^u

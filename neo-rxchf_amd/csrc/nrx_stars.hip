@@ -455,34 +455,18 @@ __global__ void __launch_bounds__(256) k_gam3_expand(PairPlan P, i64 ne, i64 q0,
 // ------------------------------------------------------------------
 constexpr int KT = 7;         // coefficients of a kinetic polynomial (degree <= 2 l + 2)
 
-// -1/4 (u_A K_B + K_A u_B) per direction, u = X^L (X = y + s), K = the second
-// derivative of X^L exp(-beta X^2) over exp(-beta X^2):
-// 4 beta^2 X^{L+2} - 2 beta (2L+1) X^L + L(L-1) X^{L-2}
-NRX_DI void kin_half(int L, double sL, double be, int l, double s, PolyT<KT> &r)
-{
-    p_const(r, 4.0 * be * be);
-    p_mul_lin(r, sL);
-    p_mul_lin(r, sL);
-    r.c[0] -= 2.0 * be * (2 * L + 1);
-    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, sL, i < L);
-    r.c[0] += L == 2 ? 2.0 : 0.0;
-    NRX_UNROLL for (int i = 0; i < NRX_LMAX; ++i) p_mul_lin(r, s, i < l);
-}
-
-// kinetic polynomials of the pair list, then of the nuclear pairs (times 1/m)
+// kinetic polynomials of the pair list, then of the nuclear pairs (times 1/m):
+// the mean of the operator on the bra and on the ket
 __global__ void __launch_bounds__(64) k_pair_kin(DevSys S, PairPlan P, double *__restrict__ kt)
 {
     const i64 t = (i64)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= 3 * (P.npl + P.nq)) return;
     const i64 k = t / 3;
-    const int d = (int)(t % 3);
     const bool nuc = k >= P.npl;
-    const PairRec &q = nuc ? S.pp[P.pp_idx[k - P.npl]] : S.ep[P.pl_idx[k]];
-    PolyT<KT> a, b;
-    kin_half(q.lb[d], q.sB[d], q.beta, q.la[d], q.sA[d], a);
-    kin_half(q.la[d], q.sA[d], q.p - q.beta, q.lb[d], q.sB[d], b);
-    const double f = nuc ? -0.25 / S.pmass : -0.25;
-    NRX_UNROLL for (int i = 0; i < KT; ++i) kt[t * KT + i] = f * (a.c[i] + b.c[i]);
+    const double w = nuc ? 0.5 / S.pmass : 0.5;
+    PolyT<KT> r;
+    pair_kin_poly(nuc ? S.pp[P.pp_idx[k - P.npl]] : S.ep[P.pl_idx[k]], (int)(t % 3), w, w, r);
+    NRX_UNROLL for (int i = 0; i < KT; ++i) kt[t * KT + i] = r.c[i];
 }
 
 // Capacity tiers of a star (largest degree per direction, total degree): the
@@ -533,87 +517,6 @@ __global__ void __launch_bounds__(256) k_bond_bin(PairPlan P, StarJob J, int sca
     if (tier >= 0) list[lb[tier] + pos] = (unsigned)t;
 }
 
-// particle i's polynomial f in the hub coordinate (hub_map's map, its
-// Gaussian quantities given)
-template <int NF, int NR>
-NRX_DI void to_hub(const PolyT<NF> &f, double iW, double beta, double m0, PolyT<NR> &r)
-{
-    PolyT<NF> t;
-    p_smooth(f, 0.5 * iW, t);
-    p_compose(t, m0, beta, t);
-    p_copy(t, r);
-}
-
-// kinetic energy T of the star (see the head of the file) and its overlap;
-// kt: the kinetic polynomials of a, b and p
-template <int NL> NRX_DI double bond_kin(const Sys &s, const double *const *kt, double pmass, double &ovl)
-{
-    constexpr int ND = NL + 2; // kinetic terms raise the degree by 2
-    constexpr int FS = NS < NL ? NS : NL, FT = KT < ND ? KT : ND, FR = FS + 1;
-    const double ga = s.gam[0], gb = s.gam[1], cross = 2.0 * ga * gb / pmass;
-    double Pr = 1.0, R = 0.0;
-    NRX_DIRS for (int d = 0; d < 3; ++d) {
-        double w = s.q[2]->p, cq = 0.0, fac = 1.0, iW[2], be[2], m0[2], dl[2];
-        NRX_UNROLL for (int i = 0; i < 2; ++i) {
-            const PairRec &Q = *s.q[i];
-            const double g = s.gam[i], rW = rsqrt(Q.p + g);
-            iW[i] = rW * rW;
-            be[i] = g * iW[i];
-            dl[i] = Q.P[d] - s.q[2]->P[d];
-            m0[i] = -be[i] * dl[i];
-            const double kap = Q.p * be[i], Wq = w + kap, iWq = rcp(Wq), df = cq - dl[i];
-            fac *= sqrt(PI) * rW * exp(-(w * kap * iWq) * df * df);
-            cq = (w * cq + kap * dl[i]) * iWq;
-            w = Wq;
-        }
-        const double rw = rsqrt(w), iw = rw * rw, norm = fac * (sqrt(PI) * rw);
-        PolyT<FS> f;
-        PolyT<FS> ma, mb;
-        PolyT<FT> ta, tb;
-        PolyT<FR> ra, rb; // (r_p - r_i)_d times the polynomial of i
-        PolyT<FT> x;
-        x.n = FT;
-        auto maps = [&](int i, PolyT<FS> &m, PolyT<FT> &tm, PolyT<FR> &rr) {
-            fpoly(*s.q[i], d, f);
-            to_hub(f, iW[i], be[i], m0[i], m);
-            NRX_UNROLL for (int k = 0; k < FT; ++k) x.c[k] = kt[i][d * KT + k];
-            to_hub(x, iW[i], be[i], m0[i], tm);
-            // y_p - y_i - (P_i - P_p)
-            PolyT<FR> yf, ym;
-            NRX_UNROLL for (int k = 0; k < FR; ++k) yf.c[k] = k ? f.c[k - 1] : 0.0;
-            yf.n = FR;
-            to_hub(yf, iW[i], be[i], m0[i], ym);
-            NRX_UNROLL for (int k = 0; k < FR; ++k)
-                rr.c[k] = (k ? m.c[k - 1] : 0.0) - (k < FS ? dl[i] * m.c[k] : 0.0) - ym.c[k];
-            rr.n = FR;
-        };
-        maps(0, ma, ta, ra);
-        maps(1, mb, tb, rb);
-        PolyT<ND> q, ab, u;
-        p_mul(ma, mb, ab);
-        NRX_UNROLL for (int k = 0; k < FT; ++k) x.c[k] = kt[2][d * KT + k];
-        p_mul(ab, x, q);
-        p_mul(ta, mb, u);
-        PolyT<ND> v;
-        p_mul(ma, tb, v);
-        NRX_UNROLL for (int k = 0; k < ND; ++k) u.c[k] += v.c[k];
-        p_mul(ra, rb, v);
-        NRX_UNROLL for (int k = 0; k < ND; ++k) u.c[k] += cross * v.c[k];
-        fpoly(*s.q[2], d, f);
-        p_mul(u, f, u);
-        NRX_UNROLL for (int k = 0; k < ND; ++k) q.c[k] += u.c[k];
-        const double Td = norm * close_expect(q, iw, cq);
-        PolyT<NL> so;
-        p_mul(ab, f, so);
-        const double Sd = norm * close_expect(so, iw, cq);
-        R = R * Sd + Pr * Td;
-        Pr *= Sd;
-    }
-    const double K = s.q[0]->K * s.q[1]->K * s.q[2]->K;
-    ovl = K * Pr;
-    return K * R;
-}
-
 // The rows of a launch's values: a row per term and geminal pair, the launch's
 // stars along it.  All: every term of B and the overlap; rxne: <1/r_ab> alone.
 enum { BT_KIN = 0, BT_AP, BT_BP, BT_AB, BT_NP, BT_NA, BT_NB, BT_OVL, BT_ROWS };
@@ -641,7 +544,11 @@ k_bond(DevSys S, PairPlan P, StarJob J, int rxne, const double *__restrict__ kt,
         if (term == BT_KIN) {
             const double *kp[3] = {kt + a * 3 * KT, kt + b * 3 * KT, kt + (P.npl + q) * 3 * KT};
             double o;
-            v = bond_kin<NL>(s, kp, S.pmass, o);
+            v = star_kin<NL + 2>(s, StarKin{{}, {}, 2.0 * J.gk[k] * J.gl[k] / S.pmass, 0.0, 0.0}, PI, o,
+                                 [&](int i, int x, auto &f) {
+                                     f.n = (int)(sizeof(f.c) / sizeof(double)); // at most KT
+                                     NRX_UNROLL for (int c = 0; c < f.n; ++c) f.c[c] = kp[i][x * KT + c];
+                                 });
             val[(BT_OVL * nkl + k) * row + star] = J.w[k] * o;
         } else if (term <= BT_BP) {
             v = -coul<NL, NBC>(s, term == BT_AP ? 0 : 1, 2);
