@@ -128,3 +128,20 @@ def test_build_reports_progress(torch_dev, monkeypatch, capfd):
     S.GAM3_IC1()
     assert "e-e-e-p" not in capfd.readouterr().err
     S.close()
+
+
+def test_gam3_more_nuclear_pairs_than_a_launch(torch_dev):
+    """32896 distinct nuclear pairs, of which the values of 32768 are held at
+    once: entries of the second batch, in both nuclear orders."""
+    s = synth.small(seed=8, n_e_centres=1, e_shells=(0,), contract=(1,), p_shells=(0,) * 256, ngtg=1)
+    assert s["nebf"] == 1 and s["npbf"] == 256
+    S = neorx.System(s)
+    # pair i <= j is number j (j + 1) / 2 + i: 32768 is (128, 255)
+    en = [[i, 255, 0, 0, 0, 0, 0, 0] for i in (0, 127, 128, 129, 200, 255)]
+    en += [[e[1], e[0]] + e[2:] for e in en] + [[254, 254, 0, 0, 0, 0, 0, 0], [0, 0, 0, 0, 0, 0, 0, 0]]
+    print("case gam3 pairs, 256 nuclear functions", flush=True)
+    g = S.GAM3_IC1()
+    ref = contracted(torch_dev, S, s, 3, 3, en, list(permutations(range(3))))[:, 0]
+    assert np.isfinite(g).all()
+    check_close(g[flat_index(s, en)], ref)
+    S.close()
