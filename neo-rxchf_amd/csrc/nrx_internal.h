@@ -103,7 +103,7 @@ NRX_HIDDEN int nrx_plan(System *s);
 // values of tuples start .. start + ntup - 1 of class cls 1..10 from source src
 // (nrx_tuples.h), up to four outputs (os, ox, oy may be null)
 NRX_HIDDEN int nrx_prims(int cls, int src, const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os,
-                         double *ox, double *oy, hipStream_t st);
+                         hipStream_t st, double *ox = nullptr, double *oy = nullptr);
 
 // ------------------------------------------------------------------
 // the l <= 3 build of the engine (nrx_wide.hip)

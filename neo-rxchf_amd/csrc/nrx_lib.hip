@@ -465,14 +465,6 @@ extern "C" int neorx_system_order(int64_t handle, int64_t *eorder, int64_t *pord
     return NEORX_OK;
 }
 
-// primitive tuples of class CLS from tuple source SRC
-template <int CLS, int SRC>
-static int launch_prims(const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os, hipStream_t st,
-                        double *ox = nullptr, double *oy = nullptr)
-{
-    return nrx_prims(CLS, SRC, d, start, ntup, idx, oe, os, ox, oy, st);
-}
-
 static int prim_list(int64_t handle, int64_t cls, int64_t ntup, const int64_t *d_idx, double *d_ansE, double *d_ansS,
                      double *d_ansX, void *stream)
 {
@@ -482,18 +474,7 @@ static int prim_list(int64_t handle, int64_t cls, int64_t ntup, const int64_t *d
     if (ntup < 0 || (ntup > 0 && (!d_idx || !d_ansE))) return fail(NEORX_E_ARG, "bad tuple list arguments");
     if (ntup == 0) return NEORX_OK;
     hipStream_t st = (hipStream_t)stream;
-    switch (cls) {
-    case 1: return launch_prims<1, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 2: return launch_prims<2, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 3: return launch_prims<3, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 4: return launch_prims<4, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 5: return launch_prims<5, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 6: return launch_prims<6, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 7: return launch_prims<7, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 9: return launch_prims<9, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    case 10: return launch_prims<10, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    default: return launch_prims<8, SRC_LIST>(s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
-    }
+    return nrx_prims((int)cls, SRC_LIST, s->d, 0, ntup, d_idx, d_ansE, d_ansS, st, d_ansX);
 }
 
 extern "C" int neorx_prim_list_dev(int64_t handle, int64_t cls, int64_t ntup, const int64_t *d_idx, double *d_ansE,
@@ -523,10 +504,7 @@ extern "C" int neorx_prim_range_dev(int64_t handle, int64_t cls, int64_t start, 
     if (count == 0) return NEORX_OK;
     if (!d_ansE) return fail(NEORX_E_ARG, "null output");
     hipStream_t st = (hipStream_t)stream;
-    if (cls == 1) return launch_prims<1, SRC_SORTED>(s->d, start, count, nullptr, d_ansE, d_ansS, st);
-    if (cls == 2) return launch_prims<2, SRC_SORTED>(s->d, start, count, nullptr, d_ansE, d_ansS, st);
-    if (cls == 4) return launch_prims<4, SRC_SORTED>(s->d, start, count, nullptr, d_ansE, d_ansS, st);
-    return launch_prims<3, SRC_SORTED>(s->d, start, count, nullptr, d_ansE, d_ansS, st);
+    return nrx_prims((int)cls, SRC_SORTED, s->d, start, count, nullptr, d_ansE, d_ansS, st);
 }
 
 // ------------------------------------------------------------------
@@ -871,7 +849,7 @@ static int build2_block(System *s, i64 p0, i64 p1, double *X, double *Xs, double
     i64 ne = s->d.nebf, ne4 = ne * ne * ne * ne, cap;
     for (auto &sl : make_slabs(s, 2, p0, p1, cap)) {
         i64 R0 = slab_start(s, 2, sl.first), R1 = slab_start(s, 2, sl.second);
-        int rc = launch_prims<CLS, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y, Ys, st);
+        int rc = nrx_prims(CLS, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y, Ys, st);
         if (rc) return rc;
         i64 n = (sl.second - sl.first) * ne4;
         hipLaunchKernelGGL(k_contract2, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y, Ys, X, Xs,
@@ -889,7 +867,7 @@ static int build3_block(System *s, i64 p0, i64 p1, double *X, double *Y, hipStre
     i64 ne = s->d.nebf, ne5 = ne * ne * ne * ne * ne, cap;
     for (auto &sl : make_slabs(s, 3, p0 * ne, p1 * ne, cap)) {
         i64 R0 = slab_start(s, 3, sl.first), R1 = slab_start(s, 3, sl.second);
-        int rc = launch_prims<CLS, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y, nullptr, st);
+        int rc = nrx_prims(CLS, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y, nullptr, st);
         if (rc) return rc;
         i64 n = (sl.second - sl.first) * ne5;
         hipLaunchKernelGGL(k_contract3, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y, X, p0 * ne);
@@ -3629,7 +3607,7 @@ extern "C" int neorx_rxchf_gam2_ic1_dev(int64_t handle, double *d_gm2_1, double 
     for (auto &sl : make_slabs(s, 2, 0, np * np, cap)) {
         const i64 R0 = slab_start(s, 2, sl.first), R1 = slab_start(s, 2, sl.second);
         // primitive values of the slab: ansE1, ansS, ansE2
-        rc = launch_prims<9, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y1.d(), YS.d(), st, Y2.d());
+        rc = nrx_prims(9, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y1.d(), YS.d(), st, Y2.d());
         if (rc) return rc;
         const i64 n = (sl.second - sl.first) * ne4;
         hipLaunchKernelGGL(k_contract2, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y1.d(), YS.d(),
@@ -3908,7 +3886,7 @@ extern "C" int neorx_rxchf_gam3_ic1_dev(int64_t handle, double *d_gm3_1, double 
         for (auto &sl : make_slabs(s, 3, b * ne, (b + 1) * ne, c2)) {
             const i64 R0 = slab_start(s, 3, sl.first), R1 = slab_start(s, 3, sl.second);
             // primitive values of the slab: ans1, ans2
-            rc = launch_prims<10, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y1.d(), Y2.d(), st);
+            rc = nrx_prims(10, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y1.d(), Y2.d(), st);
             if (rc) return rc;
             const i64 n = (sl.second - sl.first) * ne5;
             hipLaunchKernelGGL(k_contract3, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y1.d(),
@@ -4658,7 +4636,7 @@ static int mult_build2(System *s, double *X1, double *Xs, double *X2, double *X3
     i64 blk = na * na * nb * nb;
     for (auto &sl : slabs) {
         i64 R0 = slab_start(s, 5, sl.first), R1 = slab_start(s, 5, sl.second);
-        rc = launch_prims<5, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y.d(), Ys.d(), st, Yx.d(), X3 ? Yy.d() : nullptr);
+        rc = nrx_prims(5, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y.d(), Ys.d(), st, Yx.d(), X3 ? Yy.d() : nullptr);
         if (rc) return rc;
         i64 n = (sl.second - sl.first) * blk;
         hipLaunchKernelGGL(k_mcontract2, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y.d(),
@@ -4844,7 +4822,7 @@ extern "C" int neorx_rxchfmult_gam3_int_dev(int64_t handle, double *d_int_gam3, 
     if (rc) return rc;
     for (auto &sl : slabs) {
         i64 R0 = slab_start(s, 6, sl.first), R1 = slab_start(s, 6, sl.second);
-        rc = launch_prims<6, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y.d(), nullptr, st);
+        rc = nrx_prims(6, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y.d(), nullptr, st);
         if (rc) return rc;
         i64 n = (sl.second - sl.first) * blk;
         hipLaunchKernelGGL(k_mcontract3, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y.d(),
@@ -4884,7 +4862,7 @@ extern "C" int neorx_rxchfmult_gam3_ic1ex_dev(int64_t handle, double *d_int_gam3
     if (rc) return rc;
     for (auto &sl : slabs) {
         i64 R0 = slab_start(s, 6, sl.first), R1 = slab_start(s, 6, sl.second);
-        rc = launch_prims<6, SRC_ORIG>(s->d, R0, R1 - R0, nullptr, Y.d(), Ys.d(), st, Yx.d());
+        rc = nrx_prims(6, SRC_ORIG, s->d, R0, R1 - R0, nullptr, Y.d(), Ys.d(), st, Yx.d());
         if (rc) return rc;
         i64 n = (sl.second - sl.first) * blk;
         hipLaunchKernelGGL(k_mcontract3, dim3(nblocks(n, 256)), dim3(256), 0, st, s->d, sl.first, n, R0, Y.d(),

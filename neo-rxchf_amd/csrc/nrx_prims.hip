@@ -235,7 +235,7 @@ int launch_class(int src, const DevSys &d, i64 start, i64 ntup, const i64 *idx, 
 } // namespace
 
 int nrx_prims(int cls, int src, const DevSys &d, i64 start, i64 ntup, const i64 *idx, double *oe, double *os,
-              double *ox, double *oy, hipStream_t st)
+              hipStream_t st, double *ox, double *oy)
 {
     switch (cls) {
     case 1: return launch_class<1>(src, d, start, ntup, idx, oe, os, ox, oy, st);
