@@ -1539,9 +1539,11 @@ NRX_DI void eg3_tail(unsigned r, __amdgpu_buffer_rsrc_t rb, unsigned row_d, unsi
 // DE: column-major ne x ne.  With gridDim.y splits a block takes its share of
 // the b rows and writes the sums F of that share to part[split][blk][x]
 // (k_eg3_combine adds them in order).
+// The deepest FP64 form is held to the registers of five waves per SIMD (91):
+// left alone it takes 97, and 20/8 took 5012 us at four waves, 4941 at five.
 template <class T, int U>
-__global__ void __launch_bounds__(EG3_MAX_THREADS) k_eg3_slab(i64 ne_, const double *__restrict__ DE,
-                                                              const T *__restrict__ G, double *__restrict__ part)
+__global__ void __launch_bounds__(EG3_MAX_THREADS) __attribute__((amdgpu_waves_per_eu(U == 24 ? 5 : 2)))
+k_eg3_slab(i64 ne_, const double *__restrict__ DE, const T *__restrict__ G, double *__restrict__ part)
 {
     // LDS: Fw[nw][ne] (per-wavefront rows), Ff[ne^2] (per-column partials),
     // Df[ne][ne+1] with Df[f*(ne+1) + c] = D(c,f) (a lane reads its own
