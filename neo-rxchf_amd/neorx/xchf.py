@@ -213,7 +213,7 @@ class XCHF:
         from . import _check, _lib, load
         load()
         self._check, self._lib = _check, _lib
-        bits = sum({"f64": 1, "f32": 2, "bf16": 4}[k] for k in store) | (8 if autotune else 0)
+        bits = sum({"f64": 1, "f32": 2, "bf16": 4}[k] for k in set(store)) | (8 if autotune else 0)
         h = _C.c_int64()
         _check(_lib.neorx_xchf_create(S.handle, nelec, bits, _C.byref(h)))
         self.ctx = h.value

@@ -371,3 +371,25 @@ def test_context_outlives_system(torch_dev):
     for a, b in zip(results(X), want):
         assert np.array_equal(a, b)
     X.close()
+
+
+def test_store_names_a_set(torch_dev):
+    """A storage type named twice is held once (and is the one that is held)."""
+    torch = torch_dev
+    s = _small(4, seed=82, n_e_centres=1, e_shells=(0, 1), contract=(1, 2), p_shells=(0,))
+    ne, npb = s["nebf"], s["npbf"]
+    print(f"case store twice nebf={ne} npbf={npb}", flush=True)
+    de = _dev(torch, synth.density(ne, 4.0, 5).ravel(order="F"))
+    dp = _dev(torch, synth.density(npb, 1.0, 6).ravel(order="F"))
+    S = neorx.System(s)
+    got = []
+    for store in (("f64",), ("f64", "f64")):
+        X = xchf.XCHF(S, 4, store=store)
+        o = [torch.zeros(n, dtype=torch.float64, device="cuda") for n in (ne * ne, npb * npb, 14)]
+        X.fock_dev(de.data_ptr(), dp.data_ptr(), "f64", *[x.data_ptr() for x in o])
+        torch.cuda.synchronize()
+        got.append([x.cpu().numpy() for x in o])
+        X.close()
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    S.close()
