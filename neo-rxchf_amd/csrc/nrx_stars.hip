@@ -33,8 +33,8 @@
 //   B(a,b) = sum_kl b_k b_l [ T + V_p - V_a - V_b - <1/r_ap> - <1/r_bp> + <1/r_ab> ]
 // with g(a,p) = gamma_k and g(b,p) = gamma_l, V the nuclear attractions of the
 // star's members.  The kinetic part T of the average
-// needs no derivative of a geminal under the kinetic operator of the other
-// side: for an electron the two forms of the reference, g g T and g T g, are
+// (star_kin) needs no derivative of a geminal under the kinetic operator of the
+// other side: for an electron the two forms of the reference, g g T and g T g, are
 // each other's transpose, and for the proton
 //   (g_a T g_b + g_b T g_a)/2 = (T g_a g_b + g_a g_b T)/2 + (1/2m) grad g_a . grad g_b,
 // so T is the mean of the operator on the bra and on the ket -- one polynomial
@@ -44,16 +44,18 @@
 // RXCHF-ne: GM2 is L with the lone electron second and without h, GM2ex the
 // <1/r_ab> of B.
 //
-// k_lone is bound by FP64 issue: about 150 FMAs per density and lone pair (27
-// densities per star with three geminals), its operands in scalar registers
-// (the star's coefficients are wave-uniform) and LDS.  Lanes over the lone
-// pairs rather than over stars for that reason: a lane per star would read
-// 200 bytes per 150 FMAs.  GAM3_IC1 over 8 contracted functions (16 s/p
-// primitives), 4 nuclear ones: 491 ms a tuple at a time, 6.5 ms here; 7
-// functions in GAM3_DSCF + GAM2_DSCF: 4.38 ms, 0.96 ms.  GAM2_IC1 over 24
-// functions (36 s/p primitives), 8 nuclear: 504 ms, 46.9 ms, of it 41 ms in
-// k_bond and 2.8 ms in k_lone; RXCHFne_GAM2_IC1 over 24 s/p/d functions, 4
-// nuclear: 12.6 ms, 0.96 ms.
+// k_lone takes about 150 FMAs per density and lone pair (27 densities per star
+// with three geminals), its operands in scalar registers (the star's
+// coefficients are wave-uniform) and LDS.  Lanes over the lone pairs rather
+// than over stars for that reason: a lane per star would read 200 bytes per
+// 150 FMAs.  The vector units issue 47 % of the time; half of the wave cycles
+// wait, mostly on scalar loads of the records, 37 % of which miss their cache.
+// k_bond is bound by FP64 issue (68 % of the time).
+// GAM3_IC1 over 8 contracted functions (16 s/p primitives), 4 nuclear ones:
+// 491 ms a tuple at a time, 6.1 ms here, of it 5.7 ms in k_lone; 7 functions in
+// GAM3_DSCF + GAM2_DSCF: 4.38 ms, 0.44 ms.  GAM2_IC1 over 24 functions (36 s/p
+// primitives), 8 nuclear: 504 ms, 46.5 ms, of it 41 ms in k_bond and 2.8 ms in
+// k_lone; RXCHFne_GAM2_IC1 over 24 s/p/d functions, 4 nuclear: 12.6 ms, 0.75 ms.
 #include "nrx_tuples.h"
 
 #include <chrono>
@@ -397,8 +399,8 @@ __global__ void __launch_bounds__(64) k_star_ovl(DevSys S, PairPlan P, StarJob J
 // Block per (contracted pairs p1 >= p2, nuclear pair): the row over p3 of
 //   1/3 [ T(12;3) + T(13;2) + T(23;1) + X3 V12 + X2 V13 + X1 V23 ]
 // in LDS, then every copy of it in the full tensor: both orders of p1, p2
-// and of each one's bra and ket, and both nuclear orders (with two
-// destinations, blocks q of G0 and G1; G1 may be null).
+// and of each one's bra and ket, and, where the tensor holds every (ip,jp),
+// both nuclear orders.
 struct Gam3Out {
     double *G;        // full tensor, or the first block
     i64 blk;          // entries of one (ip,jp) block
@@ -600,8 +602,8 @@ __global__ void __launch_bounds__(256) k_bond_sum(PairPlan P, StarJob J, LoneJob
     }
 }
 
-// Full tensors of the nuclear pairs q0 ..: G = L(a;b) + L(b;a) + B, Gs = Y
-// (ne = 0), or with ne set G = 2 L[a][b] (star electron first), Gs = B.  np > 0: every (ip,jp)
+// Full tensors of the nuclear pairs q0 ..: G = L(a;b) + L(b;a) + B, Gs = Y, or
+// with rxne G = 2 L[a][b] (star electron first), Gs = B.  np > 0: every (ip,jp)
 // of the full tensor; np = 0: one block per pair.
 __global__ void __launch_bounds__(256) k_gam2_expand(i64 ne, i64 nc, i64 q0, i64 nq, i64 np, int rxne,
                                                      const double *__restrict__ Lq, const double *__restrict__ B,
@@ -627,8 +629,10 @@ __global__ void __launch_bounds__(256) k_gam2_expand(i64 ne, i64 nc, i64 q0, i64
 // ------------------------------------------------------------------
 // host side
 // ------------------------------------------------------------------
-// bytes of star records and lone partial sums of one launch; they stay in the
-// last-level cache
+// bytes of star records and lone partial sums of one launch, which then stay in
+// the last-level cache; the primitive stars of one contracted row and nuclear
+// pair are never divided, however many they are (24 functions of 6 s/p
+// primitives each, three geminals: up to 2.2 GB)
 constexpr i64 REC_BYTES = (i64)192 << 20;
 // most blocks of one k_bond launch and term; the blocks stride over the list
 constexpr i64 BOND_BLOCKS = 8192;
